@@ -66,13 +66,12 @@ def bandwidth_probe(cells, reps=20):
 
 
 def apply_shape(sb, shape):
-    """Solute-kernel tile shape (planes, rows, XCD remap) of a subblock."""
-    sb.set_tuning(abi.TUNE_ZM_PLANES, shape["zm"])
-    sb.set_tuning(abi.TUNE_ZM_ROWS, shape["rows"])
-    sb.set_tuning(abi.TUNE_XCD_REMAP, shape["xcd"])
-    sb.set_tuning(abi.TUNE_ZM_LDS, shape.get("lds", 0))
-    sb.set_tuning(abi.TUNE_CAPTURE_CHUNK, shape.get("chunk", 0))
-    sb.set_tuning(abi.TUNE_CAPTURE_BAND, shape.get("band", 0))
+    """Tile shape of a subblock or batch: the settings given (None: the
+    library's default for its size)."""
+    for key, name in ((abi.TUNE_ZM_PLANES, "zm"), (abi.TUNE_ZM_ROWS, "rows"), (abi.TUNE_XCD_REMAP, "xcd"),
+                      (abi.TUNE_CAPTURE_CHUNK, "chunk"), (abi.TUNE_CAPTURE_BAND, "band")):
+        if shape.get(name) is not None:
+            sb.set_tuning(key, shape[name])
 
 
 def measured_traffic(size, shape, prec="fp64"):
@@ -85,10 +84,10 @@ def measured_traffic(size, shape, prec="fp64"):
         return None
     with open(path) as fh:
         text = fh.read()
-    rec = re.search(r"shape = (\S+) zm_planes (\d+) zm_rows (\d+) xcd_remap (\d+)(?: zm_lds (\d+))?", text)
+    rec = re.search(r"shape = (\S+) zm_planes (\d+) zm_rows (\d+) xcd_remap (\d+)", text)
     m = re.search(r"traffic_bytes_per_launch = ([0-9.eE+]+)", text)
-    want = (size, str(shape["zm"]), str(shape["rows"]), str(shape["xcd"]), str(shape.get("lds", 0)))
-    if not rec or not m or rec.groups()[:4] + (rec.group(5) or "0",) != want:
+    want = (size, str(shape["zm"]), str(shape["rows"]), str(shape["xcd"]))
+    if not rec or not m or rec.groups() != want:
         return None
     return float(m.group(1))
 
@@ -240,9 +239,7 @@ def run_coupled(dims, steps, warmup, shape, nsub=(2, 2, 2)):
     nucs = [cfg.nucleation(rank=r) for r in range(nr)]
     with Batch(params, nucs) as bt:
         bt.couple(nsub)
-        bt.set_tuning(abi.TUNE_ZM_PLANES, shape["zm"])
-        bt.set_tuning(abi.TUNE_ZM_ROWS, shape["rows"])
-        bt.set_tuning(abi.TUNE_XCD_REMAP, shape["xcd"])
+        apply_shape(bt, dict(shape, chunk=None, band=None))
         bt.step(warmup)
         t0 = time.perf_counter()
         reps = bt.step(steps)
@@ -552,14 +549,11 @@ def main():
     ap.add_argument("--precision", choices=("fp64", "fp32dev"), default="fp64",
                     help="storage of the timed headline run (the line's metric is quoted on fp64)")
     ap.add_argument("--zm", type=int, default=None,
-                    help="z-marching solute kernel, planes per workgroup (0: cell-parallel; default 128 for FP64, "
-                         "8 for FP32-deviation storage)")
+                    help="z-marching solute kernel, planes per workgroup (0: cell-parallel; default: the library's)")
     ap.add_argument("--zm-rows", type=int, default=None,
-                    help="rows per z-marching workgroup (4, 8, 16; default 16 for FP64, 4 for FP32-deviation)")
+                    help="rows per z-marching workgroup (4, 8, 16; default: the library's)")
     ap.add_argument("--xcd", type=int, default=None,
-                    help="1: contiguous tile runs per XCD (default 1 for FP64, 0 for FP32-deviation)")
-    ap.add_argument("--lds", type=int, default=1,
-                    help="1: z-marching kernel with its planes staged in LDS by direct loads (k_solute_zl)")
+                    help="1: one contiguous run of tiles per XCD, 0: short runs (default: the library's)")
     ap.add_argument("--capture-chunk", type=int, default=0,
                     help=">0: capture deals its list slots in chunks of this many, pinned to XCDs")
     ap.add_argument("--capture-band", type=int, default=0,
@@ -584,15 +578,7 @@ def main():
               % args.gpus, file=sys.stderr)
         sys.exit(2)
     dims = tuple(int(v) for v in args.size.split("x"))
-    # tile shapes: long 16-row tiles for FP64 storage (the fastest over the
-    # 5000-step run), short 8 x 4 tiles for FP32-deviation storage
-    fp32_tile = {"zm": 8, "rows": 4, "xcd": 0}
-    fp64_tile = {"zm": 128, "rows": 16, "xcd": 1}
-    dflt = fp32_tile if args.precision == "fp32dev" else fp64_tile
-    args.zm = dflt["zm"] if args.zm is None else args.zm
-    args.zm_rows = dflt["rows"] if args.zm_rows is None else args.zm_rows
-    args.xcd = dflt["xcd"] if args.xcd is None else args.xcd
-    shape = {"zm": args.zm, "rows": args.zm_rows, "xcd": args.xcd, "lds": args.lds, "chunk": args.capture_chunk,
+    shape = {"zm": args.zm, "rows": args.zm_rows, "xcd": args.xcd, "chunk": args.capture_chunk,
              "band": args.capture_band}
     if args.capture_footprint:
         capture_footprint(shape)
@@ -617,6 +603,8 @@ def main():
     t0 = time.time()
     gpu = Subblock(cfg.params(check_negative_ce=True, precision=prec), cfg.nucleation(), device=0)
     apply_shape(gpu, shape)
+    used = {"zm": gpu.get_tuning(abi.TUNE_ZM_PLANES), "rows": gpu.get_tuning(abi.TUNE_ZM_ROWS),
+            "xcd": gpu.get_tuning(abi.TUNE_XCD_REMAP)}
     log("gpu set-up %.1f s" % (time.time() - t0))
     n = nx * ny * nz
     if args.warmup:
@@ -638,8 +626,8 @@ def main():
     roof = {"bound": "hbm", "achieved": round(achieved, 1) if achieved else None,
             "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
-            "traffic": measured_traffic(args.size, shape, "fp32" if fp32 else "fp64"),
-            "kernel": ("k_solute_%s<%d>" % ("zl" if args.lds else "zm", args.zm_rows)) if args.zm > 0
+            "traffic": measured_traffic(args.size, used, "fp32" if fp32 else "fp64"),
+            "kernel": ("k_solute_rw<%d>" % (1 if used["rows"] == 4 else 2)) if used["zm"] > 0
             else "k_solute<true,true>",
             "bytes_per_cell": b_alg}
     if probe and achieved:
@@ -649,7 +637,7 @@ def main():
     extra = {"bandwidth_probe": probe}
     if not args.no_extra:
         if not fp32:
-            extra["fp32dev"] = run_fp32_variant(cfg, args.extra_steps, args.warmup, dict(shape, **fp32_tile))
+            extra["fp32dev"] = run_fp32_variant(cfg, args.extra_steps, args.warmup, shape)
             log("fp32dev:", extra["fp32dev"])
         extra["literal_dt"] = run_literal_dt(dims, args.extra_steps, args.warmup, shape)
         log("literal dt:", extra["literal_dt"])
@@ -689,8 +677,8 @@ def main():
         "config": {"workload": "directional solidification %dx%dx%d, %s storage" % (nx, ny, nz,
                                                                                   "FP32-deviation" if fp32
                                                                                   else "plain FP64"),
-                   "cells": n, "dt": cfg.dt, "zm_planes": args.zm, "zm_rows": args.zm_rows,
-                   "xcd_remap": args.xcd, "zm_lds": args.lds, "capture_chunk": args.capture_chunk,
+                   "cells": n, "dt": cfg.dt, "zm_planes": used["zm"], "zm_rows": used["rows"],
+                   "xcd_remap": used["xcd"], "capture_chunk": args.capture_chunk,
                    "capture_band": args.capture_band,
                    "parallelism": "single GPU"},
         "roofline": roof,

@@ -120,6 +120,32 @@ long long padded_cells(const mmca_params &p)
     return (long long) (p.nx + 2) * (p.ny + 2) * (p.nz + 2);
 }
 
+// Tile of the solute kernel (64 cells x rows x planes) for the domains of one
+// launch.  Waves of two rows and 16 planes move the fewest bytes (halo rows
+// and planes), but a launch needs enough of them to fill the chip; below 2048
+// such workgroups single-row waves and shorter walks win, down to one plane.
+// Measured per launch, FP64: 256x256x512 403 us with 8 x 16 (4096
+// workgroups), 445 with 4 x 8; 205x251x303 (2432 workgroups) 222 against 230;
+// 150x140x165 (594) 52 against 45 with 4 x 8; 128x128x256 (512) 52 against 48;
+// 72^3 14.5 with 4 x 4, 15.9 with 4 x 8 (324 workgroups); 40x36x44 8.3 with
+// 4 x 2, 9.5 with 4 x 4.
+void default_tile(const Consts *const *doms, int n, int *planes, int *rows)
+{
+    static const struct { int rows, planes; long long least; } rule[] = {
+        { 8, 16, 2048 }, { 4, 8, 1024 }, { 4, 4, 512 }, { 4, 2, 256 }, { 4, 1, 0 } };
+    for (const auto &r : rule) {
+        long long tiles = 0;
+        for (int d = 0; d < n; d++)
+            tiles += (long long) ((doms[d]->nx + 63) / 64) * ((doms[d]->ny + r.rows - 1) / r.rows) *
+                     ((doms[d]->nz + r.planes - 1) / r.planes);
+        if (tiles >= r.least) {
+            *rows = r.rows;
+            *planes = r.planes;
+            return;
+        }
+    }
+}
+
 int build_consts(const mmca_params &p, Consts &c)
 {
     if (p.nx < 1 || p.ny < 1 || p.nz < 1)
@@ -138,24 +164,16 @@ int build_consts(const mmca_params &p, Consts &c)
     c.sxy = (long long) (p.nx + 2) * (p.ny + 2);
     c.P = padded_cells(p);
     c.w64 = (c.nx + 63) / 64;          // mask words per row (interior x)
-    c.zm_planes = 64;                   // z-marching solute kernel by default (FP32 storage:
-    c.zm_by = 16;                       // shorter tiles, below)
-    c.xcd_remap = 1;
-    c.zm_lds = 1;                       // planes staged in LDS (k_solute_zl)
+    c.xcd_remap = 0;
+    c.zm_lds = 1;
     c.capture_chunk = 0;
     c.capture_band = 0;
     c.track_d = 0;
     if (p.precision != MMCA_PREC_FP64 && p.precision != MMCA_PREC_FP32DEV)
         return MMCA_ERR_ARG;
     c.f32 = (p.precision == MMCA_PREC_FP32DEV) ? 1 : 0;
-    if (c.f32) {
-        // FP32 storage streams faster in short tiles of 64 x 4 cells x 8 planes
-        // (several workgroups per CU); FP64 storage runs as fast or faster in
-        // the long 16-row tiles over a long run
-        c.zm_planes = 8;
-        c.zm_by = 4;
-        c.xcd_remap = 0;
-    }
+    const Consts *self = &c;
+    default_tile(&self, 1, &c.zm_planes, &c.zm_by);
     const int n3[3] = { p.nx, p.ny, p.nz };
     for (int a = 0; a < 3; a++) {
         // a face is a mold wall where the global domain ends (one subblock:

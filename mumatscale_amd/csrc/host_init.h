@@ -45,6 +45,8 @@ struct SitePlan {
 
 long long padded_cells(const mmca_params &p);
 int build_consts(const mmca_params &p, Consts &c);
+// tile of the solute kernel for n domains advanced together
+void default_tile(const Consts *const *doms, int n, int *planes, int *rows);
 double host_temp(const Consts &c, double sim_time, int x, int y, int z);
 void rotmat_of(double a0, double a1, double a2, double *R);
 int plan_nucleation(const mmca_params &params, const Consts &c, const mmca_nucleation_cfg *cfg,

@@ -19,7 +19,7 @@
 namespace mmca {
 hipError_t launch_nucleate(const View &v, int mode, int cur, hipStream_t s);
 hipError_t launch_beam_field(const DevBufs &b, const Consts &c, int adv, hipStream_t s);
-hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int lds, int diff, int fsc, int rec, int cur, int nxt,
+hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int tf, int diff, int fsc, int rec, int cur, int nxt,
                          hipStream_t s);
 hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s);
 hipError_t launch_list(const View &v, int cb, int capture, int decide_realloc, hipStream_t s);
@@ -300,7 +300,7 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
     HIPCHK(hipStreamSynchronize(s));
     v->dom = *desc;
     v->ndom = n;
-    v->xcd_remap = xcd_remap;
+    v->xcd_run = xcd_remap ? (int) std::max<long long>(1, (oz[n] + 7) / 8) : XCD_RUN;
     v->zm_planes_max = 0;
     for (int d = 0; d < n; d++)
         v->zm_planes_max = std::max(v->zm_planes_max, ctxs[d]->c.zm_planes);
@@ -362,7 +362,7 @@ int enqueue_iteration(mmca_ctx *ctx, bool advance)
     }
     const int rec = ctx->b.rec != nullptr;
     HIPCHK(launch_solute(ctx->view, ctx->c.am && !ctx->c.beam_sep, ctx->c.f32, rec ? 0 : zm_rows(ctx->c),
-                         ctx->c.zm_lds, 1, 1, rec, ctx->cur, nxt, ctx->stream));
+                         ctx->c.beam_sep, 1, 1, rec, ctx->cur, nxt, ctx->stream));
     if (ctx->timing) {
         HIPCHK(hipEventRecord(ctx->ev[ev0 + 1], ctx->stream));
         ctx->ev_used = ev0 + 2;
@@ -1717,7 +1717,8 @@ struct mmca_batch {
     View view;
     bool view_dirty = true;
     int cur = 0;
-    int zm_planes = 8, zm_by = 4, xcd_remap = 0, zm_lds = 1, capture_chunk = 0, capture_band = 0, track_d = 0;
+    int zm_planes = 8, zm_by = 4;      // default_tile at creation
+    int xcd_remap = 0, zm_lds = 1, capture_chunk = 0, capture_band = 0, track_d = 0;
     bool timing = false;
     std::vector<hipEvent_t> ev;
     size_t ev_used = 0;
@@ -1787,8 +1788,8 @@ int batch_enqueue(mmca_batch *bt, int cur)
         }
         HIPCHK(hipEventRecord(bt->ev[e0], bt->stream));
     }
-    HIPCHK(launch_solute(bt->view, c0.am && !c0.beam_sep, c0.f32, bt->zm_planes > 0 ? bt->zm_by : 0, bt->zm_lds, 1,
-                         1, 0, cur, nxt, bt->stream));
+    HIPCHK(launch_solute(bt->view, c0.am && !c0.beam_sep, c0.f32, bt->zm_planes > 0 ? bt->zm_by : 0, c0.beam_sep, 1, 1, 0,
+                         cur, nxt, bt->stream));
     if (bt->timing) {
         HIPCHK(hipEventRecord(bt->ev[e0 + 1], bt->stream));
         bt->ev_used = e0 + 2;
@@ -1846,6 +1847,10 @@ int mmca_batch_create(const mmca_params *params, const mmca_nucleation_cfg *nucl
         if (nucleation)
             TRY(mmca_init_nucleation(c, &nucleation[d]));
     }
+    std::vector<const Consts *> cs;
+    for (mmca_ctx *c : bt->dom)
+        cs.push_back(&c->c);
+    default_tile(cs.data(), ndomains, &bt->zm_planes, &bt->zm_by);
     HIPCHK(hipSetDevice(device));
     HIPCHK(hipStreamCreate(&bt->stream));
     for (mmca_ctx *c : bt->dom)

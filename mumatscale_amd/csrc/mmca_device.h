@@ -26,10 +26,9 @@ __device__ __forceinline__ MMCA_GLOBAL T *G(T *p)
 // MIN(x,y) of globals.h:19
 __device__ __forceinline__ double ref_min(double x, double y) { return (x < y) ? x : y; }
 
-// Sum over a workgroup of NT threads (result valid in thread 0).
-template <int NT>
+// Sum over a workgroup of nt threads, whole waves (result valid in thread 0).
 __device__ __forceinline__ double
-block_sum(double v, double *s_red)
+block_sum(double v, double *s_red, int nt)
 {
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1)
@@ -40,9 +39,16 @@ block_sum(double v, double *s_red)
     __syncthreads();
     double s = 0.0;
     if (tid == 0)
-        for (int i = 0; i < NT / 64; ++i)
+        for (int i = 0; i < nt / 64; ++i)
             s += s_red[i];
     return s;
+}
+
+template <int NT>
+__device__ __forceinline__ double
+block_sum(double v, double *s_red)
+{
+    return block_sum(v, s_red, NT);
 }
 
 // direct_temp_calc (temperature.c:24-126); x,y,z are padded indices.  AM

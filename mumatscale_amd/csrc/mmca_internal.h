@@ -24,9 +24,9 @@ struct Consts {
     int nsub[3];            // subblocks per axis of a coupled batch (0: not coupled)
     int gdimz;              // global z extent (2-D runs use y as the axis)
     int zm_planes;          // > 0: z-marching solute kernel with this many planes per workgroup
-    int zm_by;              // rows per z-marching workgroup (4, 8, 16)
-    int xcd_remap;          // 1: contiguous tile runs per XCD
-    int zm_lds;             // 1: z-marching kernel with its planes staged in LDS (k_solute_zl)
+    int zm_by;              // rows per z-marching workgroup (4: waves of 1 row; 8, 16: waves of 2 rows)
+    int xcd_remap;          // 1: one contiguous run of tiles per XCD; 0: runs of XCD_RUN
+    int zm_lds;             // MMCA_TUNE_ZM_LDS as set (both values run the same kernel)
     int capture_chunk;      // > 0: capture deals list slots in chunks of this many, pinned to XCDs
     int capture_band;       // > 0: capture works on units of this many rows of one plane, band q on XCD q % 8
     int track_d;            // 1: keep the reference's d array (stale values of cells no longer solid)
@@ -49,6 +49,9 @@ struct Consts {
     double t_init, cool_rate, gradient, grad_coef, velocity, velo_coef;
     double lpow, lv, lsd, lab, lhs, liniT, lthcon, rho, lcp, x0, y0, z0;
 };
+
+// tiles of a run on one XCD (xcd_tile)
+constexpr int XCD_RUN = 8;
 
 // quadrature nodes of the Gaussian-beam temperature (temperature.c:104)
 constexpr int BEAM_NT = 400;
@@ -138,7 +141,7 @@ struct DomainDesc {
 struct View {
     const DomainDesc *dom;       // device array, ndom entries
     int ndom;
-    int xcd_remap;               // contiguous tile runs per XCD for the solute kernel
+    int xcd_run;                 // solute tiles in a run on one XCD (xcd_tile)
     int zm_planes_max;           // largest zm_planes of the domains (LDS of the per-plane temperatures)
     const long long *off_nuc;    // k_nuc_detect workgroups
     const long long *off_zm;     // z-marching solute tiles

@@ -4,7 +4,7 @@
 // launches on the context's stream:
 //   k_nuc_detect    cell_nucleation (grain.c:1222-1318) over the sorted site list
 //   k_nuc_activate  activateNewGrains (grain.c:841-916): ids in site order, one workgroup
-//   k_solute        diffusion + partitioning (growth.c:30-170, 177-276),
+//   k_solute_rw     diffusion + partitioning (growth.c:30-170, 177-276),
 //                   fused, and a 1-bit "solid" mask of gr > 0
 //   k_list_count    interface-list membership counts from the mask
 //                   (grow_cell_reduction, growth.c:461-538)
@@ -750,6 +750,20 @@ k_solute(View V, int cur, int nxt)
     }
 }
 
+// Tile of this workgroup.  The hardware places workgroup w on XCD w % 8; runs
+// of V.xcd_run consecutive tiles (x fastest, then y, then z, then domain) go
+// to one XCD, run q to XCD q % 8, so that tiles sharing halo rows share an L2
+// while all XCDs work on the same planes.  Runs of 8 were the fastest on
+// blocks of every size (256 x 256 x 512 FP64: 403 us, against 425 us with
+// tiles dealt one by one and 440 us with one contiguous eighth per XCD).
+// At or past V.tot_zm: no tile (the grid is rounded up to whole rounds).
+__device__ __forceinline__ long long
+xcd_tile(const View &V)
+{
+    const unsigned m = (unsigned) V.xcd_run, i = blockIdx.x / 8;
+    return ((long long) (i / m) * 8 + blockIdx.x % 8) * m + i % m;
+}
+
 // Raw storage of ce and cl (FP64 values, or FP32 deviations from c0), kept
 // unconverted while a load is in flight, so that a prefetched value is only
 // waited for where it is used.
@@ -786,219 +800,304 @@ from_raw(const Consts &c, typename Store<F32>::T r)
         return r;
 }
 
-// What the z-marching kernel loads for plane q one plane ahead: ce and gr of
-// q, the tile-edge neighbours of q, and cl and fs of q+1 (the +z neighbour at
-// plane q, the cell's own value at q+1).
-template <bool F32>
-struct ZmAhead
+// Lane shifts of a double by one over the whole wave (DPP wave_shl / wave_shr,
+// which CDNA has): lane l gets lane l + 1 (up) or l - 1 (down); the last
+// (first) lane, which has no such lane, gets `edge`.
+__device__ __forceinline__ double
+from_lane_up(double v, double edge)
 {
-    typename Store<F32>::T ce, cl2, clx, cly;
-    double fs2, fsx, fsy;
-    int g;
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x130, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x130, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double
+from_lane_down(double v, double edge)
+{
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x138, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// What a wave loads of one plane: cl and fs of rows -1 .. RY of its tile, ce
+// and gr of its own rows, the x neighbours across the tile's edges (lane 63:
+// x + 1, the others: x - 1 of lane 0) and, with a temperature field, T.
+template <int RY, bool F32, bool TF>
+struct RwPlane {
+    using S = typename Store<F32>::T;
+    S cl[RY + 2], ce[RY], ecl[RY];
+    double fs[RY + 2], efs[RY], t[TF ? RY : 1];
+    int g[RY];
 };
 
-// z-marching fused kernel: a workgroup of 64 x BY threads owns a 64 x BY
-// column tile and walks `kz` planes upward.  cl/fs of the planes k-1, k, k+1
-// stay in registers, x neighbours come from the neighbouring lanes (wave
-// shuffles), y neighbours from the rows of the other waves in LDS.
-//
-// Every load of plane k+1 (ce, gr, the tile-edge neighbours, and cl, fs of
-// plane k+2) is issued before plane k is computed, into one of two register
-// sets used in turn, so that it is in flight for a whole plane.  Lanes one
-// past the last column or row of the domain load the padding cell as their
-// own value (and compute nothing), so the cell next to the boundary reads it
-// by shuffle or LDS like any other neighbour; then only lane 0 (x-1) and lane
-// 63 (x+1), and only row 0 (y-1) and row BY-1 (y+1), read neighbours from
-// memory, one of each kind per lane.
-template <int BY, bool AM, bool F32>
-__global__ void __launch_bounds__(64 * BY)
-k_solute_zm(View V, int cur, int nxt)
+// base + byte offset: a scalar base and a 32-bit lane offset, the addressing
+// form of a global load or store that needs no 64-bit lane arithmetic
+template <typename T>
+__device__ __forceinline__ MMCA_GLOBAL T *
+at_byte(MMCA_GLOBAL T *base, unsigned off)
 {
-    static_assert(BY >= 2, "row 0 and row BY-1 must be different waves");
-    __shared__ double s_cl[BY][64];
-    __shared__ double s_fs[BY][64];
-    __shared__ double s_red[BY];
+    return (MMCA_GLOBAL T *) ((MMCA_GLOBAL char *) base + off);
+}
+
+// Fused diffusion + partitioning, rows in registers.  A wave owns 64 cells x
+// RY rows and walks `zm_planes` planes upward; the four waves of a workgroup
+// take neighbouring rows (4 RY of them) and share nothing but the caches: no
+// barrier in the walk.
+//
+// The solute that crosses a face is the same number, with the other sign, for
+// the two cells on its sides: r (growth.c:95-99) is symmetric in them and
+// IEEE subtraction is antisymmetric.  So each face is computed once: the x
+// face towards x + 1 in each lane and handed to the next lane, the y faces
+// between the rows of a wave in registers, the z face towards k + 1 kept for
+// the next plane.  A cell then costs 3 face terms instead of 6, and the sums
+// run in the reference's order, so results keep its bits.
+//
+// The loads of plane k + 1 are issued before plane k is worked on, in two
+// register sets used in turn.  A cell is finished one plane late: its z terms
+// come last in the sum, so its x and y terms wait in a register until the
+// plane above has landed.
+//
+// Bound by memory: with the arithmetic taken out (a timing copy) the walk over
+// 256 x 256 x 512 takes the same time.  Two rows per wave and 16 planes read
+// the fewest halo rows that still leave two waves per SIMD in registers.
+// FP64, 256 x 256 x 512: 403 us (447 us with planes staged in LDS, 4.2 TB/s
+// of 56 B per cell); 128 x 128 x 256: 48 us (142); 40 x 36 x 44: 8.3 us (93).
+// FP32-deviation storage, 256 x 256 x 512: 293 us (337).
+template <int RY, bool F32, bool TF>
+__global__ void __launch_bounds__(512)
+k_solute_rw(View V, int cur, int nxt)
+{
+    using S = typename Store<F32>::T;
+    constexpr unsigned E = sizeof(S);
+    __shared__ double s_red[8];
     __shared__ int s_stop;
-    // Gaussian-beam tables (AM only): the cell-independent factors of the
-    // 400 quadrature terms, and the plane-dependent one for the current plane
-    __shared__ double s_beam[AM ? sizeof(BeamTab) / sizeof(double) : 1];
-    BeamTab *beam = reinterpret_cast<BeamTab *>(s_beam);
-    // Tile of this workgroup.  With xcd_remap the workgroups that the
-    // hardware hands to one XCD (linear id mod 8) take a contiguous run of
-    // tiles (x fastest, then y, then z, then domain), so that tiles sharing
-    // halo rows and planes run on the same L2.
-    long long gtile = blockIdx.x;
-    if (V.xcd_remap)
-    {
-        const long long per = (V.tot_zm + 7) / 8;
-        gtile = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    }
+    // the non-beam temperatures depend on z only (on y in 2-D runs): one value
+    // per plane of the tile (per row); dynamic LDS
+    extern __shared__ double s_T[];
+    const long long gtile = xcd_tile(V);
     if (gtile >= V.tot_zm)
         return;                                   // uniform over the workgroup
     const int dm = find_dom(V.off_zm, V.ndom, gtile);
-    const long long tile = gtile - V.off_zm[dm];
-    const DevBufs b = V.dom[dm].b;    // private copy: stores cannot alias it
-    const Consts c = V.dom[dm].c;
-    const int kz = c.zm_planes;
-    Counters *cnt = b.cnt;
+    const unsigned tile = (unsigned) (gtile - V.off_zm[dm]);
+    const DomainDesc *dd = &V.dom[dm];
+    const Consts c = dd->c;           // private copies: stores cannot alias them
+    MMCA_GLOBAL S *clc, *cln, *ceb;
+    if constexpr (F32)
+    {
+        clc = cl32_buf(dd->b, cur);
+        cln = cl32_buf(dd->b, nxt);
+        ceb = G(dd->b.ce32);
+    }
+    else
+    {
+        clc = cl_buf(dd->b, cur);
+        cln = cl_buf(dd->b, nxt);
+        ceb = G(dd->b.ce);
+    }
+    const MMCA_GLOBAL double *fsc = fs_buf(dd->b, cur);
+    MMCA_GLOBAL double *fsn = fs_buf(dd->b, nxt);
+    MMCA_GLOBAL int *grb = G(dd->b.gr);
+    const MMCA_GLOBAL double *tb = G(dd->b.temp);
+    MMCA_GLOBAL unsigned long long *mask = G(dd->b.mask);
+    const int lane = threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int rows = blockDim.y * RY;
+    const unsigned ntx = (unsigned) (c.nx + 63) / 64, nty = (unsigned) (c.ny + rows - 1) / rows;
+    const unsigned trow = tile / ntx;
+    const int bx = (int) (tile - trow * ntx);
+    const int bz = (int) (trow / nty);
+    const int by = (int) (trow - bz * nty);
+    const int x = bx * 64 + lane + 1;
+    const int j0 = by * rows + wv * RY + 1;
+    const int k0 = bz * c.zm_planes + 1;
+    const int k1 = min(c.nz, k0 + c.zm_planes - 1);
     // this kernel itself may raise the status: read it once per workgroup so
-    // that every wave takes the same branch before the barriers below
-    if (threadIdx.x == 0 && threadIdx.y == 0)
-        s_stop = (G(b.cnt)->status != MMCA_OK);
+    // that every wave takes the same branch before the barrier of block_sum
+    if (lane == 0 && threadIdx.y == 0)
+        s_stop = (G(dd->b.cnt)->status != MMCA_OK);
+    const bool two_d = (c.gdimz == 1);
+    if constexpr (!TF)
+    {
+        const double sim_time = G(dd->b.cnt)->timestep * c.dt;
+        const int nT = two_d ? rows : k1 - k0 + 1;
+        for (int e = wv * 64 + lane; e < nT; e += 64 * blockDim.y)
+            s_T[e] = temp_model<false>(c, sim_time, 1, two_d ? by * rows + 1 + e : 1, two_d ? 1 : k0 + e);
+    }
     __syncthreads();
     if (s_stop)
         return;
-    const int lane = threadIdx.x;
-    const int ty = threadIdx.y;
-    if constexpr (AM)
-        beam_tab_terms(c, *beam, ty * 64 + lane, 64 * BY);
-    const int ntx = (c.nx + 63) / 64, nty = (c.ny + BY - 1) / BY;
-    const int bx = (int) (tile % ntx);
-    const int by = (int) ((tile / ntx) % nty);
-    const int bz = (int) (tile / ((long long) ntx * nty));
-    const int x = bx * 64 + lane + 1;
-    const int j = by * BY + ty + 1;
-    const int k0 = bz * kz + 1;
-    const int k1 = min(c.nz, k0 + kz - 1);
-    const bool rowok = (j <= c.ny);
-    const bool active = rowok && (x <= c.nx);
-    // Own cl/fs: every computing cell, and the padding cells one past the
-    // last column and row (the neighbours of the boundary cells).  Loads are
-    // issued by every lane, at addresses clamped into the padded box, so that
-    // no branch skips one and each wait covers exactly the plane it needs.
-    const int xc = min(x, c.nx + 1), jc = min(j, c.ny + 1);
-    const long long col = (long long) jc * c.sx + xc;
-    const long long row0 = (long long) jc * c.sx + bx * 64;   // x-1 of lane 0
-    const MMCA_GLOBAL double *fsc = fs_buf(b, cur);
-    MMCA_GLOBAL double *fsn_out = fs_buf(b, nxt);
-    const double sim_time = G(b.cnt)->timestep * c.dt;
-    const bool xm_mem = (lane == 0);
-    const bool xp_mem = (lane == 63);
-    const bool ym_mem = (ty == 0);
-    const bool yp_mem = (ty == BY - 1);
-    // tile-edge neighbours: lane 63 reads x+1, every other lane the x-1 of
-    // lane 0 (one shared line); row 0 reads y-1, row BY-1 y+1, the other rows
-    // the first cell of their row
-    const long long xe = xp_mem ? col + 1 : row0;
-    const long long ye = ym_mem ? col - c.sx : yp_mem ? col + c.sx : row0 + 1;
-    const int mo_x1 = (x == c.nx) ? c.pad_hi[0] : 0, mo_x0 = (x == 1) ? c.pad_lo[0] : 0;
-    const int mo_y1 = (j == c.ny) ? c.pad_hi[1] : 0, mo_y0 = (j == 1) ? c.pad_lo[1] : 0;
-    auto fetch = [&](ZmAhead<F32> &a, int q) {
-        // plane q's ce, gr and edge neighbours; plane q+1's cl and fs
-        const long long pq = q * c.sxy;
-        a.cl2 = raw_cl<F32>(b, cur, pq + c.sxy + col);
-        a.fs2 = fsc[pq + c.sxy + col];
-        a.ce = raw_ce<F32>(b, pq + col);
-        a.g = G(b.gr)[pq + col];
-        a.clx = raw_cl<F32>(b, cur, pq + xe);
-        a.fsx = fsc[pq + xe];
-        a.cly = raw_cl<F32>(b, cur, pq + ye);
-        a.fsy = fsc[pq + ye];
-    };
-    double clm = from_raw<F32>(c, raw_cl<F32>(b, cur, (k0 - 1) * c.sxy + col));
-    double fsm = fsc[(k0 - 1) * c.sxy + col];
-    double clv = from_raw<F32>(c, raw_cl<F32>(b, cur, k0 * c.sxy + col));
-    double fsv = fsc[k0 * c.sxy + col];
-    // Loads run one plane ahead, in two register sets used in turn.  (Two
-    // planes ahead, with a third set, measured slower.)
-    ZmAhead<F32> P0, P1;
-    fetch(P0, k0);
-    // the loop starts with nothing in flight, so that its waits are the
-    // steady-state ones
-    __builtin_amdgcn_s_waitcnt(0);
     double lost = 0.0;
-    bool neg = false;                             // a negative ce seen by this lane
-    // one plane: `ld` (plane k-1's set) receives plane k+1, `use` holds plane k
-    auto plane = [&](int k, ZmAhead<F32> &ld, ZmAhead<F32> &use) {
-        const long long idx = k * c.sxy + col;
-        if (k > k0)
-        {
-            clm = clv;
-            fsm = fsv;
-            clv = from_raw<F32>(c, ld.cl2);       // landed: it was plane k-1's +z neighbour
-            fsv = ld.fs2;
-        }
-        // near the top this reloads plane k1 (unused): every plane issues
-        // the same loads, so every wait is the same
-        fetch(ld, min(k + 1, k1));
-        if constexpr (AM)
-            beam_tab_plane(c, *beam, k, ty * 64 + lane, 64 * BY);   // read after the barrier below
-        s_cl[ty][lane] = clv;
-        s_fs[ty][lane] = fsv;
-        const double shxm = __shfl_up(clv, 1, 64), sfxm = __shfl_up(fsv, 1, 64);
-        const double shxp = __shfl_down(clv, 1, 64), sfxp = __shfl_down(fsv, 1, 64);
-        __syncthreads();
-        int g_new = 0;
-        if (active)
-        {
-            const double ex_cl = from_raw<F32>(c, use.clx), ey_cl = from_raw<F32>(c, use.cly);
-            const double clxm = xm_mem ? ex_cl : shxm, fsxm = xm_mem ? use.fsx : sfxm;
-            const double clxp = xp_mem ? ex_cl : shxp, fsxp = xp_mem ? use.fsx : sfxp;
-            const double clym = ym_mem ? ey_cl : s_cl[ym_mem ? 0 : ty - 1][lane];
-            const double fsym = ym_mem ? use.fsy : s_fs[ym_mem ? 0 : ty - 1][lane];
-            const double clyp = yp_mem ? ey_cl : s_cl[yp_mem ? 0 : ty + 1][lane];
-            const double fsyp = yp_mem ? use.fsy : s_fs[yp_mem ? 0 : ty + 1][lane];
-            const double clp = from_raw<F32>(c, use.cl2), fsp = use.fs2;
-            const double ce_old = from_raw<F32>(c, use.ce);
-            const int g_old = use.g;
-            const double cln[6] = { clxp, clxm, clyp, clym, clp, clm };
-            const double fsn[6] = { fsxp, fsxm, fsyp, fsym, fsp, fsm };
-            const int mo[6] = { mo_x1, mo_x0, mo_y1, mo_y0, (k == c.nz) ? c.pad_hi[2] : 0,
-                                (k == 1) ? c.pad_lo[2] : 0 };
-            const double ce_new = diffuse_cell(c, ce_old, clv, fsv, cln, fsn, mo);
-            neg |= (ce_new < 0);
-            lost += st_ce<F32>(b, c, idx, ce_new);
-            double cl_out, fs_out;
-            int branch;
-            partition_cell(
-                c,
-                [&]() {
-                    if constexpr (AM)
-                        return beam_temp_tab(c, *beam, beam->Z, sim_time, x, j, k);
-                    else
-                        return temp_step<false>(b, c, sim_time, idx, x, j, k);
-                },
-                ce_new, ce_old, clv, fsv, g_old, &cl_out, &fs_out, &g_new, &branch);
-            st_cl<F32>(b, c, nxt, idx, cl_out);
-            st_stream(fsn_out, idx, fs_out);
-            if (g_new != g_old)
-                G(b.gr)[idx] = g_new;
-            keep_stale_d(c, b, idx, g_old, g_new, fsv);
-        }
-        unsigned long long bits = __ballot(active && g_new > 0);
-        if (rowok && lane == 0)
-            G(b.mask)[((long long) k * (c.ny + 2) + j) * c.w64 + bx] = bits;
-        __syncthreads();
-    };
-    // Whole rounds of two planes, so that the loop is only re-entered after
-    // a whole round and its waits see the same loads on every path; then the
-    // plane left over.
-    int k = k0;
-    for (; k + 1 <= k1; k += 2)
+    bool neg = false;
+    if (j0 <= c.ny)
     {
-        plane(k, P1, P0);
-        plane(k + 1, P0, P1);
+        // every lane issues every load, at an address clamped into the padded box
+        const unsigned xc = (unsigned) min(x, c.nx + 1);
+        const unsigned xe = lane == 63 ? (unsigned) min(x + 1, c.nx + 1) : (unsigned) (bx * 64);
+        const double wxr = (x == c.nx) ? (double) (1 - c.pad_hi[0]) : 1.0;
+        const double wxl = (x == 1) ? (double) (1 - c.pad_lo[0]) : 1.0;
+        // rows relative to row j0 - 1: the padding row is the last one loaded
+        const int rmax = c.ny + 2 - j0;
+        const long long row0 = (long long) (j0 - 1) * c.sx;
+        auto load = [&](RwPlane<RY, F32, TF> &p, int k) {
+            const long long at = k * c.sxy + row0;
+#pragma unroll
+            for (int r = 0; r < RY + 2; ++r)
+            {
+                const unsigned o = (unsigned) (min(r, rmax) * c.sx) + xc;
+                p.cl[r] = *at_byte(clc + at, o * E);
+                p.fs[r] = *at_byte(fsc + at, o * 8);
+            }
+#pragma unroll
+            for (int r = 0; r < RY; ++r)
+            {
+                const unsigned rb = (unsigned) (min(r + 1, rmax) * c.sx);
+                p.ecl[r] = *at_byte(clc + at, (rb + xe) * E);
+                p.efs[r] = *at_byte(fsc + at, (rb + xe) * 8);
+                p.ce[r] = *at_byte(ceb + at, (rb + xc) * E);
+                p.g[r] = *at_byte(grb + at, (rb + xc) * 4);
+                if constexpr (TF)
+                    p.t[r] = *at_byte(tb + at, (rb + xc) * 8);
+            }
+        };
+        // solute through the face from cell a to cell b (growth.c:95-99)
+        auto face = [&](double cla, double fsa, double clb, double fsb, double w) -> double {
+            const double f = 0.5 * (fsa + fsb);
+            const double r = (c.rs * f + c.rl * (1 - f)) * w;
+            return r * (clb - cla);
+        };
+        // the plane below, not finished yet: x and y terms, own values, and
+        // the z face below it
+        double psum[RY], pcl[RY], pfs[RY], pce[RY], pfz[RY], pt[TF ? RY : 1];
+        int pg[RY];
+        RwPlane<RY, F32, TF> P0, P1;
+        load(P0, k0);
+        {
+            const long long at = (k0 - 1) * c.sxy + row0;
+#pragma unroll
+            for (int r = 0; r < RY; ++r)
+            {
+                const unsigned o = (unsigned) (min(r + 1, rmax) * c.sx) + xc;
+                pcl[r] = from_raw<F32>(c, *at_byte(clc + at, o * E));
+                pfs[r] = *at_byte(fsc + at, o * 8);
+                psum[r] = pce[r] = pfz[r] = 0.0;
+                pg[r] = 0;
+            }
+        }
+        // plane k in A (landed); plane k + 1 goes to N
+        auto plane = [&](int k, RwPlane<RY, F32, TF> &A, RwPlane<RY, F32, TF> &N) {
+            load(N, min(k + 1, k1 + 1));
+            const double wz = (k == 1) ? (double) (1 - c.pad_lo[2])
+                                       : (k == c.nz + 1) ? (double) (1 - c.pad_hi[2]) : 1.0;
+            double cl = from_raw<F32>(c, A.cl[1]);
+            double fy = face(from_raw<F32>(c, A.cl[0]), A.fs[0], cl, A.fs[1],
+                             (j0 == 1) ? (double) (1 - c.pad_lo[1]) : 1.0);
+#pragma unroll
+            for (int r = 0; r < RY; ++r)
+            {
+                const int j = j0 + r;
+                const double fs = A.fs[r + 1];
+                const double fz = face(pcl[r], pfs[r], cl, fs, wz);
+                if (k > k0)
+                {
+                    // finish plane k - 1
+                    double sum = psum[r];
+                    sum += fz;
+                    sum -= pfz[r];
+                    const double ce_new = pce[r] + sum;
+                    int g_new = 0;
+                    if (j <= c.ny && x <= c.nx)
+                    {
+                        const long long at = (k - 1) * c.sxy + row0;
+                        const unsigned o = (unsigned) ((r + 1) * c.sx) + (unsigned) x;
+                        neg |= (ce_new < 0);
+                        double cl_out, fs_out;
+                        int branch;
+                        partition_cell(
+                            c,
+                            [&]() {
+                                if constexpr (TF)
+                                    return pt[r];
+                                else
+                                    return s_T[two_d ? wv * RY + r : k - 1 - k0];
+                            },
+                            ce_new, pce[r], pcl[r], pfs[r], pg[r], &cl_out, &fs_out, &g_new, &branch);
+                        if constexpr (F32)
+                        {
+                            const double dev = ce_new - c.cinit;
+                            const float f = (float) dev;
+                            lost += dev - (double) f;
+                            *at_byte(ceb + at, o * E) = f;
+                            *at_byte(cln + at, o * E) = (float) (cl_out - c.cinit);
+                        }
+                        else
+                        {
+                            *at_byte(ceb + at, o * E) = ce_new;
+                            *at_byte(cln + at, o * E) = cl_out;
+                        }
+                        *at_byte(fsn + at, o * 8) = fs_out;
+                        if (g_new != pg[r])
+                        {
+                            *at_byte(grb + at, o * 4) = g_new;
+                            if (c.track_d)
+                                keep_stale_d(c, dd->b, at + o, pg[r], g_new, pfs[r]);
+                        }
+                    }
+                    const unsigned long long bits = __ballot(g_new > 0);
+                    if (lane == 0 && j <= c.ny)
+                        mask[((long long) (k - 1) * (c.ny + 2) + j) * c.w64 + bx] = bits;
+                }
+                // x and y terms of plane k
+                const double ecl = from_raw<F32>(c, A.ecl[r]);
+                const double fx = face(cl, fs, from_lane_up(cl, ecl), from_lane_up(fs, A.efs[r]), wxr);
+                const double fe = face(ecl, A.efs[r], cl, fs, wxl);  // lane 0: from x - 1
+                const double clu = from_raw<F32>(c, A.cl[r + 2]);
+                const double fyu = face(cl, fs, clu, A.fs[r + 2], (j == c.ny) ? (double) (1 - c.pad_hi[1]) : 1.0);
+                double sum = 0.0 + fx;
+                sum -= from_lane_down(fx, fe);
+                sum += fyu;
+                sum -= fy;
+                psum[r] = sum;
+                pcl[r] = cl;
+                pfs[r] = fs;
+                pce[r] = from_raw<F32>(c, A.ce[r]);
+                pg[r] = A.g[r];
+                pfz[r] = fz;
+                if constexpr (TF)
+                    pt[r] = A.t[r];
+                fy = fyu;
+                cl = clu;
+            }
+        };
+        // the loop starts with nothing in flight, so that its waits are the
+        // steady-state ones
+        __builtin_amdgcn_s_waitcnt(0);
+        for (int k = k0;;)
+        {
+            plane(k, P0, P1);
+            if (++k > k1 + 1)
+                break;
+            plane(k, P1, P0);
+            if (++k > k1 + 1)
+                break;
+        }
     }
-    if (k <= k1)
-        plane(k, P1, P0);
-    // status and step of a negative ce (any plane of the tile: the step is
-    // the same for all)
     if (c.check_neg && neg)
-        flag_negative_ce(V, c, cnt);
+        flag_negative_ce(V, c, dd->b.cnt);
     if (F32)
     {
-        const double tot = block_sum<64 * BY>(lost, s_red);
-        if (lane == 0 && ty == 0 && tot != 0.0)
-            ledger_add(b, tile, tot);
+        const double tot = block_sum(lost, s_red, 64 * blockDim.y);
+        if (lane == 0 && threadIdx.y == 0 && tot != 0.0)
+            ledger_add(dd->b, tile, tot);
     }
 }
 
 // ---------------------------------------------------------------------------
-// z-marching fused kernel with its planes staged in LDS by direct global->LDS
-// loads (gfx950 global_load_lds_dword): k_solute_zl.
+// The fused kernel of the Gaussian-beam quadrature (k_solute_zl): z-marching,
+// with its planes staged in LDS by direct global->LDS loads (gfx950
+// global_load_lds_dword).
 //
 // A workgroup of 64 x BY threads owns a 64 x BY column tile and walks its
-// planes upward, as k_solute_zm does, with the same arithmetic per cell.  The
+// planes upward, with the same arithmetic per cell as k_solute.  The
 // planes come through a ring of ZL_RING slots in LDS instead of registers:
 // each slot holds one plane's cl and fs over the tile with a one-cell halo in
 // x and y ((BY + 2) rows x 66), and its ce and gr over the tile.  The loads
@@ -1071,7 +1170,7 @@ zl_wait()
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int BY, bool AM, bool F32>
+template <int BY, bool F32>
 __global__ void __launch_bounds__(64 * BY)
 k_solute_zl(View V, int cur, int nxt)
 {
@@ -1081,21 +1180,10 @@ k_solute_zl(View V, int cur, int nxt)
     __shared__ __attribute__((aligned(16))) unsigned s_ring[ZL_RING * L::DW];
     __shared__ double s_red[BY];
     __shared__ int s_stop;
-    __shared__ double s_beam[AM ? sizeof(BeamTab) / sizeof(double) : 1];
-    __shared__ double s_z[AM ? 2 : 1][AM ? BEAM_NT : 1];      // plane factors of the beam, double-buffered
-    // the other temperature models depend on z only (on y in 2-D runs): one
-    // value per plane of the tile, computed before the walk, so that their
-    // constants need no registers during it; dynamic LDS of V.zm_planes_max
-    // doubles (none for the beam), so that short tiles leave room for more
-    // workgroups per CU
-    extern __shared__ double s_T[];
+    __shared__ double s_beam[sizeof(BeamTab) / sizeof(double)];
+    __shared__ double s_z[2][BEAM_NT];           // plane factors of the beam, double-buffered
     BeamTab *beam = reinterpret_cast<BeamTab *>(s_beam);
-    long long gtile = blockIdx.x;
-    if (V.xcd_remap)
-    {
-        const long long per = (V.tot_zm + 7) / 8;
-        gtile = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    }
+    const long long gtile = xcd_tile(V);
     if (gtile >= V.tot_zm)
         return;                                   // uniform over the workgroup
     const int dm = find_dom(V.off_zm, V.ndom, gtile);
@@ -1199,20 +1287,8 @@ k_solute_zl(View V, int cur, int nxt)
     issue(1);
     issue(2);
     issue(3);
-    if constexpr (AM)
-    {
-        beam_tab_terms(c, *beam, ty * 64 + lane, 64 * BY);
-        beam_tab_plane(c, s_z[1], k0, ty * 64 + lane, 64 * BY);
-    }
-    double t_row = 0.0;                          // 2-D runs: the row's temperature (all planes)
-    if constexpr (!AM)
-    {
-        if (c.gdimz == 1)
-            t_row = temp_model<false>(c, sim_time, x, j, k0);
-        else
-            for (int e = ty * 64 + lane; e < n; e += 64 * BY)
-                s_T[e] = temp_model<false>(c, sim_time, x0, j0, k0 + e);   // read after the loop's first barrier
-    }
+    beam_tab_terms(c, *beam, ty * 64 + lane, 64 * BY);
+    beam_tab_plane(c, s_z[1], k0, ty * 64 + lane, 64 * BY);
     zl_wait<2 * L::NPW>();                       // planes k0 - 1 and k0 have landed
     __syncthreads();
     double clm = cl_at(0, ty + 1, lane + 1), fsm = fs_at(0, ty + 1, lane + 1);
@@ -1226,9 +1302,8 @@ k_solute_zl(View V, int cur, int nxt)
         zl_wait<L::NPW>();                       // this wave's share of plane k + 1 has landed
         __syncthreads();                         // every wave's share; the slot of plane k - 1 is free
         issue(s + 3);
-        if constexpr (AM)
-            if (s < n)
-                beam_tab_plane(c, s_z[(s + 1) & 1], k + 1, ty * 64 + lane, 64 * BY);
+        if (s < n)
+            beam_tab_plane(c, s_z[(s + 1) & 1], k + 1, ty * 64 + lane, 64 * BY);
         const double clp = cl_at(q1, ty + 1, lane + 1), fsp = fs_at(q1, ty + 1, lane + 1);
         int g_new = 0;
         if (active)
@@ -1252,14 +1327,7 @@ k_solute_zl(View V, int cur, int nxt)
             int branch;
             partition_cell(
                 c,
-                [&]() {
-                    if constexpr (AM)
-                        return beam_temp_tab(c, *beam, s_z[s & 1], sim_time, x, j, k);
-                    else if (c.beam_sep)
-                        return G(b.temp)[idx];
-                    else
-                        return c.gdimz == 1 ? t_row : s_T[s - 1];
-                },
+                [&]() { return beam_temp_tab(c, *beam, s_z[s & 1], sim_time, x, j, k); },
                 ce_new, ce_old, clv, fsv, g_old, &cl_out, &fs_out, &g_new, &branch);
             st_cl<F32>(b, c, nxt, idx, cl_out);
             st_stream(fsn_out, idx, fs_out);
@@ -2195,7 +2263,7 @@ hipError_t launch_halo_exchange(const View &v, int phase, int cb, long long max_
 // zm_by: rows of the z-marching kernel (all domains of a view share it); 0
 // selects the cell-parallel kernel.
 template <bool AM, bool F32>
-static void launch_solute_t(const View &v, int zm_by, int lds, int diff, int fsc, int rec, int cur, int nxt,
+static void launch_solute_t(const View &v, int zm_by, int tf, int diff, int fsc, int rec, int cur, int nxt,
                             hipStream_t s)
 {
     dim3 blk(SOL_BX, SOL_BY);
@@ -2207,26 +2275,34 @@ static void launch_solute_t(const View &v, int zm_by, int lds, int diff, int fsc
                                cur, nxt);
         return;
     }
-    if (diff && fsc && zm_by > 0 && lds)
+    const unsigned ng = (unsigned) ((v.tot_zm + 8ll * v.xcd_run - 1) / (8ll * v.xcd_run) * (8ll * v.xcd_run));
+    if (!AM && diff && fsc && zm_by > 0)
     {
-        const long long ng = v.xcd_remap ? ((v.tot_zm + 7) / 8) * 8 : v.tot_zm;
-        const size_t tlds = AM ? 0 : (size_t) v.zm_planes_max * sizeof(double);   // per-plane temperatures
-        if (zm_by == 16)
-            hipLaunchKernelGGL((k_solute_zl<16, AM, F32>), dim3((unsigned) ng), dim3(64, 16), tlds, s, v, cur, nxt);
-        else if (zm_by == 8)
-            hipLaunchKernelGGL((k_solute_zl<8, AM, F32>), dim3((unsigned) ng), dim3(64, 8), tlds, s, v, cur, nxt);
+        const size_t tlds = tf ? 0 : (size_t) std::max(v.zm_planes_max, 16) * sizeof(double);   // per plane or row
+        const dim3 wg(64, zm_by == 16 ? 8 : 4);      // waves of 2 rows (of 1 row for 4-row tiles)
+        if (zm_by == 4)
+        {
+            if (tf)
+                hipLaunchKernelGGL((k_solute_rw<1, F32, true>), dim3(ng), wg, tlds, s, v, cur, nxt);
+            else
+                hipLaunchKernelGGL((k_solute_rw<1, F32, false>), dim3(ng), wg, tlds, s, v, cur, nxt);
+        }
+        else if (tf)
+            hipLaunchKernelGGL((k_solute_rw<2, F32, true>), dim3(ng), wg, tlds, s, v, cur, nxt);
         else
-            hipLaunchKernelGGL((k_solute_zl<4, AM, F32>), dim3((unsigned) ng), dim3(64, 4), tlds, s, v, cur, nxt);
+            hipLaunchKernelGGL((k_solute_rw<2, F32, false>), dim3(ng), wg, tlds, s, v, cur, nxt);
     }
     else if (diff && fsc && zm_by > 0)
     {
-        const long long ng = v.xcd_remap ? ((v.tot_zm + 7) / 8) * 8 : v.tot_zm;
-        if (zm_by == 16)
-            hipLaunchKernelGGL((k_solute_zm<16, AM, F32>), dim3((unsigned) ng), dim3(64, 16), 0, s, v, cur, nxt);
-        else if (zm_by == 8)
-            hipLaunchKernelGGL((k_solute_zm<8, AM, F32>), dim3((unsigned) ng), dim3(64, 8), 0, s, v, cur, nxt);
-        else
-            hipLaunchKernelGGL((k_solute_zm<4, AM, F32>), dim3((unsigned) ng), dim3(64, 4), 0, s, v, cur, nxt);
+        if constexpr (AM)
+        {
+            if (zm_by == 16)
+                hipLaunchKernelGGL((k_solute_zl<16, F32>), dim3(ng), dim3(64, 16), 0, s, v, cur, nxt);
+            else if (zm_by == 8)
+                hipLaunchKernelGGL((k_solute_zl<8, F32>), dim3(ng), dim3(64, 8), 0, s, v, cur, nxt);
+            else
+                hipLaunchKernelGGL((k_solute_zl<4, F32>), dim3(ng), dim3(64, 4), 0, s, v, cur, nxt);
+        }
     }
     else if (diff && fsc)
         hipLaunchKernelGGL((k_solute<true, true, AM, F32>), dim3((unsigned) v.tot_cell), blk, 0, s, v, cur, nxt);
@@ -2240,22 +2316,22 @@ static void launch_solute_t(const View &v, int zm_by, int lds, int diff, int fsc
                            nxt);
 }
 
-hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int lds, int diff, int fsc, int rec, int cur,
+hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int tf, int diff, int fsc, int rec, int cur,
                          int nxt, hipStream_t s)
 {
     if (am)
     {
         if (f32)
-            launch_solute_t<true, true>(v, zm_by, lds, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<true, true>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
         else
-            launch_solute_t<true, false>(v, zm_by, lds, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<true, false>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
     }
     else
     {
         if (f32)
-            launch_solute_t<false, true>(v, zm_by, lds, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<false, true>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
         else
-            launch_solute_t<false, false>(v, zm_by, lds, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<false, false>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
     }
     return hipGetLastError();
 }
