@@ -34,6 +34,8 @@ long long zm_tiles(const Consts &c, int by);
 hipError_t launch_reduce(const DevBufs &b, const Consts &c, int cb, double *out2, hipStream_t s);
 hipError_t launch_fill_temp(const DevBufs &b, const Consts &c, double *out, hipStream_t s);
 hipError_t launch_grow_octahedra(const DevBufs &b, const Consts &c, int cb, hipStream_t s);
+hipError_t launch_gather_counters(const View &v, Counters *out, hipStream_t s);
+hipError_t launch_reset_new_grains(const View &v, hipStream_t s);
 hipError_t launch_fill_f64(double *p, long long n, double v, hipStream_t s);
 hipError_t launch_eval_exp(const double *x, double *y, long long n, hipStream_t s);
 hipError_t launch_probe(int mix, long long n, double *a, double *b, double *f, float *ea, float *eb, int *g,
@@ -82,6 +84,9 @@ struct mmca_ctx {
     int rand_filled = 0;
     int rand_capacity = 0;
     double *d_red = nullptr;           // 2 doubles
+    // counters of the chunks of steps in flight (pinned), and their events
+    Counters *h_chunk = nullptr;
+    hipEvent_t chunk_ev[2] = { nullptr, nullptr };
     // device view of this context as a one-domain launch
     DomainDesc *d_desc = nullptr;
     long long *d_off = nullptr;
@@ -175,6 +180,18 @@ int ensure_random(mmca_ctx *ctx, long long upto)
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->rand_filled = (int) upto;
     return MMCA_OK;
+}
+
+// Orientations are drawn on the host ahead of the steps that may use them: at
+// most one per nucleation site and step, mostly none.  The queue holds the
+// worst case of two chunks of this many steps (a restart draws it anew), and
+// mmca_step looks at the counters of one chunk while the next one runs.  A
+// draw costs 52 ns: the former queue of 256 per site (at least 65536) took
+// 3 ms for a small block and 60 ms for the 6900 sites of the 256 x 256 x 512
+// directional block, at every restart.
+long long chunk_steps(const mmca_ctx *ctx)
+{
+    return std::min<long long>(64, std::max<long long>(4, 2048 / std::max(1, ctx->b.nsites)));
 }
 
 // After mmca_rand: the queued orientations past the consumed ones were drawn
@@ -574,6 +591,9 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
     b.nblk_red = reduce_blocks(c);
     TRY(dev_alloc(&b.red_part, (size_t) 2 * b.nblk_red));
     TRY(dev_alloc(&ctx->d_red, 2));
+    HIPCHK(hipHostMalloc((void **) &ctx->h_chunk, 2 * sizeof(Counters), hipHostMallocDefault));
+    for (int i = 0; i < 2; i++)
+        HIPCHK(hipEventCreateWithFlags(&ctx->chunk_ev[i], hipEventDisableTiming));
     const size_t G = (size_t) ctx->p.max_total_grains + 1;
     TRY(dev_alloc(&b.g_rot, G * 9));
     TRY(dev_alloc(&b.g_cell, G));
@@ -642,6 +662,11 @@ int mmca_destroy(mmca_ctx *ctx)
             (void) hipFree(p);
     for (auto e : ctx->ev)
         (void) hipEventDestroy(e);
+    for (auto e : ctx->chunk_ev)
+        if (e)
+            (void) hipEventDestroy(e);
+    if (ctx->h_chunk)
+        (void) hipHostFree(ctx->h_chunk);
     if (ctx->stream)
         (void) hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -695,8 +720,7 @@ int mmca_init_nucleation(mmca_ctx *ctx, const mmca_nucleation_cfg *cfg)
     ctx->q0 = 0;
     ctx->rand_dirty = false;
     // draw the first orientations now, outside any timed stepping
-    TRY(ensure_random(ctx, std::min<long long>(ctx->rand_capacity,
-                                               std::max<long long>(65536, 256LL * (long long) ns))));
+    TRY(ensure_random(ctx, 2 * chunk_steps(ctx) * (long long) ns));
     return MMCA_OK;
 }
 
@@ -725,21 +749,32 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
         TRY(push_counters(ctx));
     } else {
         // Steps are issued in chunks small enough that the orientations
-        // already drawn cover every grain the chunk can create (at most one
-        // per site and step); the counters are read back between chunks.
-        int done = 0;
-        while (done < nsteps) {
+        // already drawn cover every grain they can create (at most one per
+        // site and step); two chunks are in flight, and the counters of the
+        // older one, read while the newer runs, say how many were used.
+        const long long ns = ctx->b.nsites, ch = chunk_steps(ctx);
+        long long used = ctx->hc.random_used, flight[2] = { 0, 0 };
+        int done = 0, first = 0, nflight = 0;
+        while (done < nsteps && ctx->hc.status == MMCA_OK) {
             long long k = nsteps - done;
-            if (ctx->b.nsites > 0 && ctx->rand_filled < ctx->rand_capacity) {
-                long long spare = (long long) ctx->rand_filled - ctx->hc.random_used;
-                if (spare < (long long) ctx->b.nsites * 16) {
-                    long long want = (long long) ctx->hc.random_used +
-                                     std::max((long long) ctx->b.nsites * 256, 2 * spare + 65536);
-                    TRY(ensure_random(ctx, want));
-                    spare = (long long) ctx->rand_filled - ctx->hc.random_used;
+            if (ns > 0 && ctx->rand_filled < ctx->rand_capacity) {
+                if (nflight == 2) {
+                    HIPCHK(hipEventSynchronize(ctx->chunk_ev[first]));
+                    used = ctx->h_chunk[first].random_used;
+                    ctx->hc.status = ctx->h_chunk[first].status;
+                    flight[first] = 0;
+                    first ^= 1;
+                    nflight--;
+                    continue;
+                }
+                const long long pend = flight[0] + flight[1];
+                long long cover = (ctx->rand_filled - used) / ns - pend;
+                if (cover < std::min(k, (ch + 1) / 2)) {
+                    TRY(ensure_random(ctx, used + (pend + 2 * ch) * ns));
+                    cover = (ctx->rand_filled - used) / ns - pend;
                 }
                 if (ctx->rand_filled < ctx->rand_capacity)
-                    k = std::min(k, spare / ctx->b.nsites);
+                    k = std::min({ k, ch, cover });
             }
             if (k < 1)
                 return MMCA_ERR_STATE;
@@ -747,9 +782,12 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
                 TRY(enqueue_iteration(ctx, true));
             done += (int) k;
             if (done < nsteps) {
-                TRY(sync_counters(ctx));
-                if (ctx->hc.status != MMCA_OK)
-                    break;
+                const int slot = (first + nflight) & 1;
+                HIPCHK(hipMemcpyAsync(&ctx->h_chunk[slot], ctx->b.cnt, sizeof(Counters), hipMemcpyDeviceToHost,
+                                      ctx->stream));
+                HIPCHK(hipEventRecord(ctx->chunk_ev[slot], ctx->stream));
+                flight[slot] = k;
+                nflight++;
             }
         }
         if (want_sums)
@@ -1460,7 +1498,6 @@ int load_block(mmca_ctx *ctx, StateIO &io, TablePart table, StateHeader *out_h, 
     ctx->rand_filled = hc.random_used;
     ctx->rand_dirty = false;
     ctx->have_oce = false;
-    ctx->view_dirty = true;
     ctx->hc = hc;
     TRY(push_counters(ctx));
     if (out_h)
@@ -1716,6 +1753,9 @@ struct mmca_batch {
     int cap = 0;
     View view;
     bool view_dirty = true;
+    // counters of all domains: gathered on the device, and their pinned copy
+    Counters *d_cnt = nullptr, *h_cnt = nullptr;
+    double *d_sums = nullptr;    // 2 per domain (k_reduce_final)
     int cur = 0;
     int zm_planes = 8, zm_by = 4;      // default_tile at creation
     int xcd_remap = 0, zm_lds = 1, capture_chunk = 0, capture_band = 0, track_d = 0;
@@ -1758,12 +1798,28 @@ int batch_view(mmca_batch *bt)
     return MMCA_OK;
 }
 
+// the counters of every domain: one gather on the device, one copy
 int batch_sync(mmca_batch *bt)
 {
-    for (mmca_ctx *c : bt->dom)
-        HIPCHK(hipMemcpyAsync(&c->hc, c->b.cnt, sizeof(Counters), hipMemcpyDeviceToHost, bt->stream));
+    TRY(batch_view(bt));
+    HIPCHK(launch_gather_counters(bt->view, bt->d_cnt, bt->stream));
+    HIPCHK(hipMemcpyAsync(bt->h_cnt, bt->d_cnt, bt->dom.size() * sizeof(Counters), hipMemcpyDeviceToHost,
+                          bt->stream));
     HIPCHK(hipStreamSynchronize(bt->stream));
+    for (size_t d = 0; d < bt->dom.size(); d++)
+        bt->dom[d]->hc = bt->h_cnt[d];
     return MMCA_OK;
+}
+
+// Steps whose worst case of grains the orientation queues of a batch cover
+// after they were topped up (chunk_steps, with one look at the counters of
+// all domains per chunk and no second chunk in flight).
+long long batch_chunk_steps(const mmca_batch *bt)
+{
+    long long ns = 0;
+    for (const mmca_ctx *c : bt->dom)
+        ns += c->b.nsites;
+    return std::min<long long>(64, std::max<long long>(8, 32768 / std::max<long long>(1, ns)));
 }
 
 // one doiteration() of every domain: seven launches whatever the batch size
@@ -1853,6 +1909,9 @@ int mmca_batch_create(const mmca_params *params, const mmca_nucleation_cfg *nucl
     default_tile(cs.data(), ndomains, &bt->zm_planes, &bt->zm_by);
     HIPCHK(hipSetDevice(device));
     HIPCHK(hipStreamCreate(&bt->stream));
+    TRY(dev_alloc(&bt->d_cnt, (size_t) ndomains));
+    TRY(dev_alloc(&bt->d_sums, (size_t) 2 * ndomains));
+    HIPCHK(hipHostMalloc((void **) &bt->h_cnt, (size_t) ndomains * sizeof(Counters), hipHostMallocDefault));
     for (mmca_ctx *c : bt->dom)
         HIPCHK(hipStreamSynchronize(c->stream));
     return MMCA_OK;
@@ -1997,7 +2056,6 @@ int mmca_batch_load_state(mmca_batch *bt, const void *buf, int64_t size)
             return MMCA_ERR_ARG;
     }
     bt->cur = h.cur;
-    bt->view_dirty = true;
     return MMCA_OK;
 }
 
@@ -2017,6 +2075,12 @@ int mmca_batch_destroy(mmca_batch *bt)
         (void) hipFree(bt->d_desc);
     if (bt->d_off)
         (void) hipFree(bt->d_off);
+    if (bt->d_cnt)
+        (void) hipFree(bt->d_cnt);
+    if (bt->d_sums)
+        (void) hipFree(bt->d_sums);
+    if (bt->h_cnt)
+        (void) hipHostFree(bt->h_cnt);
     for (mmca_ctx *c : bt->dom)
         mmca_destroy(c);
     if (bt->stream)
@@ -2117,11 +2181,10 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
     HIPCHK(hipSetDevice(bt->device));
     TRY(batch_view(bt));
     TRY(batch_sync(bt));
+    HIPCHK(launch_reset_new_grains(bt->view, bt->stream));
     for (mmca_ctx *c : bt->dom) {
         TRY(replan_random(c));
         c->hc.new_grains = 0;
-        HIPCHK(hipMemcpyAsync(&c->b.cnt->new_grains, &c->hc.new_grains, sizeof(int), hipMemcpyHostToDevice,
-                              bt->stream));
         int st = courant_check(c);
         if (st != MMCA_OK && nsteps > 0 && c->hc.status == MMCA_OK) {
             c->hc.status = st;
@@ -2135,6 +2198,7 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
     std::vector<std::pair<int, uint64_t>> start(bt->dom.size());
     for (size_t d = 0; d < bt->dom.size(); d++)
         start[d] = { bt->dom[d]->cur, bt->dom[d]->hc.timestep };
+    const long long ch = batch_chunk_steps(bt);
     int done = 0;
     while (done < nsteps) {
         // chunk bound: drawn orientations cover every grain the chunk can create
@@ -2142,11 +2206,10 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
         for (mmca_ctx *c : bt->dom) {
             if (c->b.nsites == 0 || c->rand_filled >= c->rand_capacity || c->hc.status != MMCA_OK)
                 continue;
+            const long long ns = c->b.nsites;
             long long spare = (long long) c->rand_filled - c->hc.random_used;
-            if (spare < (long long) c->b.nsites * 16) {
-                long long want = (long long) c->hc.random_used +
-                                 std::max((long long) c->b.nsites * 256, 2 * spare + 65536);
-                TRY(ensure_random(c, want));
+            if (spare < std::min<long long>(k, ch / 2) * ns) {
+                TRY(ensure_random(c, (long long) c->hc.random_used + std::min<long long>(k, ch) * ns));
                 spare = (long long) c->rand_filled - c->hc.random_used;
             }
             if (c->rand_filled < c->rand_capacity)
@@ -2171,8 +2234,12 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
         mmca_ctx *c = bt->dom[d];
         c->cur = c->hc.status == MMCA_OK ? bt->cur : start[d].first ^ (int) ((c->hc.timestep - start[d].second) & 1);
         if (want_sums)
-            HIPCHK(launch_reduce(c->b, c->c, c->cur, c->d_red, bt->stream));
+            HIPCHK(launch_reduce(c->b, c->c, c->cur, bt->d_sums + 2 * d, bt->stream));
     }
+    std::vector<double> sums(2 * bt->dom.size());
+    if (want_sums)
+        HIPCHK(hipMemcpyAsync(sums.data(), bt->d_sums, sums.size() * sizeof(double), hipMemcpyDeviceToHost,
+                              bt->stream));
     TRY(batch_sync(bt));
     if (bt->timing) {
         double tot = 0.0;
@@ -2203,10 +2270,8 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
         r->status = c->hc.status;
         r->failed_step = c->hc.failed_step;
         if (want_sums && c->hc.status == MMCA_OK) {
-            double s2[2];
-            HIPCHK(hipMemcpy(s2, c->d_red, sizeof(s2), hipMemcpyDeviceToHost));
-            r->solid_sum = s2[0];
-            r->solute_sum = s2[1];
+            r->solid_sum = sums[2 * d];
+            r->solute_sum = sums[2 * d + 1];
             if (c->c.f32) {
                 r->solute_sum += (double) c->c.nx * c->c.ny * c->c.nz * c->c.cinit;
                 TRY(read_ledger(c, &r->solute_ledger));

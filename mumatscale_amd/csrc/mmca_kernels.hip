@@ -2375,6 +2375,33 @@ hipError_t launch_capture_only(const View &v, const DevBufs &b, int cb, hipStrea
     return hipGetLastError();
 }
 
+// the counters of every domain of a view, side by side
+__global__ void __launch_bounds__(64)
+k_gather_counters(View V, Counters *out)
+{
+    for (int d = blockIdx.x * 64 + threadIdx.x; d < V.ndom; d += 64 * gridDim.x)
+        out[d] = *V.dom[d].b.cnt;
+}
+
+hipError_t launch_gather_counters(const View &v, Counters *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_gather_counters, dim3((unsigned) std::min(1024, (v.ndom + 63) / 64)), dim3(64), 0, s, v, out);
+    return hipGetLastError();
+}
+
+__global__ void __launch_bounds__(64)
+k_reset_new_grains(View V)
+{
+    for (int d = blockIdx.x * 64 + threadIdx.x; d < V.ndom; d += 64 * gridDim.x)
+        V.dom[d].b.cnt->new_grains = 0;
+}
+
+hipError_t launch_reset_new_grains(const View &v, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_reset_new_grains, dim3((unsigned) std::min(1024, (v.ndom + 63) / 64)), dim3(64), 0, s, v);
+    return hipGetLastError();
+}
+
 int reduce_blocks(const Consts &c)
 {
     long long N = (long long) c.nx * c.ny * c.nz;
