@@ -331,12 +331,13 @@ int  mmca_orientation_draws(const mmca_params *params, const mmca_nucleation_cfg
 #define MMCA_TUNE_TRACK_D    6   /* 1: keep d as the reference's array holds it (growth.c:392-403 writes
                                     solid cells only, so a cell that melts keeps its last value);
                                     MMCA_FIELD_D then gives that array */
-#define MMCA_TUNE_BEAM_SEP   7   /* FP32-deviation Gaussian-beam blocks only (default 1 there): the
-                                    beam temperature (temperature.c:104-112) as the sum over its 400
-                                    nodes of the product of an x, a y and a z factor, computed per
-                                    step for the whole block (within 1e-13 of the quadrature,
-                                    not its bits); 0: the quadrature per cell.  FP64 storage
-                                    always uses the quadrature (value 1 is refused there) */
+#define MMCA_TUNE_BEAM_SEP   7   /* FP32-deviation Gaussian-beam blocks only (default 1 there): temperature
+                                    outputs of the interior (MMCA_FIELD_TEMP, mmca_io_fields) from the sum
+                                    over the quadrature's 400 nodes (temperature.c:104-112) of the product
+                                    of an x, a y and a z factor, within 1e-13 of the quadrature; 0: the
+                                    quadrature per cell.  FP64 storage always gives the quadrature (value
+                                    1 is refused there).  The step uses the quadrature's value, bit for
+                                    bit, in every case */
 #define MMCA_TUNE_CAPTURE_BAND 8 /* >0: capture works on units of this many rows of one plane, band q
                                      of every plane on XCD q % 8, units taken plane by plane; used
                                      when the block has at least 8 bands and the step builds the

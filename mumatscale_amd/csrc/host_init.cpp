@@ -236,6 +236,100 @@ int build_consts(const mmca_params &p, Consts &c)
     return MMCA_OK;
 }
 
+// Factor of the beam's x dependence at time t behind the beam, for a cell lx
+// ahead of it (temperature.c:104-112)
+static double beam_x_factor(const Consts &c, double lx, double t)
+{
+    const double ls = c.lsd / (2. * 1.414), lalpha = c.lthcon / (c.rho * c.lcp);
+    const double u = lx + c.lv * t;
+    return exp(-(u * u) / (ls * ls + 4. * lalpha * t));
+}
+
+// Chebyshev points of the quadrature's time range, and the Lagrange
+// polynomials through them at its BEAM_NT nodes (barycentric form)
+void beam_interpolation(const Consts &c, int r, std::vector<double> &tau, std::vector<double> &weights)
+{
+    const double invlv = 1. / c.lv, lalpha = c.lthcon / (c.rho * c.lcp);
+    const double ldt = 20 * lalpha * invlv * invlv / BEAM_NT;
+    tau.resize(r);
+    weights.assign((size_t) BEAM_NT * r, 0.0);
+    if (r == BEAM_NT) {                         // the nodes themselves
+        for (int i = 0; i < r; i++) {
+            tau[i] = (0.5 + i) * ldt;
+            weights[(size_t) i * r + i] = 1.0;
+        }
+        return;
+    }
+    std::vector<double> bw(r);
+    for (int j = 0; j < r; j++) {
+        const double a = (2 * j + 1) * M_PI / (2 * r);
+        tau[j] = 0.5 * BEAM_NT * ldt + 0.5 * (BEAM_NT - 1) * ldt * cos(a);
+        bw[j] = (j & 1 ? -1.0 : 1.0) * sin(a);
+    }
+    for (int i = 0; i < BEAM_NT; i++) {
+        const double t = (0.5 + i) * ldt;
+        double *w = &weights[(size_t) i * r], sum = 0.0;
+        int hit = -1;
+        for (int j = 0; j < r; j++) {
+            if (t == tau[j])
+                hit = j;
+            w[j] = bw[j] / (t - tau[j]);
+            sum += w[j];
+        }
+        for (int j = 0; j < r; j++)
+            w[j] = hit >= 0 ? (j == hit ? 1.0 : 0.0) : w[j] / sum;
+    }
+}
+
+// The smallest number of interpolation points that reproduces the beam's x
+// factor to 1e-9 at every node, for cells from 7 widths ahead of the beam to 7
+// widths behind its tail (beyond, it is below 1e-21), and the bound that
+// follows for the temperature with a margin of 10; the nodes themselves when
+// 96 points are not enough.  The AM track's beam (spot 130 um, 0.8 m/s,
+// diffusivity 5e-6 m^2/s) needs 32.
+void plan_beam(Consts &c)
+{
+    const double invlv = 1. / c.lv, lalpha = c.lthcon / (c.rho * c.lcp);
+    const double ldt = 20 * lalpha * invlv * invlv / BEAM_NT, ls = c.lsd / (2. * 1.414);
+    const double A0 = ls * ls + 4. * lalpha * 0.5 * ldt, A1 = ls * ls + 4. * lalpha * (BEAM_NT - 0.5) * ldt;
+    const double lo = -(c.lv * BEAM_NT * ldt + 7 * sqrt(A1)), hi = 7 * sqrt(A1);
+    double peak = 0.0;                          // largest sum of terms: every factor is at most 1
+    for (int i = 0; i < BEAM_NT; i++) {
+        const double t = (0.5 + i) * ldt;
+        peak += ldt / (sqrt(lalpha * t) * (ls * ls + 4. * lalpha * t));
+    }
+    c.beam_tol = 1e-8 * fabs(c.lab * c.lpow * lalpha / (5.568328 * c.lthcon)) * peak;
+    c.beam_rank = BEAM_NT;
+    std::vector<double> tau, w;
+    for (int r = 16; r <= 96; r += 16) {
+        beam_interpolation(c, r, tau, w);
+        bool good = true;
+        std::vector<double> x(r);
+        for (int p = 0; p <= 96 && good; p++) {
+            const double lx = lo + (hi - lo) * p / 96;
+            for (int j = 0; j < r; j++)
+                x[j] = beam_x_factor(c, lx, tau[j]);
+            for (int i = 0; i < BEAM_NT && good; i += 3) {
+                double v = 0.0;
+                for (int j = 0; j < r; j++)
+                    v += w[(size_t) i * r + j] * x[j];
+                good = fabs(v - beam_x_factor(c, lx, (0.5 + i) * ldt)) < 1e-9;
+            }
+        }
+        if (good) {
+            c.beam_rank = r;
+            break;
+        }
+    }
+    // ranges in which div_by is exact: no intermediate leaves the exponent range
+    auto in = [](double v, double a, double b) { return fabs(v) >= a && fabs(v) <= b; };
+    const double T0 = sqrt(lalpha * 0.5 * ldt) * A0, T1 = sqrt(lalpha * (BEAM_NT - 0.5) * ldt) * A1;
+    c.beam_fast = in(c.cell_size, 1e-30, 1e30) && in(c.lv * 0.5 * ldt, 1e-60, 1e30) && in(A0, 1e-100, 1e100) &&
+                  in(A1, 1e-100, 1e100) && in(T0, 1e-100, 1e100) && in(T1, 1e-100, 1e100) && in(ldt, 1e-25, 1e30);     // exp(-512) * ldt > 1e-250
+    for (double v : { c.origin[0], c.origin[1], c.origin[2], c.x0, c.y0, c.z0, c.lhs, c.lsd })
+        c.beam_fast = c.beam_fast && fabs(v) <= 1e30;
+}
+
 // direct_temp_calc on the host, for the initial lsindex of AM sites
 // (tempPrepareSB_int, temperature.c:156-192)
 double host_temp(const Consts &c, double sim_time, int x, int y, int z)

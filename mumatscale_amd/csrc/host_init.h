@@ -47,6 +47,11 @@ long long padded_cells(const mmca_params &p);
 int build_consts(const mmca_params &p, Consts &c);
 // tile of the solute kernel for n domains advanced together
 void default_tile(const Consts *const *doms, int n, int *planes, int *rows);
+// beam_rank, beam_tol and beam_fast of a beam block
+void plan_beam(Consts &c);
+// interpolation of the beam's x factors between `rank` times: the times and the
+// weights (BEAM_NT x rank)
+void beam_interpolation(const Consts &c, int rank, std::vector<double> &tau, std::vector<double> &weights);
 double host_temp(const Consts &c, double sim_time, int x, int y, int z);
 void rotmat_of(double a0, double a1, double a2, double *R);
 int plan_nucleation(const mmca_params &params, const Consts &c, const mmca_nucleation_cfg *cfg,

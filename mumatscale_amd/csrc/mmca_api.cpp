@@ -18,9 +18,12 @@
 
 namespace mmca {
 hipError_t launch_nucleate(const View &v, int mode, int cur, hipStream_t s);
-hipError_t launch_beam_field(const DevBufs &b, const Consts &c, int adv, hipStream_t s);
-hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int tf, int diff, int fsc, int rec, int cur, int nxt,
+hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int diff, int fsc, int rec, int cur, int nxt,
                          hipStream_t s);
+hipError_t launch_beam_nodes(const DevBufs &b, const Consts &c, hipStream_t s);
+hipError_t launch_beam_field(const DevBufs &b, const Consts &c, const BeamSet &p, int out, int adv, int rows,
+                             hipStream_t s);
+hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStream_t s);
 hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s);
 hipError_t launch_list(const View &v, int cb, int capture, int decide_realloc, hipStream_t s);
 hipError_t launch_nucleate_coupled(const View &v, int cur, hipStream_t s);
@@ -69,6 +72,10 @@ struct mmca_ctx {
     hipStream_t stream = nullptr;
     int device = 0;
     int cur = 0;                 // buffer index of the latest cl/fs
+    // beam blocks: the points of the approximate temperature and of the
+    // separable outputs, and whether the former's row factors are built
+    BeamSet beam_step = {}, beam_out = {};
+    bool beam_rows = false;
     bool have_oce = false;       // single-operator diffusion ran
     // host mirror of the counters after the last synchronisation
     Counters hc;
@@ -242,35 +249,71 @@ int check_grain_ids(const void *gr, size_t n, long long max_total_grains)
     return MMCA_OK;
 }
 
-// buffers of the separable beam temperature (Consts::beam_sep)
+// a point set of k_beam_field with its tables
+int make_beam_set(mmca_ctx *ctx, int rank, BeamSet *p)
+{
+    const Consts &c = ctx->c;
+    const size_t r = (size_t) rank;
+    std::vector<double> tau, weights;
+    beam_interpolation(c, rank, tau, weights);
+    // x factors in whole 128-column tiles, row factors in whole 64-row tiles (zero past ny nz)
+    const size_t wrows = ((size_t) c.ny * c.nz + 63) / 64 * 64;
+    p->rank = rank;
+    TRY(dev_alloc(&p->tau, r));
+    if (rank != BEAM_NT)
+        TRY(dev_alloc(&p->weights, (size_t) BEAM_NT * r));
+    TRY(dev_alloc(&p->ax, r * ((c.nx + 127) / 128 * 128)));
+    TRY(dev_alloc(&p->aw, wrows * r));
+    HIPCHK(hipMemsetAsync(p->aw, 0, wrows * r * sizeof(double), ctx->stream));
+    const double key[2] = { NAN, 1.0 };          // no position yet: the row factors are built on first use
+    HIPCHK(hipMemcpyAsync(p->tau, tau.data(), r * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    if (p->weights)
+        HIPCHK(hipMemcpyAsync(p->weights, weights.data(), weights.size() * sizeof(double), hipMemcpyHostToDevice,
+                              ctx->stream));
+    TRY(dev_alloc(&p->key, 2));
+    HIPCHK(hipMemcpyAsync(p->key, key, sizeof(key), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return MMCA_OK;
+}
+
+// buffers of a beam block's step
 int ensure_beam(mmca_ctx *ctx)
 {
     DevBufs &b = ctx->b;
     const Consts &c = ctx->c;
-    if (!b.temp) {
-        // X rows of whole 128-column tiles, W rows in whole 64-row tiles (zero past ny nz)
-        const size_t wrows = ((size_t) c.ny * c.nz + 63) / 64 * 64;
-        TRY(dev_alloc(&b.temp, (size_t) c.P));
-        TRY(dev_alloc(&b.beam_x, (size_t) BEAM_NT * ((c.nx + 127) / 128 * 128)));
-        TRY(dev_alloc(&b.beam_y, (size_t) BEAM_NT * c.ny));
-        TRY(dev_alloc(&b.beam_z, (size_t) BEAM_NT * c.nz));
-        TRY(dev_alloc(&b.beam_w, (size_t) BEAM_NT * wrows));
-        TRY(dev_alloc(&b.beam_key, 2));
-        HIPCHK(hipMemsetAsync(b.temp, 0, (size_t) c.P * sizeof(double), ctx->stream));
-        HIPCHK(hipMemsetAsync(b.beam_w, 0, (size_t) BEAM_NT * wrows * sizeof(double), ctx->stream));
-        const double key[2] = { NAN, 1.0 };      // no position yet: W is built on the first step
-        HIPCHK(hipMemcpyAsync(b.beam_key, key, sizeof(key), hipMemcpyHostToDevice, ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));
-        ctx->view_dirty = true;
-    }
+    TRY(dev_alloc(&b.beam_nodes, (size_t) 5 * BEAM_NT));
+    TRY(dev_alloc(&b.beam_zq, (size_t) BEAM_NT * (c.nz + 2)));
+    TRY(dev_alloc(&b.temp32, (size_t) c.P));
+    TRY(dev_alloc(&b.und, (size_t) c.nx * c.ny * c.nz));
+    TRY(dev_alloc(&b.und_n, 1));
+    HIPCHK(hipMemsetAsync(b.temp32, 0, (size_t) c.P * sizeof(float), ctx->stream));
+    HIPCHK(hipMemsetAsync(b.und_n, 0, sizeof(int), ctx->stream));
+    HIPCHK(launch_beam_nodes(b, c, ctx->stream));
+    return make_beam_set(ctx, c.beam_rank, &ctx->beam_step);
+}
+
+// the approximate beam temperature of timestep + adv, before the kernels that read it
+int refresh_beam(mmca_ctx *ctx, int adv, hipStream_t s)
+{
+    if (!ctx->c.am)
+        return MMCA_OK;
+    // the row factors change with the track only
+    HIPCHK(launch_beam_field(ctx->b, ctx->c, ctx->beam_step, 0, adv, ctx->c.am_tracks > 1 || !ctx->beam_rows, s));
+    ctx->beam_rows = true;
     return MMCA_OK;
 }
 
-// the separable beam field of timestep + adv, before a kernel that reads it
-int refresh_beam(mmca_ctx *ctx, int adv, hipStream_t s)
+// the temperature of a beam block at the current timestep into b.temp, halo included
+int beam_output(mmca_ctx *ctx)
 {
-    if (ctx->c.beam_sep)
-        HIPCHK(launch_beam_field(ctx->b, ctx->c, adv, s));
+    if (!ctx->b.temp)
+        TRY(dev_alloc(&ctx->b.temp, (size_t) ctx->c.P));
+    if (ctx->c.beam_sep) {
+        if (!ctx->beam_out.key)
+            TRY(make_beam_set(ctx, BEAM_NT, &ctx->beam_out));
+        HIPCHK(launch_beam_field(ctx->b, ctx->c, ctx->beam_out, 1, 0, 1, ctx->stream));
+    }
+    HIPCHK(launch_fill_temp(ctx->b, ctx->c, ctx->b.temp, ctx->stream));
     return MMCA_OK;
 }
 
@@ -378,8 +421,10 @@ int enqueue_iteration(mmca_ctx *ctx, bool advance)
         HIPCHK(hipEventRecord(ctx->ev[ev0], ctx->stream));
     }
     const int rec = ctx->b.rec != nullptr;
-    HIPCHK(launch_solute(ctx->view, ctx->c.am && !ctx->c.beam_sep, ctx->c.f32, rec ? 0 : zm_rows(ctx->c),
-                         ctx->c.beam_sep, 1, 1, rec, ctx->cur, nxt, ctx->stream));
+    HIPCHK(launch_solute(ctx->view, ctx->c.am, ctx->c.f32, rec ? 0 : zm_rows(ctx->c), 1, 1, rec, ctx->cur, nxt,
+                         ctx->stream));
+    if (ctx->c.am && !rec)
+        HIPCHK(launch_beam_finish(ctx->view, ctx->c.f32, ctx->cur, nxt, ctx->stream));
     if (ctx->timing) {
         HIPCHK(hipEventRecord(ctx->ev[ev0 + 1], ctx->stream));
         ctx->ev_used = ev0 + 2;
@@ -552,6 +597,8 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
         delete ctx;
         return st;
     }
+    if (ctx->c.am)
+        plan_beam(ctx->c);
     memset(&ctx->b, 0, sizeof(ctx->b));
     *out = ctx;     // destroy() frees partial allocations on failure
     HIPCHK(hipSetDevice(device));
@@ -603,7 +650,7 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
     ctx->rand_capacity = (int) ctx->p.max_total_grains;
     TRY(dev_alloc(&b.rand_rot, (size_t) ctx->rand_capacity * 9));
     TRY(dev_alloc(&b.cnt, 1));
-    if (c.beam_sep)
+    if (c.am)
         TRY(ensure_beam(ctx));
     b.nsites = 0;
     // SetupInitialConditions (setup.c:58-65): ce = cl = Cinit, all else 0
@@ -655,7 +702,9 @@ int mmca_destroy(mmca_ctx *ctx)
                      b.diff_id, b.nbr, b.dtx, b.dty, b.dtz, b.blk_count, b.row_first, b.site_idx, b.site_thr, b.site_fixed,
                      b.site_ls, b.events, b.ev_blk, b.ev_cnt, b.g_rot, b.g_cell, b.g_step, b.g_src, b.g_dom, b.fixed_rot,
                      b.rand_rot,
-                     b.oce, b.d, b.temp, b.beam_x, b.beam_y, b.beam_z, b.beam_w, b.beam_key, b.red_part, b.cnt, ctx->d_red,
+                     b.oce, b.d, b.temp, b.temp32, b.beam_nodes, b.beam_zq, b.und, b.und_n,
+                     ctx->beam_step.tau, ctx->beam_step.weights, ctx->beam_step.ax, ctx->beam_step.aw, ctx->beam_step.key,
+                     ctx->beam_out.tau, ctx->beam_out.ax, ctx->beam_out.aw, ctx->beam_out.key, b.red_part, b.cnt, ctx->d_red,
                      ctx->d_desc, ctx->d_off, ctx->io_buf };
     for (void *p : ptrs)
         if (p)
@@ -907,7 +956,7 @@ int mmca_sb_diffuse_alloy_decentered(mmca_ctx *ctx)
     HIPCHK(hipMemcpyAsync(ctx->b.oce, ctx->b.ce, (size_t) ctx->c.P * sizeof(double),
                           hipMemcpyDeviceToDevice, ctx->stream));
     TRY(ensure_view(ctx));
-    HIPCHK(launch_solute(ctx->view, ctx->c.am, 0, 0, 0, 1, 0, 0, ctx->cur, ctx->cur, ctx->stream));
+    HIPCHK(launch_solute(ctx->view, ctx->c.am, 0, 0, 1, 0, 0, ctx->cur, ctx->cur, ctx->stream));
     ctx->have_oce = true;
     return check_status(ctx);
 }
@@ -922,7 +971,7 @@ int mmca_fs_change_diffuse(mmca_ctx *ctx)
         return MMCA_ERR_STATE;
     HIPCHK(hipSetDevice(ctx->device));
     TRY(ensure_view(ctx));
-    HIPCHK(launch_solute(ctx->view, ctx->c.am, 0, 0, 0, 0, 1, 0, ctx->cur, ctx->cur, ctx->stream));
+    HIPCHK(launch_solute(ctx->view, ctx->c.am, 0, 0, 0, 1, 0, ctx->cur, ctx->cur, ctx->stream));
     return check_status(ctx);
 }
 
@@ -1092,9 +1141,14 @@ int mmca_download_field(mmca_ctx *ctx, int field, void *host)
         HIPCHK(hipStreamSynchronize(ctx->stream));
         break;
     case MMCA_FIELD_TEMP: {
+        if (c.am) {
+            TRY(beam_output(ctx));
+            HIPCHK(hipMemcpyAsync(host, b.temp, P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+            break;
+        }
         double *tmp = nullptr;
         TRY(dev_alloc(&tmp, P));
-        TRY(refresh_beam(ctx, 0, ctx->stream));
         HIPCHK(launch_fill_temp(b, c, tmp, ctx->stream));
         HIPCHK(hipMemcpyAsync(host, tmp, P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -1563,8 +1617,8 @@ int mmca_io_fields(mmca_ctx *ctx, float *fs_io, float *ce_io, float *temperature
         TRY(dev_alloc(&ctx->io_buf, 4 * P));
     float *d_fs = ctx->io_buf, *d_ce = d_fs + P, *d_t = d_ce + P;
     int *d_gr = (int *) (d_t + P);
-    if (temperature_io)
-        TRY(refresh_beam(ctx, 0, ctx->stream));
+    if (temperature_io && ctx->c.am)
+        TRY(beam_output(ctx));
     HIPCHK(launch_io_fields(ctx->b, ctx->c, ctx->cur, fs_io ? d_fs : nullptr, ce_io ? d_ce : nullptr,
                             temperature_io ? d_t : nullptr, gr_io ? d_gr : nullptr, ctx->stream));
     if (fs_io)
@@ -1676,10 +1730,7 @@ int mmca_set_tuning(mmca_ctx *ctx, int key, int value)
     case MMCA_TUNE_BEAM_SEP:
         if (value && !(ctx->c.am && ctx->c.f32))
             return MMCA_ERR_ARG;   // FP64 storage keeps the reference's quadrature
-        if (value)
-            TRY(ensure_beam(ctx));
-        ctx->c.beam_sep = value ? 1 : 0;
-        ctx->view_dirty = true;
+        ctx->c.beam_sep = value ? 1 : 0;         // read by temperature outputs only
         return MMCA_OK;
     default:
         return MMCA_ERR_ARG;
@@ -1844,8 +1895,9 @@ int batch_enqueue(mmca_batch *bt, int cur)
         }
         HIPCHK(hipEventRecord(bt->ev[e0], bt->stream));
     }
-    HIPCHK(launch_solute(bt->view, c0.am && !c0.beam_sep, c0.f32, bt->zm_planes > 0 ? bt->zm_by : 0, c0.beam_sep, 1, 1, 0,
-                         cur, nxt, bt->stream));
+    HIPCHK(launch_solute(bt->view, c0.am, c0.f32, bt->zm_planes > 0 ? bt->zm_by : 0, 1, 1, 0, cur, nxt, bt->stream));
+    if (c0.am)
+        HIPCHK(launch_beam_finish(bt->view, c0.f32, cur, nxt, bt->stream));
     if (bt->timing) {
         HIPCHK(hipEventRecord(bt->ev[e0 + 1], bt->stream));
         bt->ev_used = e0 + 2;

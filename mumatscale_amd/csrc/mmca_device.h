@@ -113,18 +113,6 @@ temp_model(const Consts &c, double sim_time, int x, int y, int z)
     return c.liniT + Tfront * Tinteg;
 }
 
-// The Gaussian-beam quadrature of temp_model<true> with the factors of its
-// 400 terms that do not depend on the cell tabulated (same operations and
-// order as temp_model<true>, so the same values):
-//   vlt[i] = lv * lt,  A[i] = ls*ls + 4.*lalpha*lt,
-//   Tl[i] = sqrt(lalpha*lt) * (ls*ls + 4.*lalpha*lt),
-//   Z[i] = lz*lz / (4.*lalpha*lt) for one plane (lz depends on z only),
-// and a copy of the exp table, so that its lookups are LDS reads.
-struct BeamTab {
-    double vlt[BEAM_NT], A[BEAM_NT], Tl[BEAM_NT], Z[BEAM_NT];
-    uint64_t exp_tab[EXP_TAB_WORDS];
-};
-
 __device__ __forceinline__ double beam_lalpha(const Consts &c) { return c.lthcon / (c.rho * c.lcp); }
 
 __device__ __forceinline__ double
@@ -135,85 +123,189 @@ beam_ldt(const Consts &c)
     return tsteady / BEAM_NT;
 }
 
-// fills vlt, A, Tl; threads tid = 0..nthreads-1 of the workgroup share the work
-__device__ __forceinline__ void
-beam_tab_terms(const Consts &c, BeamTab &t, int tid, int nthreads)
-{
-    const double ls = c.lsd / (2. * 1.414);
-    const double lalpha = beam_lalpha(c);
-    const double ldt = beam_ldt(c);
-    for (int i = tid; i < BEAM_NT; i += nthreads)
-    {
-        const double lt = (0.5 + i) * ldt;
-        t.vlt[i] = c.lv * lt;
-        t.A[i] = ls * ls + 4. * lalpha * lt;
-        t.Tl[i] = sqrt(lalpha * lt) * (ls * ls + 4. * lalpha * lt);
-    }
-    for (int i = tid; i < EXP_TAB_WORDS; i += nthreads)
-        t.exp_tab[i] = exp_tab[i];
-}
+// beam position and amplitude at sim_time (temperature.c:62-103)
+struct BeamNow {
+    double xnow, ynow, znow, Tfront;
+};
 
-// fills Z (BEAM_NT values) for padded plane z
-__device__ __forceinline__ void
-beam_tab_plane(const Consts &c, double *Z, int z, int tid, int nthreads)
+__device__ __forceinline__ BeamNow
+beam_now(const Consts &c, double sim_time)
 {
-    const double lalpha = beam_lalpha(c);
-    const double ldt = beam_ldt(c);
-    const double rz = c.origin[2] + ((c.off[2] + z) + 0.5) * c.cell_size;
-    const double lz = rz - c.z0;
-    for (int i = tid; i < BEAM_NT; i += nthreads)
-    {
-        const double lt = (0.5 + i) * ldt;
-        Z[i] = lz * lz / (4. * lalpha * lt);
-    }
-}
-
-__device__ __forceinline__ void
-beam_tab_plane(const Consts &c, BeamTab &t, int z, int tid, int nthreads)
-{
-    beam_tab_plane(c, t.Z, z, tid, nthreads);
-}
-
-// temp_model<true> on the tables; Z holds the plane factors of plane z
-__device__ __forceinline__ double
-beam_temp_tab(const Consts &c, const BeamTab &t, const double *Z, double sim_time, int x, int y, int z)
-{
-    double rx = c.origin[0] + ((c.off[0] + x) + 0.5) * c.cell_size;
-    double ry = c.origin[1] + ((c.off[1] + y) + 0.5) * c.cell_size;
-    double rz = c.origin[2] + ((c.off[2] + z) + 0.5) * c.cell_size;
-    double lv = c.lv;
-    double invlv = 1. / lv;
+    const double invlv = 1. / c.lv;
     double xlen = c.gnsbx * c.nx * c.cell_size;
     xlen = xlen + c.lsd;
     double tline = xlen * invlv;
-    double tpause = 1.5e-4 * invlv;
+    const double tpause = 1.5e-4 * invlv;
     tline = tline + tpause;
     double trackno = 0;
     if (c.am_tracks > 1)
         trackno = floor(sim_time / tline);
-    double xnow = c.x0 + (sim_time - trackno * tline) * lv;
-    double ynow = c.y0 + trackno * c.lhs;
-    double znow = c.z0;
-    double lpow = c.lpow;
-    double lx = rx - xnow;
-    double ly = ry - ynow;
-    if (!(rz <= znow + c.cell_size))
+    BeamNow n;
+    n.xnow = c.x0 + (sim_time - trackno * tline) * c.lv;
+    n.ynow = c.y0 + trackno * c.lhs;
+    n.znow = c.z0;
+    const double lpow = (sim_time < 1e-4) ? 0.0 : c.lpow;
+    n.Tfront = c.lab * lpow * beam_lalpha(c) / (5.568328 * c.lthcon);
+    return n;
+}
+
+// The Gaussian-beam quadrature of temp_model<true> with the factors of its
+// 400 terms that do not depend on the cell tabulated (same operations and
+// order as temp_model<true>, so the same values):
+//   vlt[i] = lv * lt,  A[i] = ls*ls + 4.*lalpha*lt,
+//   Tl[i] = sqrt(lalpha*lt) * (ls*ls + 4.*lalpha*lt),
+// the correctly rounded reciprocals of A and Tl, and a copy of the exp table,
+// so that its lookups are LDS reads.  k_beam_nodes computes the tables once
+// per block into DevBufs::beam_nodes (BEAM_NODE_ROWS x BEAM_NT), and
+//   Zq[z][i] = lz*lz / (4.*lalpha*lt)
+// per padded plane into DevBufs::beam_zq.
+enum { BN_VLT, BN_A, BN_RA, BN_TL, BN_RTL, BEAM_NODE_ROWS };
+
+struct BeamTab {
+    double node[BEAM_NODE_ROWS][BEAM_NT];
+    uint64_t exp_tab[EXP_TAB_WORDS];
+};
+
+__device__ __forceinline__ void
+beam_tab_load(const DevBufs &b, BeamTab &t, int tid, int nthreads)
+{
+    for (int i = tid; i < BEAM_NODE_ROWS * BEAM_NT; i += nthreads)
+        (&t.node[0][0])[i] = G(b.beam_nodes)[i];
+    for (int i = tid; i < EXP_TAB_WORDS; i += nthreads)
+        t.exp_tab[i] = exp_tab[i];
+}
+
+// a / b, correctly rounded, from rb = 1 / b correctly rounded: a product and
+// two corrections with exact remainders.  The first brings the quotient
+// within one unit of its last place, the second then rounds it correctly
+// (Markstein's theorem: q + (a - b q) rb rounds to a / b when q is that close
+// and rb is the rounded reciprocal).  Needs a and b so far from the limits of
+// the exponent range that no intermediate leaves it; 5 operations where the
+// division sequence takes 11 and a quarter-rate reciprocal.
+__device__ __forceinline__ double
+div_by(double a, double b, double rb)
+{
+    double q = a * rb;
+    q = fma(fma(-b, q, a), rb, q);
+    return fma(fma(-b, q, a), rb, q);
+}
+
+// lane Q of every group of LANES (2 or 4) lanes, to all of the group
+template <int LANES, int Q>
+__device__ __forceinline__ double
+group_lane(double v)
+{
+    constexpr int ctrl = LANES == 4 ? Q | Q << 2 | Q << 4 | Q << 6                       // DPP quad_perm
+                                    : Q | Q << 2 | (2 + Q) << 4 | (2 + Q) << 6;
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// temp_model<true> on the tables, one cell per LANES lanes (1, 2 or 4): lane g
+// of a group computes the terms LANES m + g and every lane adds all of them in
+// node order.  All lanes of a group pass the same cell.
+//
+// Four terms at a time, so that their chains overlap.  Where c.beam_fast holds
+// and every exponent of the wave is in exp's normal range (then ldt * exp is
+// above 1e-250, far from where a division by a reciprocal could go wrong) the
+// terms are straight-line code, 28 FP64 operations each.
+//
+// The node factors are the same for every lane of a wave with one lane per
+// cell: they come as scalar loads, because reading them from LDS (20 of the 44
+// clocks of LDS time a term took) held the four SIMDs of a CU to two thirds of
+// their FP64 rate.  With more lanes per cell they are LDS reads.
+template <int LANES>
+__device__ __forceinline__ double
+beam_quad(const Consts &c, const DevBufs &b, const BeamTab &t, const MMCA_GLOBAL double *Z, const BeamNow &bn, int x, int y, int z, int g)
+{
+    constexpr int U = 4;
+    static_assert(BEAM_NT % (4 * U) == 0, "whole rounds of four terms per lane");
+    const double rx = c.origin[0] + ((c.off[0] + x) + 0.5) * c.cell_size;
+    const double ry = c.origin[1] + ((c.off[1] + y) + 0.5) * c.cell_size;
+    const double rz = c.origin[2] + ((c.off[2] + z) + 0.5) * c.cell_size;
+    if (!(rz <= bn.znow + c.cell_size))
         return 0.0;
-    double pi15 = 5.568328;
-    double lalpha = beam_lalpha(c);
-    double ldt = beam_ldt(c);
-    if (sim_time < 1e-4)
-        lpow = 0;
-    double Tfront = c.lab * lpow * lalpha / (pi15 * c.lthcon);
-    if (Tfront == 0.0)
-        return c.liniT + Tfront * 0.0;     // every term is finite, so Tfront * Tinteg is this
+    if (bn.Tfront == 0.0)
+        return c.liniT + bn.Tfront * 0.0;         // every term is finite, so Tfront * Tinteg is this
+    const double lx = rx - bn.xnow;
+    const double ly = ry - bn.ynow;
+    const double ly2 = ly * ly;
+    const double ldt = beam_ldt(c);
+    auto node = [&](int row, int i) -> double {
+        if constexpr (LANES == 1)
+            return ((const __attribute__((address_space(4))) double *) (unsigned long long) b.beam_nodes)[row * BEAM_NT + i];
+        else
+            return t.node[row][i];
+    };
     double Tinteg = 0.0;
-    for (int i = 0; i < BEAM_NT; i++)
+    for (int m = 0; m < BEAM_NT / LANES; m += U)
     {
-        const double u = lx + t.vlt[i];
-        Tinteg += ldt * exp_glibc(-(u * u + ly * ly) / t.A[i] - Z[i], t.exp_tab) / t.Tl[i];
+        double term[U], e[U];
+        bool normal = c.beam_fast;
+        if (c.beam_fast)
+        {
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+            {
+                const int i = LANES * (m + k) + g;
+                const double u = lx + node(BN_VLT, i);
+                const double a = u * u + ly2;
+                e[k] = -div_by(a, node(BN_A, i), node(BN_RA, i)) - Z[i];
+                normal = normal && e[k] > -512.0 && e[k] < -0x1p-54;
+            }
+        }
+        if (__all(normal))
+        {
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+            {
+                const int i = LANES * (m + k) + g;
+                term[k] = div_by(ldt * exp_normal(e[k], t.exp_tab), node(BN_TL, i), node(BN_RTL, i));
+            }
+        }
+        else
+        {
+#pragma unroll 1
+            for (int k = 0; k < U; ++k)
+            {
+                const int i = LANES * (m + k) + g;
+                const double u = lx + node(BN_VLT, i);
+                const double v = ldt * exp_glibc(-(u * u + ly2) / node(BN_A, i) - Z[i], t.exp_tab) / node(BN_TL, i);
+                term[0] = k == 0 ? v : term[0];
+                term[1] = k == 1 ? v : term[1];
+                term[2] = k == 2 ? v : term[2];
+                term[3] = k == 3 ? v : term[3];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+        {
+            if constexpr (LANES == 1)
+                Tinteg += term[k];
+            else
+            {
+                Tinteg += group_lane<LANES, 0>(term[k]);
+                Tinteg += group_lane<LANES, 1>(term[k]);
+                if constexpr (LANES == 4)
+                {
+                    Tinteg += group_lane<LANES, 2>(term[k]);
+                    Tinteg += group_lane<LANES, 3>(term[k]);
+                }
+            }
+        }
     }
-    return c.liniT + Tfront * Tinteg;
+    return c.liniT + bn.Tfront * Tinteg;
+}
+
+// Half-width of the interval around an approximate beam temperature T
+// (DevBufs::temp32) that holds the quadrature's value: its FP32 storage and
+// rounding (far below 1e-5 relative to the terms it is the sum of) and the
+// interpolation's error (c.beam_tol times the largest sum of terms).
+__device__ __forceinline__ double
+beam_margin(const Consts &c, double T)
+{
+    return 1e-5 * (fabs(T) + fabs(c.liniT)) + c.beam_tol;
 }
 
 // Octahedron half-diagonal of a solid cell (grow_octahedra, growth.c:392-403)
@@ -267,12 +359,6 @@ rec_code(const Consts &c, const unsigned char *rec, int x, int j, int k)
     const unsigned long long *w = reinterpret_cast<const unsigned long long *>(rec) + rec_word(c, (x - 1) >> 6, j, k);
     const int bit = (x - 1) & 63;
     return (int) ((w[0] >> bit) & 1ull) | (int) (((w[1] >> bit) & 1ull) << 1) | (int) (((w[2] >> bit) & 1ull) << 2);
-}
-
-__device__ inline double
-temp_at(const Consts &c, double sim_time, int x, int y, int z)
-{
-    return c.am ? temp_model<true>(c, sim_time, x, y, z) : temp_model<false>(c, sim_time, x, y, z);
 }
 
 // ---------------------------------------------------------------------------

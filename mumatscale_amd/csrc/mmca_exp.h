@@ -74,9 +74,11 @@ exp_special(double tmp, uint64_t sbits, uint64_t ki)
     return 0x1p-1022 * y;
 }
 
-// tab: EXP_TAB_WORDS words of mmca_exp_table.inc (constant memory or a copy in LDS)
+// 2^-54 <= |x| < 512: no special case.  tab: EXP_TAB_WORDS words of
+// mmca_exp_table.inc (constant memory or a copy in LDS).  The scale's bits and
+// the value relative to it; exp(x) = scale + scale * tmp.
 MMCA_HD inline double
-exp_glibc(double x, const uint64_t *tab)
+exp_reduce(double x, const uint64_t *tab, uint64_t *sbits, uint64_t *kint)
 {
     const double inv_ln2_n = 0x1.71547652b82fep0 * EXP_TAB_N;
     const double neg_ln2_hi_n = -0x1.62e42fefa0000p-8;
@@ -86,7 +88,31 @@ exp_glibc(double x, const uint64_t *tab)
     const double c3 = 0x1.555555555543cp-3;
     const double c4 = 0x1.55555cf172b91p-5;
     const double c5 = 0x1.1111167a4d017p-7;
+    double kd = fma(inv_ln2_n, x, shift);
+    const uint64_t ki = exp_as_u64(kd);
+    kd -= shift;
+    const double r = fma(kd, neg_ln2_lo_n, fma(kd, neg_ln2_hi_n, x));
+    const uint32_t idx = 2u * (uint32_t) (ki % EXP_TAB_N);
+    const uint64_t top = ki << (52 - EXP_TAB_BITS);
+    const double tail = exp_as_f64(tab[idx]);
+    *sbits = tab[idx + 1] + top;
+    *kint = ki;
+    const double r2 = r * r;
+    return fma(r2 * r2, fma(r, c5, c4), fma(r2, fma(r, c3, c2), tail + r));
+}
 
+MMCA_HD inline double
+exp_normal(double x, const uint64_t *tab)
+{
+    uint64_t sbits, ki;
+    const double tmp = exp_reduce(x, tab, &sbits, &ki);
+    const double scale = exp_as_f64(sbits);
+    return fma(scale, tmp, scale);
+}
+
+MMCA_HD inline double
+exp_glibc(double x, const uint64_t *tab)
+{
     // top 12 bits without the sign; 0x3c9 = top12(2^-54), 0x408 = top12(512), 0x409 = top12(1024)
     uint32_t abstop = (uint32_t) (exp_as_u64(x) >> 52) & 0x7ff;
     if (abstop - 0x3c9u >= 0x408u - 0x3c9u)
@@ -103,16 +129,8 @@ exp_glibc(double x, const uint64_t *tab)
         }
         abstop = 0;                               // 512 <= |x| < 1024
     }
-    double kd = fma(inv_ln2_n, x, shift);
-    const uint64_t ki = exp_as_u64(kd);
-    kd -= shift;
-    const double r = fma(kd, neg_ln2_lo_n, fma(kd, neg_ln2_hi_n, x));
-    const uint32_t idx = 2u * (uint32_t) (ki % EXP_TAB_N);
-    const uint64_t top = ki << (52 - EXP_TAB_BITS);
-    const double tail = exp_as_f64(tab[idx]);
-    const uint64_t sbits = tab[idx + 1] + top;
-    const double r2 = r * r;
-    const double tmp = fma(r2 * r2, fma(r, c5, c4), fma(r2, fma(r, c3, c2), tail + r));
+    uint64_t sbits, ki;
+    const double tmp = exp_reduce(x, tab, &sbits, &ki);
     if (abstop == 0)
         return exp_special(tmp, sbits, ki);
     const double scale = exp_as_f64(sbits);

@@ -42,8 +42,11 @@ struct Consts {
     int check_neg;
     // temperature (temperature.c:24-126)
     int am;                 // 1: Gaussian-beam model
-    int beam_sep;           // 1 (FP32-deviation AM only): the beam temperature from its separable
-                            // factors, computed per step into DevBufs::temp
+    int beam_sep;           // 1 (FP32-deviation AM only): interior temperature outputs from the beam's
+                            // separable factors; 0: from the quadrature
+    int beam_rank;          // interpolation points in time of the approximate beam temperature
+    int beam_fast;          // 1: the quadrature's divisors allow division by reciprocals (div_by)
+    double beam_tol;        // bound on the interpolation's error [K]
     int am_layers, am_tracks, gnsbx;
     double dt, cell_size, origin[3];
     double t_init, cool_rate, gradient, grad_coef, velocity, velo_coef;
@@ -109,11 +112,14 @@ struct DevBufs {
     double *fixed_rot;               // 9 per fixed nucleation point
     double *rand_rot;                // 9 per random orientation draw
     int rand_cap;                    // random orientations uploaded
-    // separable beam temperature (Consts::beam_sep): T per padded cell, the
-    // factor tables X[i][x], Y[y][i], Zf[z][i], W[(z-1) ny + y-1][i] =
-    // Y[y][i] Zf[z][i], and the track position W was built for (2 doubles)
+    // Gaussian beam: the approximate temperature per padded cell (float), and
+    // for temperature outputs the temperature; the quadrature's node factors
+    // and plane factors (BeamTab); and the padded indices, in no order, of the
+    // cells whose partitioning waits for the exact temperature, and their number
+    float *temp32;
     double *temp;
-    double *beam_x, *beam_y, *beam_z, *beam_w, *beam_key;
+    double *beam_nodes, *beam_zq;
+    int *und, *und_n;
     // single-operator buffers (allocated on first use)
     double *oce;
     double *d;
@@ -127,6 +133,15 @@ struct DevBufs {
     unsigned char *rec;
     unsigned long long rec_t0;
     long long rec_steps;
+};
+
+// Points in time of the beam's separable temperature (k_beam_field) and its
+// factors: the points, the weights at the quadrature's nodes (BEAM_NT x rank;
+// null: the points are the nodes), the factors in x and per (z, y) row, and the
+// track position the row factors were built for (2 doubles).
+struct BeamSet {
+    double *tau, *weights, *ax, *aw, *key;
+    int rank;
 };
 
 // One domain (subblock) as the hot kernels see it.

@@ -198,7 +198,25 @@ k_nuc_detect(View V, int advance, int cur)
         int rem = (int) (idx - z * c.sxy);
         int y = rem / c.sx;
         int x = rem - y * c.sx;
-        double T = c.beam_sep ? G(b.temp)[idx] : temp_at(c, sim_time, x, y, z);
+        double T;
+        if (c.am)
+        {
+            // The tests below read T only through comparisons (undercooling
+            // falls with T where the slope m is constant): where they all come
+            // out the same at both ends of the approximate temperature's
+            // interval, it will do.
+            T = (double) G(b.temp32)[idx];
+            const double d = beam_margin(c, T);
+            const double lo = T - d, hi = T + d;
+            const double cl = c.f32 ? ld_cl<true>(b, c, cur, idx) : ld_cl<false>(b, c, cur, idx);
+            const double add = c.mc * (cl - c.cinit), thr = (double) G(b.site_thr)[s];
+            const bool same = (lo > c.Tliq || hi <= c.Tliq) && (lo >= c.Tsol || hi < c.Tsol) &&
+                              ((c.Tliq - hi) + add > thr || (c.Tliq - lo) + add <= thr);
+            if (!(c.ma == 0.0 && c.mb == 0.0 && same))
+                T = temp_model<true>(c, sim_time, x, y, z);
+        }
+        else
+            T = temp_model<false>(c, sim_time, x, y, z);
         int layerno = 1, initnuc = 1;
         if (c.am)
         {
@@ -593,19 +611,49 @@ partition_cell(const Consts &c, TempFn temp, double ce_new, double ce_prev, doub
     *g_out = g;
 }
 
-// The temperature the partitioning of cell idx reads (tempUpdateSB_int,
-// temperature.c:218-262): the model itself, or with beam_sep the separable
-// beam field computed into b.temp before the step (the kernels then run
-// their non-AM form).
-template <bool AM>
-__device__ __forceinline__ double
-temp_step(const DevBufs &b, const Consts &c, double sim_time, long long idx, int x, int y, int z)
+// What a solid cell's partitioning does at every temperature in [T - d, T + d]
+// (fs_change_diffuse's tests, growth.c:228-241, which read T only through
+// comparisons that hold or fail for the whole interval): true if it is the
+// same branch, LIQUID or SOLID, so that an approximate T gives the cell's
+// result to the bit.  Tunder falls with T, in floating point too.  A growing
+// or remelting cell needs the exact T (false), and so does a NaN.
+__device__ __forceinline__ bool
+branch_decided(const Consts &c, double T, double d, double conc, double lspfs)
 {
-    if constexpr (AM)
-        return temp_model<true>(c, sim_time, x, y, z);
-    if (c.beam_sep)
-        return G(b.temp)[idx];
-    return temp_model<false>(c, sim_time, x, y, z);
+    if (T - d > c.Tliq || T + d < 1.0)
+        return true;
+    return lspfs == 1.0 && T - d >= 1.0 && T + d <= c.Tliq &&
+           (c.Tliq - (T + d)) + c.liq_slope * (conc - c.cinit) >= 0.0;
+}
+
+// Appends the padded indices of the lanes with `flag` to the block's list of
+// waiting cells: one atomic per wave.  All lanes call it.
+__device__ __forceinline__ void
+und_append(const DevBufs &b, bool flag, int idx)
+{
+    const unsigned long long m = __ballot(flag);
+    if (!m)
+        return;
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    if (lane == (int) __ffsll(m) - 1)
+        base = atomicAdd(b.und_n, __popcll(m));
+    base = __shfl(base, (int) __ffsll(m) - 1, 64);
+    if (flag)
+        G(b.und)[base + __popcll(m & ((1ull << lane) - 1ull))] = idx;
+}
+
+// A cell whose partitioning waits for the exact temperature (k_beam_finish)
+// keeps what that needs in its output slots: FP64 storage, the ce before
+// diffusion in fs (the new one is in ce); FP32 storage, the new ce unrounded in
+// fs and the stored ce before diffusion in cl.
+template <bool F32>
+__device__ __forceinline__ void
+defer_cell(const DevBufs &b, const Consts &c, int nxt, long long idx, double ce_new, double ce_prev)
+{
+    fs_buf(b, nxt)[idx] = F32 ? ce_new : ce_prev;
+    if (F32)
+        cl32_buf(b, nxt)[idx] = (float) (ce_prev - c.cinit);
 }
 
 // growth.c:163-165: error() ends every rank.  In a coupled batch the status
@@ -641,6 +689,10 @@ template <bool DIFF, bool FSC, bool AM, bool F32, bool REC = false>
 __global__ void __launch_bounds__(SOL_BX *SOL_BY)
 k_solute(View V, int cur, int nxt)
 {
+    // the fused step of a beam block works from the approximate temperature
+    // and leaves the cells that need the exact one to k_beam_finish; the single
+    // operators and the recorded step evaluate the quadrature in place
+    constexpr bool DEFER = AM && DIFF && FSC && !REC;
     __shared__ double s_red[SOL_BX * SOL_BY / 64];
     __shared__ int s_stop;
     const int dm = find_dom(V.off_cell, V.ndom, blockIdx.x);
@@ -674,6 +726,7 @@ k_solute(View V, int cur, int nxt)
     {
         int g_new = 0;
         int br_rec = 0;
+        bool wait = false;
         if (active)
         {
             const long long idx = k * c.sxy + (long long) j * c.sx + x;
@@ -705,22 +758,42 @@ k_solute(View V, int cur, int nxt)
             {
                 const double ce_prev = DIFF ? ce_old : G(b.oce)[idx];
                 const int g_old = G(b.gr)[idx];
+                if constexpr (DEFER)
+                    if (g_old > 0)
+                    {
+                        const double T = (double) G(b.temp32)[idx];
+                        wait = !branch_decided(c, T, beam_margin(c, T), conc, lspfs);
+                    }
                 double cl_out, fs_out;
-                int g, branch;
-                partition_cell(c, [&]() { return temp_step<AM>(b, c, sim_time, idx, x, j, k); }, ce_new, ce_prev,
-                               conc, lspfs, g_old, &cl_out, &fs_out, &g, &branch);
-                br_rec = branch;
-                st_cl<F32>(b, c, nxt, idx, cl_out);
-                st_stream(fs_buf(b, nxt), idx, fs_out);
-                if (g != g_old)
-                    G(b.gr)[idx] = g;
-                keep_stale_d(c, b, idx, g_old, g, lspfs);
+                int g = g_old, branch;
+                if (wait)
+                    defer_cell<F32>(b, c, nxt, idx, ce_new, ce_prev);
+                else
+                {
+                    partition_cell(
+                        c,
+                        [&]() {
+                            if constexpr (DEFER)
+                                return (double) G(b.temp32)[idx];
+                            else
+                                return temp_model<AM>(c, sim_time, x, j, k);
+                        },
+                        ce_new, ce_prev, conc, lspfs, g_old, &cl_out, &fs_out, &g, &branch);
+                    br_rec = branch;
+                    st_cl<F32>(b, c, nxt, idx, cl_out);
+                    st_stream(fs_buf(b, nxt), idx, fs_out);
+                    if (g != g_old)
+                        G(b.gr)[idx] = g;
+                    keep_stale_d(c, b, idx, g_old, g, lspfs);
+                }
                 g_new = g;
             }
         }
         if (FSC)
         {
-            unsigned long long bits = __ballot(active && g_new > 0);
+            if (DEFER)
+                und_append(b, wait, (int) (k * c.sxy + (long long) j * c.sx + x));
+            const unsigned long long bits = __ballot(active && g_new > 0 && !wait);
             if (threadIdx.x == 0 && rowok)
                 G(b.mask)[((long long) k * (c.ny + 2) + j) * c.w64 + bx] = bits;
         }
@@ -821,12 +894,14 @@ from_lane_down(double v, double edge)
 
 // What a wave loads of one plane: cl and fs of rows -1 .. RY of its tile, ce
 // and gr of its own rows, the x neighbours across the tile's edges (lane 63:
-// x + 1, the others: x - 1 of lane 0) and, with a temperature field, T.
+// x + 1, the others: x - 1 of lane 0) and, in beam blocks (TF), the
+// approximate temperature.
 template <int RY, bool F32, bool TF>
 struct RwPlane {
     using S = typename Store<F32>::T;
     S cl[RY + 2], ce[RY], ecl[RY];
-    double fs[RY + 2], efs[RY], t[TF ? RY : 1];
+    double fs[RY + 2], efs[RY];
+    float t[TF ? RY : 1];
     int g[RY];
 };
 
@@ -863,6 +938,8 @@ at_byte(MMCA_GLOBAL T *base, unsigned off)
 // FP64, 256 x 256 x 512: 403 us (447 us with planes staged in LDS, 4.2 TB/s
 // of 56 B per cell); 128 x 128 x 256: 48 us (142); 40 x 36 x 44: 8.3 us (93).
 // FP32-deviation storage, 256 x 256 x 512: 293 us (337).
+constexpr int RW_LATE = 2048;                    // waiting cells of a tile buffered in LDS
+
 template <int RY, bool F32, bool TF>
 __global__ void __launch_bounds__(512)
 k_solute_rw(View V, int cur, int nxt)
@@ -874,6 +951,10 @@ k_solute_rw(View V, int cur, int nxt)
     // the non-beam temperatures depend on z only (on y in 2-D runs): one value
     // per plane of the tile (per row); dynamic LDS
     extern __shared__ double s_T[];
+    // beam blocks: the tile's waiting cells (s_late: their number, and where
+    // the buffer ended), appended to the block's list with one atomic; cells
+    // past the buffer go to the list directly
+    __shared__ int s_cell[TF ? RW_LATE : 1], s_late[TF ? 3 : 1];
     const long long gtile = xcd_tile(V);
     if (gtile >= V.tot_zm)
         return;                                   // uniform over the workgroup
@@ -897,7 +978,7 @@ k_solute_rw(View V, int cur, int nxt)
     const MMCA_GLOBAL double *fsc = fs_buf(dd->b, cur);
     MMCA_GLOBAL double *fsn = fs_buf(dd->b, nxt);
     MMCA_GLOBAL int *grb = G(dd->b.gr);
-    const MMCA_GLOBAL double *tb = G(dd->b.temp);
+    const MMCA_GLOBAL float *tb = G(dd->b.temp32);
     MMCA_GLOBAL unsigned long long *mask = G(dd->b.mask);
     const int lane = threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
@@ -914,7 +995,11 @@ k_solute_rw(View V, int cur, int nxt)
     // this kernel itself may raise the status: read it once per workgroup so
     // that every wave takes the same branch before the barrier of block_sum
     if (lane == 0 && threadIdx.y == 0)
+    {
         s_stop = (G(dd->b.cnt)->status != MMCA_OK);
+        if constexpr (TF)
+            s_late[0] = 0, s_late[1] = RW_LATE;
+    }
     const bool two_d = (c.gdimz == 1);
     if constexpr (!TF)
     {
@@ -956,7 +1041,7 @@ k_solute_rw(View V, int cur, int nxt)
                 p.ce[r] = *at_byte(ceb + at, (rb + xc) * E);
                 p.g[r] = *at_byte(grb + at, (rb + xc) * 4);
                 if constexpr (TF)
-                    p.t[r] = *at_byte(tb + at, (rb + xc) * 8);
+                    p.t[r] = *at_byte(tb + at, (rb + xc) * 4);
             }
         };
         // solute through the face from cell a to cell b (growth.c:95-99)
@@ -967,7 +1052,8 @@ k_solute_rw(View V, int cur, int nxt)
         };
         // the plane below, not finished yet: x and y terms, own values, and
         // the z face below it
-        double psum[RY], pcl[RY], pfs[RY], pce[RY], pfz[RY], pt[TF ? RY : 1];
+        double psum[RY], pcl[RY], pfs[RY], pce[RY], pfz[RY];
+        float pt[TF ? RY : 1];
         int pg[RY];
         RwPlane<RY, F32, TF> P0, P1;
         load(P0, k0);
@@ -1005,46 +1091,80 @@ k_solute_rw(View V, int cur, int nxt)
                     sum -= pfz[r];
                     const double ce_new = pce[r] + sum;
                     int g_new = 0;
+                    bool wait = false;
                     if (j <= c.ny && x <= c.nx)
                     {
                         const long long at = (k - 1) * c.sxy + row0;
                         const unsigned o = (unsigned) ((r + 1) * c.sx) + (unsigned) x;
                         neg |= (ce_new < 0);
-                        double cl_out, fs_out;
-                        int branch;
-                        partition_cell(
-                            c,
-                            [&]() {
-                                if constexpr (TF)
-                                    return pt[r];
-                                else
-                                    return s_T[two_d ? wv * RY + r : k - 1 - k0];
-                            },
-                            ce_new, pce[r], pcl[r], pfs[r], pg[r], &cl_out, &fs_out, &g_new, &branch);
                         if constexpr (F32)
                         {
                             const double dev = ce_new - c.cinit;
                             const float f = (float) dev;
                             lost += dev - (double) f;
                             *at_byte(ceb + at, o * E) = f;
-                            *at_byte(cln + at, o * E) = (float) (cl_out - c.cinit);
+                        }
+                        else
+                            *at_byte(ceb + at, o * E) = ce_new;
+                        if constexpr (TF)
+                            wait = pg[r] > 0 && !branch_decided(c, (double) pt[r], beam_margin(c, (double) pt[r]),
+                                                                pcl[r], pfs[r]);
+                        if (wait)
+                        {
+                            // as defer_cell
+                            *at_byte(fsn + at, o * 8) = F32 ? ce_new : pce[r];
+                            if constexpr (F32)
+                                *at_byte(cln + at, o * E) = (float) (pce[r] - c.cinit);
                         }
                         else
                         {
-                            *at_byte(ceb + at, o * E) = ce_new;
-                            *at_byte(cln + at, o * E) = cl_out;
-                        }
-                        *at_byte(fsn + at, o * 8) = fs_out;
-                        if (g_new != pg[r])
-                        {
-                            *at_byte(grb + at, o * 4) = g_new;
-                            if (c.track_d)
-                                keep_stale_d(c, dd->b, at + o, pg[r], g_new, pfs[r]);
+                            double cl_out, fs_out;
+                            int branch;
+                            partition_cell(
+                                c,
+                                [&]() {
+                                    if constexpr (TF)
+                                        return (double) pt[r];
+                                    else
+                                        return s_T[two_d ? wv * RY + r : k - 1 - k0];
+                                },
+                                ce_new, pce[r], pcl[r], pfs[r], pg[r], &cl_out, &fs_out, &g_new, &branch);
+                            if constexpr (F32)
+                                *at_byte(cln + at, o * E) = (float) (cl_out - c.cinit);
+                            else
+                                *at_byte(cln + at, o * E) = cl_out;
+                            *at_byte(fsn + at, o * 8) = fs_out;
+                            if (g_new != pg[r])
+                            {
+                                *at_byte(grb + at, o * 4) = g_new;
+                                if (c.track_d)
+                                    keep_stale_d(c, dd->b, at + o, pg[r], g_new, pfs[r]);
+                            }
                         }
                     }
                     const unsigned long long bits = __ballot(g_new > 0);
                     if (lane == 0 && j <= c.ny)
                         mask[((long long) (k - 1) * (c.ny + 2) + j) * c.w64 + bx] = bits;
+                    if constexpr (TF)
+                    {
+                        const unsigned long long late = __ballot(wait);
+                        if (late)
+                        {
+                            const int cell = (int) ((k - 1) * c.sxy + (long long) j * c.sx + x);
+                            int base = 0;
+                            if (lane == 0)
+                            {
+                                base = atomicAdd(&s_late[0], __popcll(late));
+                                if (base + __popcll(late) > RW_LATE)
+                                    atomicMin(&s_late[1], base);
+                            }
+                            base = __builtin_amdgcn_readfirstlane(base);
+                            if (base + __popcll(late) > RW_LATE)
+                                und_append(dd->b, wait, cell);
+                            else if (wait)
+                                s_cell[base + __popcll(late & ((1ull << lane) - 1ull))] = cell;
+                        }
+                    }
                 }
                 // x and y terms of plane k
                 const double ecl = from_raw<F32>(c, A.ecl[r]);
@@ -1083,274 +1203,24 @@ k_solute_rw(View V, int cur, int nxt)
     }
     if (c.check_neg && neg)
         flag_negative_ce(V, c, dd->b.cnt);
+    if constexpr (TF)
+    {
+        __syncthreads();
+        const int n = min(s_late[0], s_late[1]);
+        if (n > 0)                                // uniform over the workgroup
+        {
+            if (lane == 0 && threadIdx.y == 0)
+                s_late[2] = atomicAdd(dd->b.und_n, n);
+            __syncthreads();
+            for (int e = wv * 64 + lane; e < n; e += 64 * blockDim.y)
+                G(dd->b.und)[s_late[2] + e] = s_cell[e];
+        }
+    }
     if (F32)
     {
         const double tot = block_sum(lost, s_red, 64 * blockDim.y);
         if (lane == 0 && threadIdx.y == 0 && tot != 0.0)
             ledger_add(dd->b, tile, tot);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// The fused kernel of the Gaussian-beam quadrature (k_solute_zl): z-marching,
-// with its planes staged in LDS by direct global->LDS loads (gfx950
-// global_load_lds_dword).
-//
-// A workgroup of 64 x BY threads owns a 64 x BY column tile and walks its
-// planes upward, with the same arithmetic per cell as k_solute.  The
-// planes come through a ring of ZL_RING slots in LDS instead of registers:
-// each slot holds one plane's cl and fs over the tile with a one-cell halo in
-// x and y ((BY + 2) rows x 66), and its ce and gr over the tile.  The loads
-// write LDS directly, so a plane in flight costs no VGPRs, and two planes are
-// in flight while one is computed.  Every wave issues an equal share of a
-// slot's loads (64 lanes x 4 bytes each, per-lane offsets computed once: they
-// are the same for every plane), then waits for its own share of the plane it
-// needs next; the one barrier per plane makes every wave's share visible and
-// frees the slot of the plane before the last.
-//
-// The loads are issued from inline asm, which the compiler's wait-count pass
-// does not see: it would otherwise make every LDS read wait for all loads in
-// flight.  Their completion is waited for explicitly with vmcnt(N), where N
-// counts only loads of this ring issued after the awaited ones; any other
-// memory operation issued in between makes that wait stricter, never looser.
-// Every load address is clamped into the padded box of its field.
-constexpr int ZL_RING = 4;
-
-template <int BY, bool F32>
-struct ZlSlot {
-    static constexpr int E = F32 ? 4 : 8;          // bytes per stored ce, cl value
-    static constexpr int HR = BY + 2, HW = 66;     // halo'd rows and row width
-    static constexpr int pad64(int n) { return (n + 63) / 64 * 64; }
-    static constexpr int CL_DW = pad64(HR * HW * E / 4);
-    static constexpr int FS_DW = pad64(HR * HW * 2);
-    static constexpr int CE_DW = pad64(BY * 64 * E / 4);
-    static constexpr int GR_DW = pad64(BY * 64);
-    static constexpr int CL0 = 0, FS0 = CL_DW, CE0 = FS0 + FS_DW, GR0 = CE0 + CE_DW;
-    static constexpr int DW = GR0 + GR_DW;         // dwords per slot
-    static constexpr int NI = DW / 64;             // load instructions per slot
-    static constexpr int NPW = (NI + BY - 1) / BY; // per wave: loads NPW w .. NPW w + NPW - 1 of the slot
-    // field region of load i (every region is whole loads: cl, fs, ce, gr)
-    static constexpr int region_of(int i)
-    {
-        return i * 64 < FS0 ? 0 : i * 64 < CE0 ? 1 : i * 64 < GR0 ? 2 : 3;
-    }
-    // a wave's loads span at most two regions, so it keeps two base pointers
-    static constexpr bool two_regions()
-    {
-        for (int w = 0; w < BY; ++w)
-        {
-            const int a = w * NPW < NI - 1 ? w * NPW : NI - 1;
-            const int z = w * NPW + NPW - 1 < NI - 1 ? w * NPW + NPW - 1 : NI - 1;
-            if (region_of(z) - region_of(a) > 1)
-                return false;
-        }
-        return true;
-    }
-    static_assert(two_regions(), "a wave's share of a slot must lie in at most two field regions");
-};
-
-// One dword per lane from global (sbase + voff) into LDS (lds + lane * 4).
-__device__ __forceinline__ void
-zl_load(const void *sbase, unsigned voff, unsigned lds)
-{
-    unsigned save;
-    asm volatile("s_mov_b32 %0, m0\n\t"
-                 "s_mov_b32 m0, %3\n\t"
-                 "global_load_lds_dword %1, %2\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(save)
-                 : "v"(voff), "s"(sbase), "s"(lds)
-                 : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void
-zl_wait()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-template <int BY, bool F32>
-__global__ void __launch_bounds__(64 * BY)
-k_solute_zl(View V, int cur, int nxt)
-{
-    using L = ZlSlot<BY, F32>;
-    using T = typename Store<F32>::T;
-    static_assert(L::NPW * 3 + 16 < 64, "loads in flight must stay within the vmcnt range");
-    __shared__ __attribute__((aligned(16))) unsigned s_ring[ZL_RING * L::DW];
-    __shared__ double s_red[BY];
-    __shared__ int s_stop;
-    __shared__ double s_beam[sizeof(BeamTab) / sizeof(double)];
-    __shared__ double s_z[2][BEAM_NT];           // plane factors of the beam, double-buffered
-    BeamTab *beam = reinterpret_cast<BeamTab *>(s_beam);
-    const long long gtile = xcd_tile(V);
-    if (gtile >= V.tot_zm)
-        return;                                   // uniform over the workgroup
-    const int dm = find_dom(V.off_zm, V.ndom, gtile);
-    const long long tile = gtile - V.off_zm[dm];
-    const DevBufs b = V.dom[dm].b;
-    const Consts c = V.dom[dm].c;
-    const int kz = c.zm_planes;
-    Counters *cnt = b.cnt;
-    if (threadIdx.x == 0 && threadIdx.y == 0)
-        s_stop = (G(b.cnt)->status != MMCA_OK);
-    __syncthreads();
-    if (s_stop)
-        return;
-    const int lane = threadIdx.x;
-    const int ty = threadIdx.y;
-    const int wv = __builtin_amdgcn_readfirstlane(ty);
-    const int ntx = (c.nx + 63) / 64, nty = (c.ny + BY - 1) / BY;
-    const int bx = (int) (tile % ntx);
-    const int by = (int) ((tile / ntx) % nty);
-    const int bz = (int) (tile / ((long long) ntx * nty));
-    const int x0 = bx * 64 + 1, j0 = by * BY + 1;
-    const int x = x0 + lane;
-    const int j = j0 + ty;
-    const int k0 = bz * kz + 1;
-    const int k1 = min(c.nz, k0 + kz - 1);
-    const int n = k1 - k0 + 1;
-    const bool rowok = (j <= c.ny);
-    const bool active = rowok && (x <= c.nx);
-
-    // this wave's share of a slot: loads i = NPW wv + m (the last load of the
-    // slot repeated past its end), which lie in at most two field regions rA
-    // and rB (rB from load mB on); each load reads at per-lane byte offset
-    // off[m] within a plane of its field.  Few scalar registers hold this
-    // state (two bases, two strides), so the kernel's constants stay in
-    // scalar registers too.
-    const char *fbase[4] = { (const char *) (F32 ? (const void *) cl32_buf(b, cur) : (const void *) cl_buf(b, cur)),
-                             (const char *) fs_buf(b, cur),
-                             (const char *) (F32 ? (const void *) b.ce32 : (const void *) b.ce),
-                             (const char *) b.gr };
-    const long long fplane[4] = { c.sxy * L::E, c.sxy * 8, c.sxy * L::E, c.sxy * 4 };
-    const int ibase = wv * L::NPW;
-    const int rA = L::region_of(min(ibase, L::NI - 1)), rB = L::region_of(min(ibase + L::NPW - 1, L::NI - 1));
-    const int rstart = rB == 0 ? 0 : rB == 1 ? L::FS0 / 64 : rB == 2 ? L::CE0 / 64 : L::GR0 / 64;
-    const int mB = rA == rB ? 0 : rstart - ibase;              // loads m >= mB are in rB
-    const char *baseA = (rA == 0) ? fbase[0] : (rA == 1) ? fbase[1] : (rA == 2) ? fbase[2] : fbase[3];
-    const char *baseB = (rB == 0) ? fbase[0] : (rB == 1) ? fbase[1] : (rB == 2) ? fbase[2] : fbase[3];
-    const long long strA = (rA == 0) ? fplane[0] : (rA == 1) ? fplane[1] : (rA == 2) ? fplane[2] : fplane[3];
-    const long long strB = (rB == 0) ? fplane[0] : (rB == 1) ? fplane[1] : (rB == 2) ? fplane[2] : fplane[3];
-    unsigned off[L::NPW];
-#pragma unroll
-    for (int m = 0; m < L::NPW; ++m)
-    {
-        const int i = min(ibase + m, L::NI - 1);
-        const int d = i * 64 + lane;
-        int dw, esz, rows_halo;
-        if (d < L::FS0)
-            dw = d - L::CL0, esz = L::E, rows_halo = 1;
-        else if (d < L::CE0)
-            dw = d - L::FS0, esz = 8, rows_halo = 1;
-        else if (d < L::GR0)
-            dw = d - L::CE0, esz = L::E, rows_halo = 0;
-        else
-            dw = d - L::GR0, esz = 4, rows_halo = 0;
-        const int per = esz / 4;                          // dwords per value
-        const int width = rows_halo ? L::HW : 64;
-        const int nval = rows_halo ? L::HR * L::HW : BY * 64;
-        const int e = min(dw / per, nval - 1);            // padding dwords repeat the last value
-        const int half = dw - (dw / per) * per;
-        const int row = e / width, col = e - row * width;
-        const int gj = min(j0 - rows_halo + row, c.ny + 1);
-        const int gx = min(x0 - rows_halo + col, c.nx + 1);
-        off[m] = (unsigned) ((gj * c.sx + gx) * esz + half * 4);
-    }
-    const unsigned ring_lds = (unsigned) (unsigned long) (__attribute__((address_space(3))) unsigned *) s_ring;
-    // loads of plane sequence number s (plane k0 - 1 + s, clamped to k1 + 1) into slot s % ZL_RING
-    auto issue = [&](int s) {
-        const long long p = min(k0 - 1 + s, k1 + 1);
-        const unsigned slot = ring_lds + (unsigned) ((s % ZL_RING) * L::DW) * 4u;
-        const char *pa = baseA + p * strA, *pb = baseB + p * strB;
-#pragma unroll
-        for (int m = 0; m < L::NPW; ++m)
-            zl_load(m >= mB ? pb : pa, off[m], slot + (unsigned) min(ibase + m, L::NI - 1) * 256u);
-    };
-    auto cl_at = [&](int q, int row, int col) -> double {
-        const unsigned *sl = s_ring + q * L::DW + L::CL0;
-        return from_raw<F32>(c, reinterpret_cast<const T *>(sl)[row * L::HW + col]);
-    };
-    auto fs_at = [&](int q, int row, int col) -> double {
-        const unsigned *sl = s_ring + q * L::DW + L::FS0;
-        return reinterpret_cast<const double *>(sl)[row * L::HW + col];
-    };
-
-    const MMCA_GLOBAL double *fsc = fs_buf(b, cur);
-    (void) fsc;
-    MMCA_GLOBAL double *fsn_out = fs_buf(b, nxt);
-    const double sim_time = G(b.cnt)->timestep * c.dt;
-    const int mo_x1 = (x == c.nx) ? c.pad_hi[0] : 0, mo_x0 = (x == 1) ? c.pad_lo[0] : 0;
-    const int mo_y1 = (j == c.ny) ? c.pad_hi[1] : 0, mo_y0 = (j == 1) ? c.pad_lo[1] : 0;
-
-    issue(0);
-    issue(1);
-    issue(2);
-    issue(3);
-    beam_tab_terms(c, *beam, ty * 64 + lane, 64 * BY);
-    beam_tab_plane(c, s_z[1], k0, ty * 64 + lane, 64 * BY);
-    zl_wait<2 * L::NPW>();                       // planes k0 - 1 and k0 have landed
-    __syncthreads();
-    double clm = cl_at(0, ty + 1, lane + 1), fsm = fs_at(0, ty + 1, lane + 1);
-    double clv = cl_at(1, ty + 1, lane + 1), fsv = fs_at(1, ty + 1, lane + 1);
-    double lost = 0.0;
-    bool neg = false;
-    for (int s = 1; s <= n; ++s)
-    {
-        const int k = k0 - 1 + s;
-        const int q = s % ZL_RING, q1 = (s + 1) % ZL_RING;
-        zl_wait<L::NPW>();                       // this wave's share of plane k + 1 has landed
-        __syncthreads();                         // every wave's share; the slot of plane k - 1 is free
-        issue(s + 3);
-        if (s < n)
-            beam_tab_plane(c, s_z[(s + 1) & 1], k + 1, ty * 64 + lane, 64 * BY);
-        const double clp = cl_at(q1, ty + 1, lane + 1), fsp = fs_at(q1, ty + 1, lane + 1);
-        int g_new = 0;
-        if (active)
-        {
-            const long long idx = k * c.sxy + (long long) j * c.sx + x;
-            const double clxm = cl_at(q, ty + 1, lane), fsxm = fs_at(q, ty + 1, lane);
-            const double clxp = cl_at(q, ty + 1, lane + 2), fsxp = fs_at(q, ty + 1, lane + 2);
-            const double clym = cl_at(q, ty, lane + 1), fsym = fs_at(q, ty, lane + 1);
-            const double clyp = cl_at(q, ty + 2, lane + 1), fsyp = fs_at(q, ty + 2, lane + 1);
-            const unsigned *sl = s_ring + q * L::DW;
-            const double ce_old = from_raw<F32>(c, reinterpret_cast<const T *>(sl + L::CE0)[ty * 64 + lane]);
-            const int g_old = reinterpret_cast<const int *>(sl + L::GR0)[ty * 64 + lane];
-            const double cln[6] = { clxp, clxm, clyp, clym, clp, clm };
-            const double fsn[6] = { fsxp, fsxm, fsyp, fsym, fsp, fsm };
-            const int mo[6] = { mo_x1, mo_x0, mo_y1, mo_y0, (k == c.nz) ? c.pad_hi[2] : 0,
-                                (k == 1) ? c.pad_lo[2] : 0 };
-            const double ce_new = diffuse_cell(c, ce_old, clv, fsv, cln, fsn, mo);
-            neg |= (ce_new < 0);
-            lost += st_ce<F32>(b, c, idx, ce_new);
-            double cl_out, fs_out;
-            int branch;
-            partition_cell(
-                c,
-                [&]() { return beam_temp_tab(c, *beam, s_z[s & 1], sim_time, x, j, k); },
-                ce_new, ce_old, clv, fsv, g_old, &cl_out, &fs_out, &g_new, &branch);
-            st_cl<F32>(b, c, nxt, idx, cl_out);
-            st_stream(fsn_out, idx, fs_out);
-            if (g_new != g_old)
-                G(b.gr)[idx] = g_new;
-            keep_stale_d(c, b, idx, g_old, g_new, fsv);
-        }
-        unsigned long long bits = __ballot(active && g_new > 0);
-        if (rowok && lane == 0)
-            G(b.mask)[((long long) k * (c.ny + 2) + j) * c.w64 + bx] = bits;
-        clm = clv;
-        fsm = fsv;
-        clv = clp;
-        fsv = fsp;
-    }
-    zl_wait<0>();                                // no load may land in LDS after the workgroup ends
-    if (c.check_neg && neg)
-        flag_negative_ce(V, c, cnt);
-    if (F32)
-    {
-        const double tot = block_sum<64 * BY>(lost, s_red);
-        if (lane == 0 && ty == 0 && tot != 0.0)
-            ledger_add(b, tile, tot);
     }
 }
 
@@ -1894,52 +1764,32 @@ k_reduce_final(DevBufs b, int nblk, double *out)
 }
 
 // ---------------------------------------------------------------------------
-// Separable Gaussian-beam temperature (Consts::beam_sep, FP32-deviation AM).
-// Term i of the quadrature of temp_model<true> (temperature.c:104-112),
-//   ldt * exp(-((lx + lv t_i)^2 + ly^2) / A_i - lz^2 / (4 alpha t_i)) / Tl_i,
-// is the product X_i(x) Y_i(y) Zf_i(z) of
-//   X_i = exp(-(lx + lv t_i)^2 / A_i),   Y_i = ldt / Tl_i * exp(-ly^2 / A_i),
-//   Zf_i = exp(-lz^2 / (4 alpha t_i)),
-// so that over the interior of a block T = liniT + Tfront * sum_i X_i(x)
-// W_i(y, z) with W_i(y, z) = Y_i(y) Zf_i(z): a product of a (BEAM_NT x nx)
-// and a ((nz ny) x BEAM_NT) matrix, 400 multiply-adds per cell and
-// 400 (nx + ny + nz) exps per step in place of 400 exps per cell.  The three
-// factors round separately and the sum runs in another order, so T differs
-// from the quadrature's in its last bits.  Every factor is at most 1 (the
-// exponents are not positive), so a factor that underflows stands for a term
-// below the smallest double.
+// Gaussian beam in the step.  The reference evaluates a 400-term quadrature at
+// every solid cell; its value matters only where a cell grows or remelts.  So
+// a step computes an approximate temperature of the whole block (k_beam_field,
+// a few multiply-adds per cell), the solute kernel finishes every cell whose
+// branch is the same over the approximation's whole error interval
+// (branch_decided) and marks the others, and k_beam_finish evaluates the
+// quadrature for the marked ones, bit for bit the reference's.
+//
+// The approximation: as functions of the time node t, the x factors
+// exp(-(lx + v t)^2 / A(t)) are smooth over the quadrature's short range, so
+// they are interpolated between beam_rank Chebyshev points tau_j (chosen on
+// the host so that the error is below 1e-9).  With w_i(y, z) = ldt / Tl_i *
+// exp(-ly^2 / A_i - lz^2 / (4 alpha t_i)) and interpolation weights C[i][j],
+//   T = liniT + Tfront * sum_j X_j(x) (sum_i C[i][j] w_i(y, z)),
+// where the inner sums change only with the track.
 
-// beam position and amplitude at sim_time (temperature.c:62-103)
-struct BeamNow {
-    double xnow, ynow, znow, Tfront;
-};
+// With beam_sep (FP32-deviation storage) the temperature outputs of the block's
+// interior come from the same product with all 400 nodes as points (then the
+// weights are the unit matrix), in double: the quadrature's sum of products of
+// separately rounded factors, within 1e-13 of it.
 
-__device__ __forceinline__ BeamNow
-beam_now(const Consts &c, double sim_time)
-{
-    const double invlv = 1. / c.lv;
-    double xlen = c.gnsbx * c.nx * c.cell_size;
-    xlen = xlen + c.lsd;
-    double tline = xlen * invlv;
-    const double tpause = 1.5e-4 * invlv;
-    tline = tline + tpause;
-    double trackno = 0;
-    if (c.am_tracks > 1)
-        trackno = floor(sim_time / tline);
-    BeamNow n;
-    n.xnow = c.x0 + (sim_time - trackno * tline) * c.lv;
-    n.ynow = c.y0 + trackno * c.lhs;
-    n.znow = c.z0;
-    const double lpow = (sim_time < 1e-4) ? 0.0 : c.lpow;
-    n.Tfront = c.lab * lpow * beam_lalpha(c) / (5.568328 * c.lthcon);
-    return n;
-}
-
-// Table shapes: X rows (one per node) of beam_x_pitch columns, zero past
-// nx; W rows (one per (y, z) row of the block, q = (z-1) ny + y-1) of
-// BEAM_NT nodes, beam_w_rows of them, zero past ny nz.
+// Table shapes: x factors, one row per interpolation point, of beam_x_pitch
+// columns (zero past nx); row factors, one row per (z, y) row of the block, of
+// beam_rank values, beam_w_rows of them (zero past ny nz).
 constexpr int BF_COLS = 128;                      // columns per workgroup of k_beam_field
-constexpr int BF_ROWS = 64;                       // W rows per workgroup
+constexpr int BF_ROWS = 64;                       // rows per workgroup
 __host__ __device__ __forceinline__ int beam_x_pitch(const Consts &c) { return (c.nx + BF_COLS - 1) / BF_COLS * BF_COLS; }
 __host__ __device__ __forceinline__ long long
 beam_w_rows(const Consts &c)
@@ -1947,91 +1797,110 @@ beam_w_rows(const Consts &c)
     return ((long long) c.ny * c.nz + BF_ROWS - 1) / BF_ROWS * BF_ROWS;
 }
 
-// The factor tables at the time of timestep cnt->timestep + adv:
-// X[i][x-1], Y[y-1][i], Zf[z-1][i].  W depends on the time only through
-// the track's y position; beam_key[0] holds the position W was built for,
-// and beam_key[1] tells k_beam_w whether to build it again.
+// node factors (BeamTab) and plane factors of the quadrature
 __global__ void __launch_bounds__(256)
-k_beam_tabs(DevBufs b, Consts c, int adv)
+k_beam_nodes(DevBufs b, Consts c)
 {
-    const MMCA_GLOBAL Counters *cnt = G(b.cnt);
-    if (cnt->status != MMCA_OK)
-        return;
-    const double sim_time = (cnt->timestep + (unsigned long long) adv) * c.dt;
-    const BeamNow bn = beam_now(c, sim_time);
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-    {
-        const double held = G(b.beam_key)[0];
-        const bool same = __double_as_longlong(held) == __double_as_longlong(bn.ynow);
-        G(b.beam_key)[1] = same ? 0.0 : 1.0;
-        G(b.beam_key)[0] = bn.ynow;
-    }
     const double ls = c.lsd / (2. * 1.414);
     const double lalpha = beam_lalpha(c);
     const double ldt = beam_ldt(c);
-    const int xp = beam_x_pitch(c);
-    const long long nX = (long long) BEAM_NT * xp, nY = (long long) BEAM_NT * c.ny;
-    const long long n = nX + nY + (long long) BEAM_NT * c.nz;
-    for (long long e = (long long) blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long) gridDim.x * blockDim.x)
+    for (long long e = (long long) blockIdx.x * 256 + threadIdx.x; e < (long long) BEAM_NT * (c.nz + 3);
+         e += 256ll * gridDim.x)
     {
-        if (e < nX)
+        const int z = (int) (e / BEAM_NT) - 1, i = (int) (e % BEAM_NT);
+        const double lt = (0.5 + i) * ldt;
+        if (z < 0)
         {
-            const int i = (int) (e / xp), q = (int) (e - (long long) i * xp);
-            const double lt = (0.5 + i) * ldt;
             const double A = ls * ls + 4. * lalpha * lt;
-            double v = 0.0;                       // columns past nx pad the row
-            if (q < c.nx)
-            {
-                const double rx = c.origin[0] + ((c.off[0] + q + 1) + 0.5) * c.cell_size;
-                const double u = (rx - bn.xnow) + c.lv * lt;
-                v = exp_glibc(-(u * u) / A, exp_tab);
-            }
-            G(b.beam_x)[e] = v;
-        }
-        else if (e < nX + nY)
-        {
-            const long long f = e - nX;
-            const int y = (int) (f / BEAM_NT), i = (int) (f - (long long) y * BEAM_NT);
-            const double lt = (0.5 + i) * ldt;
-            const double A = ls * ls + 4. * lalpha * lt;
-            const double ry = c.origin[1] + ((c.off[1] + y + 1) + 0.5) * c.cell_size;
-            const double ly = ry - bn.ynow;
             const double Tl = sqrt(lalpha * lt) * (ls * ls + 4. * lalpha * lt);
-            G(b.beam_y)[f] = ldt / Tl * exp_glibc(-(ly * ly) / A, exp_tab);
+            G(b.beam_nodes)[BN_VLT * BEAM_NT + i] = c.lv * lt;
+            G(b.beam_nodes)[BN_A * BEAM_NT + i] = A;
+            G(b.beam_nodes)[BN_RA * BEAM_NT + i] = 1.0 / A;
+            G(b.beam_nodes)[BN_TL * BEAM_NT + i] = Tl;
+            G(b.beam_nodes)[BN_RTL * BEAM_NT + i] = 1.0 / Tl;
         }
         else
         {
-            const long long f = e - nX - nY;
-            const int z = (int) (f / BEAM_NT), i = (int) (f - (long long) z * BEAM_NT);
-            const double lt = (0.5 + i) * ldt;
-            const double rz = c.origin[2] + ((c.off[2] + z + 1) + 0.5) * c.cell_size;
-            const double lz = rz - bn.znow;
-            G(b.beam_z)[f] = exp_glibc(-(lz * lz) / (4. * lalpha * lt), exp_tab);
+            const double rz = c.origin[2] + ((c.off[2] + z) + 0.5) * c.cell_size;
+            const double lz = rz - c.z0;
+            G(b.beam_zq)[(long long) z * BEAM_NT + i] = lz * lz / (4. * lalpha * lt);
         }
     }
 }
 
-// W[q][i] = Y[y-1][i] * Zf[z-1][i] for q = (z-1) ny + y-1, when the track's
-// y position changed (beam_key[1]); one row per wave at a time
+// x factors at the interpolation nodes for timestep cnt->timestep + adv; says
+// in beam_key[1] whether the row factors have to be built for a new track, and
+// empties the list of waiting cells
 __global__ void __launch_bounds__(256)
-k_beam_w(DevBufs b, Consts c)
+k_beam_ax(DevBufs b, Consts c, BeamSet p, int adv)
 {
-    if (G(b.cnt)->status != MMCA_OK || G(b.beam_key)[1] == 0.0)
-        return;
-    const long long rows = (long long) c.nz * c.ny;
-    const long long waves = (long long) gridDim.x * (blockDim.x / 64);
-    for (long long q = (long long) blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; q < rows; q += waves)
+    const double sim_time = (G(b.cnt)->timestep + (unsigned long long) adv) * c.dt;
+    const BeamNow bn = beam_now(c, sim_time);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
     {
-        const int z = (int) (q / c.ny), y = (int) (q - (long long) z * c.ny);
-        const MMCA_GLOBAL double *Y = G(b.beam_y) + (long long) y * BEAM_NT;
-        const MMCA_GLOBAL double *Z = G(b.beam_z) + (long long) z * BEAM_NT;
-        for (int i = threadIdx.x % 64; i < BEAM_NT; i += 64)
-            G(b.beam_w)[q * BEAM_NT + i] = Y[i] * Z[i];
+        const double held = G(p.key)[0];
+        G(p.key)[1] = __double_as_longlong(held) == __double_as_longlong(bn.ynow) ? 0.0 : 1.0;
+        G(p.key)[0] = bn.ynow;
+        *b.und_n = 0;
+    }
+    const double ls = c.lsd / (2. * 1.414);
+    const double lalpha = beam_lalpha(c);
+    const int e = blockIdx.x * 256 + threadIdx.x, xp = beam_x_pitch(c);
+    const int j = e / xp, q = e - j * xp;
+    if (j >= p.rank)
+        return;
+    const double t = G(p.tau)[j];
+    const double rx = c.origin[0] + ((c.off[0] + q + 1) + 0.5) * c.cell_size;
+    const double u = (rx - bn.xnow) + c.lv * t;
+    G(p.ax)[e] = q < c.nx ? exp(-(u * u) / (ls * ls + 4. * lalpha * t)) : 0.0;   // columns past nx pad the row
+}
+
+// row factors: one workgroup per (z, y) row; 16 groups of 16 threads share the
+// nodes, each thread sums for one interpolation point at a time
+__global__ void __launch_bounds__(256)
+k_beam_aw(DevBufs b, Consts c, BeamSet p)
+{
+    __shared__ double s_w[BEAM_NT];
+    __shared__ double s_p[16][17];
+    if (G(p.key)[1] == 0.0)
+        return;
+    const int z = (int) (blockIdx.x / (unsigned) c.ny), y = (int) (blockIdx.x - (unsigned) z * (unsigned) c.ny);
+    const double ldt = beam_ldt(c);
+    const double ry = c.origin[1] + ((c.off[1] + y + 1) + 0.5) * c.cell_size;
+    const double ly = ry - G(p.key)[0];
+    for (int i = threadIdx.x; i < BEAM_NT; i += 256)
+        s_w[i] = ldt / G(b.beam_nodes)[BN_TL * BEAM_NT + i] *
+                 exp(-(ly * ly) / G(b.beam_nodes)[BN_A * BEAM_NT + i] - G(b.beam_zq)[(long long) (z + 1) * BEAM_NT + i]);
+    __syncthreads();
+    if (!p.weights)
+    {
+        for (int i = threadIdx.x; i < BEAM_NT; i += 256)
+            G(p.aw)[(long long) blockIdx.x * BEAM_NT + i] = s_w[i];
+        return;
+    }
+    const int jj = threadIdx.x & 15, g = threadIdx.x >> 4;
+    for (int j0 = 0; j0 < p.rank; j0 += 16)
+    {
+        double v = 0.0;
+        for (int i = g; i < BEAM_NT; i += 16)
+            v += s_w[i] * G(p.weights)[(long long) i * p.rank + j0 + jj];
+        s_p[g][jj] = v;
+        __syncthreads();
+        if (g == 0)
+        {
+            double t = 0.0;
+            for (int q = 0; q < 16; ++q)
+                t += s_p[q][jj];
+            G(p.aw)[(long long) blockIdx.x * p.rank + j0 + jj] = t;
+        }
+        __syncthreads();
     }
 }
 
-// T over the interior into out (padded indexing): the product of W (rows q)
-// and X on the matrix cores.  v_mfma_f64_16x16x4f64 multiplies a 16 x 4
+// T over the interior (padded indexing; 49 us for 500 x 256 x 128 cells and 32
+// points, where 400 points took 230): the product of the row factors (rows
+// q = (z-1) ny + y-1) and the x factors on the matrix cores, in double into
+// b.temp (OUT), or rounded to float into b.temp32.  v_mfma_f64_16x16x4f64 multiplies a 16 x 4
 // tile of W (lane l: row l % 16, node slot l / 16) by a 4 x 16 tile of X
 // (lane l: node slot l / 16, column l % 16) into a 16 x 16 tile held as four
 // doubles per lane (lane l, register r: row l / 16 + 4 r, column l % 16).
@@ -2041,29 +1910,34 @@ k_beam_w(DevBufs b, Consts c)
 // rows x 32 columns (4 x 2 tiles, 32 accumulators per lane); the four waves
 // of a workgroup share its 64 rows and take 32 columns each.
 typedef double dvec4 __attribute__((ext_vector_type(4)));
-static_assert(BEAM_NT % 16 == 0, "nodes come in blocks of 16");
 
+template <bool OUT>
 __global__ void __launch_bounds__(256)
-k_beam_field(DevBufs b, Consts c, int adv, double *out)
+k_beam_field(DevBufs b, Consts c, BeamSet p, int adv)
 {
     const MMCA_GLOBAL Counters *cnt = G(b.cnt);
     if (cnt->status != MMCA_OK)
         return;                                   // uniform over the workgroup
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const long long q0 = (long long) blockIdx.y * BF_ROWS;
-    const int x0 = blockIdx.x * BF_COLS + wave * 32;      // 0-based interior column
+    const int xp = beam_x_pitch(c), K = p.rank;
+    const unsigned ntx = (unsigned) (xp / BF_COLS), slab = blockIdx.x / ntx;
+    const long long q0 = (long long) slab * BF_ROWS;
+    const int x0 = (int) (blockIdx.x - slab * ntx) * BF_COLS + wave * 32;      // 0-based interior column
     const int kk = lane >> 4, lr = lane & 15;
     const double sim_time = (cnt->timestep + (unsigned long long) adv) * c.dt;
     const BeamNow bn = beam_now(c, sim_time);
     const long long nq = (long long) c.ny * c.nz;
     // stores tile (a, bb) register r: row q0 + 16 a + kk + 4 r, column x0 + 16 bb + lr
+    const unsigned uy = (unsigned) c.ny;
+    const int z0 = (int) (q0 / uy), y0 = (int) (q0 - (long long) z0 * uy);       // 0-based plane and row of q0
     auto store = [&](int a, int bb, int r, double sum, bool sep) {
-        const long long q = q0 + 16 * a + kk + 4 * r;
-        const int x = x0 + 16 * bb + lr;
-        if (q >= nq || x >= c.nx)
+        const int d = 16 * a + kk + 4 * r, x = x0 + 16 * bb + lr;
+        if (q0 + d >= nq || x >= c.nx)
             return;
-        const int z = (int) (q / c.ny) + 1, y = (int) (q - (long long) (z - 1) * c.ny) + 1;
+        // 32-bit arithmetic: a 64-bit division per value cost more than the product
+        const unsigned t0 = (unsigned) (y0 + d), dz = uy >= BF_ROWS ? (t0 >= uy ? 1u : 0u) : t0 / uy;
+        const int z = z0 + (int) dz + 1, y = (int) (t0 - dz * uy) + 1;
         const double rz = c.origin[2] + ((c.off[2] + z) + 0.5) * c.cell_size;
         double t;
         if (!(rz <= bn.znow + c.cell_size))
@@ -2072,7 +1946,11 @@ k_beam_field(DevBufs b, Consts c, int adv, double *out)
             t = c.liniT + bn.Tfront * 0.0;        // every term is finite: liniT + 0
         else
             t = c.liniT + bn.Tfront * sum;
-        out[(long long) z * c.sxy + (long long) y * c.sx + x + 1] = t;
+        const long long at = (long long) z * c.sxy + (long long) y * c.sx + x + 1;
+        if (OUT)
+            G(b.temp)[at] = t;
+        else
+            G(b.temp32)[at] = (float) t;
     };
     if (bn.Tfront == 0.0)
     {
@@ -2082,13 +1960,12 @@ k_beam_field(DevBufs b, Consts c, int adv, double *out)
                     store(a, bb, r, 0.0, false);
         return;
     }
-    const int xp = beam_x_pitch(c);
     // this lane's W rows (one per row tile) and X columns (one per column tile)
     const MMCA_GLOBAL double *Wr[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a)
-        Wr[a] = G(b.beam_w) + (q0 + 16 * a + lr) * BEAM_NT + 4 * kk;
-    const MMCA_GLOBAL double *Xc = G(b.beam_x) + x0 + lr + (long long) (4 * kk) * xp;
+        Wr[a] = G(p.aw) + (q0 + 16 * a + lr) * K + 4 * kk;
+    const MMCA_GLOBAL double *Xc = G(p.ax) + x0 + lr + (long long) (4 * kk) * xp;
     dvec4 acc[4][2];
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -2108,12 +1985,12 @@ k_beam_field(DevBufs b, Consts c, int adv, double *out)
                 xb[bb][m] = Xc[(long long) (16 * t + m) * xp + 16 * bb];
     };
     load(0);
-    for (int t = 0; t < BEAM_NT / 16; ++t)
+    for (int t = 0; t < K / 16; ++t)
     {
         const dvec4 ca[4] = { wa[0], wa[1], wa[2], wa[3] };
         const double cb[2][4] = { { xb[0][0], xb[0][1], xb[0][2], xb[0][3] },
                                   { xb[1][0], xb[1][1], xb[1][2], xb[1][3] } };
-        if (t + 1 < BEAM_NT / 16)
+        if (t + 1 < K / 16)
             load(t + 1);                          // the next block's loads overlap this block's MFMAs
 #pragma unroll
         for (int m = 0; m < 4; ++m)
@@ -2132,31 +2009,144 @@ k_beam_field(DevBufs b, Consts c, int adv, double *out)
                 store(a, bb, r, acc[a][bb][r], true);
 }
 
-// The separable temperature of timestep cnt->timestep + adv into b.temp
-hipError_t launch_beam_field(const DevBufs &b, const Consts &c, int adv, hipStream_t s)
+// The cells the solute kernel left (DevBufs::und): the quadrature, then the
+// partitioning from what defer_cell kept.  The listed cells are dealt evenly to
+// the grid's threads: one thread per cell, or two or four while the grid has
+// that many, so that the 400-term chains stay short.
+//
+// Bound by the FP64 VALU of the quadrature, about 40 instructions per term.
+// About 120 000 waiting cells of a 250 x 190 x 94 block: 85 us; a kernel that
+// evaluated every solid cell in place took 10 ms a step.
+template <bool F32>
+__global__ void __launch_bounds__(256)
+k_beam_finish(View V, int cur, int nxt)
 {
-    const long long tabs = (long long) BEAM_NT * (beam_x_pitch(c) + c.ny + c.nz);
-    hipLaunchKernelGGL(k_beam_tabs, dim3((unsigned) std::min<long long>((tabs + 255) / 256, 4096)), dim3(256), 0, s,
-                       b, c, adv);
-    const long long rows = (long long) c.ny * c.nz;
-    hipLaunchKernelGGL(k_beam_w, dim3((unsigned) std::min<long long>((rows + 3) / 4, 2048)), dim3(256), 0, s, b, c);
-    const dim3 grid((unsigned) (beam_x_pitch(c) / BF_COLS), (unsigned) (beam_w_rows(c) / BF_ROWS));
-    hipLaunchKernelGGL(k_beam_field, grid, dim3(256), 0, s, b, c, adv, b.temp);
+    __shared__ BeamTab s_tab;
+    const DevBufs b = V.dom[blockIdx.y].b;    // private copy: stores cannot alias it
+    const Consts c = V.dom[blockIdx.y].c;
+    if (G(b.cnt)->status != MMCA_OK)
+        return;
+    const int tid = threadIdx.x;
+    const int n = *G(b.und_n);
+    const long long nthr = 256ll * gridDim.x;
+    // log2 of the threads per cell: up to about one wave on each of the 1024 SIMDs
+    const int sh = n <= 16384 ? 2 : n <= 32768 ? 1 : 0;
+    if (256ll * blockIdx.x >= (long long) n << sh)
+        return;                                   // uniform over the workgroup
+    beam_tab_load(b, s_tab, tid, 256);
+    __syncthreads();
+    const BeamNow bn = beam_now(c, G(b.cnt)->timestep * c.dt);
+    const int g = tid & ((1 << sh) - 1);
+    for (long long i = (256ll * blockIdx.x + tid) >> sh; i < n; i += nthr >> sh)
+    {
+        const int idx = G(b.und)[i];
+        const int k = (int) (idx / c.sxy), rem = (int) (idx - k * c.sxy), j = rem / c.sx, x = rem - j * c.sx;
+        const MMCA_GLOBAL double *Z = G(b.beam_zq) + (long long) k * BEAM_NT;
+        const double T = sh == 2   ? beam_quad<4>(c, b, s_tab, Z, bn, x, j, k, g)
+                         : sh == 1 ? beam_quad<2>(c, b, s_tab, Z, bn, x, j, k, g)
+                                   : beam_quad<1>(c, b, s_tab, Z, bn, x, j, k, 0);
+        const double kept = fs_buf(b, nxt)[idx];
+        const double ce_new = F32 ? kept : G(b.ce)[idx];
+        const double ce_prev = F32 ? c.cinit + (double) cl32_buf(b, nxt)[idx] : kept;
+        const double conc = ld_cl<F32>(b, c, cur, idx), lspfs = fs_buf(b, cur)[idx];
+        const int g_old = G(b.gr)[idx];
+        double cl_out, fs_out;
+        int g_new, branch;
+        partition_cell(c, [&]() { return T; }, ce_new, ce_prev, conc, lspfs, g_old, &cl_out, &fs_out, &g_new, &branch);
+        if (g == 0)
+        {
+            st_cl<F32>(b, c, nxt, idx, cl_out);
+            st_stream(fs_buf(b, nxt), idx, fs_out);
+            if (g_new != g_old)
+                G(b.gr)[idx] = g_new;
+            if (g_new > 0)
+                atomicOr(&b.mask[((long long) k * (c.ny + 2) + j) * c.w64 + (x - 1) / 64], 1ull << ((x - 1) & 63));
+            keep_stale_d(c, b, idx, g_old, g_new, lspfs);
+        }
+    }
+}
+
+// The quadrature over the padded box, or over its halo cells only
+__global__ void __launch_bounds__(256)
+k_beam_fill(DevBufs b, Consts c, int halo, double *out)
+{
+    __shared__ BeamTab s_tab;
+    beam_tab_load(b, s_tab, threadIdx.x, 256);
+    __syncthreads();
+    const BeamNow bn = beam_now(c, G(b.cnt)->timestep * c.dt);
+    const long long nA = 2 * c.sxy, nB = 2ll * c.nz * c.sx, nC = 2ll * c.ny * c.nz;
+    const long long n = halo ? nA + nB + nC : c.P;
+    for (long long e = (long long) blockIdx.x * 256 + threadIdx.x; e < n; e += 256ll * gridDim.x)
+    {
+        int x, y, z;
+        if (!halo || e < nA)
+        {
+            z = (int) (e / c.sxy);
+            const long long rem = e - z * c.sxy;
+            y = (int) (rem / c.sx);
+            x = (int) (rem - (long long) y * c.sx);
+            if (halo && z == 1)
+                z = c.nz + 1;
+        }
+        else if (e < nA + nB)
+        {
+            const long long f = e - nA, row = f / c.sx;
+            x = (int) (f - row * c.sx);
+            z = (int) (row >> 1) + 1;
+            y = (row & 1) ? c.ny + 1 : 0;
+        }
+        else
+        {
+            const long long f = e - nA - nB, row = f >> 1;
+            x = (f & 1) ? c.nx + 1 : 0;
+            z = (int) (row / c.ny) + 1;
+            y = (int) (row - (long long) (z - 1) * c.ny) + 1;
+        }
+        out[z * c.sxy + (long long) y * c.sx + x] =
+            beam_quad<1>(c, b, s_tab, G(b.beam_zq) + (long long) z * BEAM_NT, bn, x, y, z, 0);
+    }
+}
+
+hipError_t launch_beam_nodes(const DevBufs &b, const Consts &c, hipStream_t s)
+{
+    const long long n = (long long) BEAM_NT * (c.nz + 3);
+    hipLaunchKernelGGL(k_beam_nodes, dim3((unsigned) std::min<long long>((n + 255) / 256, 1024)), dim3(256), 0, s, b, c);
+    return hipGetLastError();
+}
+
+// The beam temperature of timestep cnt->timestep + adv from the point set p,
+// in double into b.temp (out) or rounded into b.temp32; the row factors too
+// when `rows` (they may be stale)
+hipError_t launch_beam_field(const DevBufs &b, const Consts &c, const BeamSet &p, int out, int adv, int rows,
+                             hipStream_t s)
+{
+    const long long n = (long long) p.rank * beam_x_pitch(c);
+    hipLaunchKernelGGL(k_beam_ax, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, b, c, p, adv);
+    if (rows)
+        hipLaunchKernelGGL(k_beam_aw, dim3((unsigned) ((long long) c.ny * c.nz)), dim3(256), 0, s, b, c, p);
+    const dim3 grid((unsigned) (beam_x_pitch(c) / BF_COLS * (beam_w_rows(c) / BF_ROWS)));
+    if (out)
+        hipLaunchKernelGGL(k_beam_field<true>, grid, dim3(256), 0, s, b, c, p, adv);
+    else
+        hipLaunchKernelGGL(k_beam_field<false>, grid, dim3(256), 0, s, b, c, p, adv);
+    return hipGetLastError();
+}
+
+// at most 1024 workgroups per domain: four waves per SIMD of the whole chip
+hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStream_t s)
+{
+    const long long per = (v.tot_list * LIST_BS * 64 / v.ndom + 1023) / 1024;     // cells per domain / 1024, about
+    const dim3 grid((unsigned) std::max<long long>(1, std::min<long long>(1024, per)), (unsigned) v.ndom);
+    if (f32)
+        hipLaunchKernelGGL(k_beam_finish<true>, grid, dim3(256), 0, s, v, cur, nxt);
+    else
+        hipLaunchKernelGGL(k_beam_finish<false>, grid, dim3(256), 0, s, v, cur, nxt);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// Derived fields for download.  With beam_sep the interior temperature is
-// the separable one, refreshed into b.temp by the caller; the halo cells
-// (read by no step) keep the quadrature.
-__device__ __forceinline__ double
-field_temp(const DevBufs &b, const Consts &c, long long i, int x, int y, int z)
-{
-    if (c.beam_sep && x >= 1 && x <= c.nx && y >= 1 && y <= c.ny && z >= 1 && z <= c.nz)
-        return G(b.temp)[i];
-    return temp_at(c, G(b.cnt)->timestep * c.dt, x, y, z);
-}
-
+// Derived fields for download: the temperature of the other models (the
+// beam's comes from k_beam_fill and, with beam_sep, k_beam_field).
 __global__ void
 k_fill_temp(DevBufs b, Consts c, double *out)
 {
@@ -2167,12 +2157,12 @@ k_fill_temp(DevBufs b, Consts c, double *out)
     long long rem = i - z * c.sxy;
     int y = (int) (rem / c.sx);
     int x = (int) (rem - (long long) y * c.sx);
-    out[i] = field_temp(b, c, i, x, y, z);
+    out[i] = temp_model<false>(c, G(b.cnt)->timestep * c.dt, x, y, z);
 }
 
 // cache_io_data (loop.c:74-113): FP32 copies of fs, ce and the temperature
 // and a copy of gr over the padded box, for the output writers.  A null
-// output is skipped.
+// output is skipped; a beam's temperature is in b.temp.
 template <bool F32>
 __global__ void
 k_io_fields(DevBufs b, Consts c, int cur, float *fs_io, float *ce_io, float *t_io, int *gr_io)
@@ -2186,13 +2176,15 @@ k_io_fields(DevBufs b, Consts c, int cur, float *fs_io, float *ce_io, float *t_i
         ce_io[i] = (float) ld_ce<F32>(b, c, i);
     if (gr_io)
         gr_io[i] = G(b.gr)[i];
-    if (t_io)
+    if (t_io && c.am)
+        t_io[i] = (float) G(b.temp)[i];
+    else if (t_io)
     {
         int z = (int) (i / c.sxy);
         long long rem = i - z * c.sxy;
         int y = (int) (rem / c.sx);
         int x = (int) (rem - (long long) y * c.sx);
-        t_io[i] = (float) field_temp(b, c, i, x, y, z);
+        t_io[i] = (float) temp_model<false>(c, G(b.cnt)->timestep * c.dt, x, y, z);
     }
 }
 
@@ -2263,8 +2255,7 @@ hipError_t launch_halo_exchange(const View &v, int phase, int cb, long long max_
 // zm_by: rows of the z-marching kernel (all domains of a view share it); 0
 // selects the cell-parallel kernel.
 template <bool AM, bool F32>
-static void launch_solute_t(const View &v, int zm_by, int tf, int diff, int fsc, int rec, int cur, int nxt,
-                            hipStream_t s)
+static void launch_solute_t(const View &v, int zm_by, int diff, int fsc, int rec, int cur, int nxt, hipStream_t s)
 {
     dim3 blk(SOL_BX, SOL_BY);
     if (rec)
@@ -2275,34 +2266,16 @@ static void launch_solute_t(const View &v, int zm_by, int tf, int diff, int fsc,
                                cur, nxt);
         return;
     }
-    const unsigned ng = (unsigned) ((v.tot_zm + 8ll * v.xcd_run - 1) / (8ll * v.xcd_run) * (8ll * v.xcd_run));
-    if (!AM && diff && fsc && zm_by > 0)
+    if (diff && fsc && zm_by > 0)
     {
-        const size_t tlds = tf ? 0 : (size_t) std::max(v.zm_planes_max, 16) * sizeof(double);   // per plane or row
+        const long long run = 8ll * v.xcd_run;
+        const dim3 grid((unsigned) ((v.tot_zm + run - 1) / run * run));
+        const size_t tlds = AM ? 0 : (size_t) std::max(v.zm_planes_max, 16) * sizeof(double);   // per plane or row
         const dim3 wg(64, zm_by == 16 ? 8 : 4);      // waves of 2 rows (of 1 row for 4-row tiles)
         if (zm_by == 4)
-        {
-            if (tf)
-                hipLaunchKernelGGL((k_solute_rw<1, F32, true>), dim3(ng), wg, tlds, s, v, cur, nxt);
-            else
-                hipLaunchKernelGGL((k_solute_rw<1, F32, false>), dim3(ng), wg, tlds, s, v, cur, nxt);
-        }
-        else if (tf)
-            hipLaunchKernelGGL((k_solute_rw<2, F32, true>), dim3(ng), wg, tlds, s, v, cur, nxt);
+            hipLaunchKernelGGL((k_solute_rw<1, F32, AM>), grid, wg, tlds, s, v, cur, nxt);
         else
-            hipLaunchKernelGGL((k_solute_rw<2, F32, false>), dim3(ng), wg, tlds, s, v, cur, nxt);
-    }
-    else if (diff && fsc && zm_by > 0)
-    {
-        if constexpr (AM)
-        {
-            if (zm_by == 16)
-                hipLaunchKernelGGL((k_solute_zl<16, F32>), dim3(ng), dim3(64, 16), 0, s, v, cur, nxt);
-            else if (zm_by == 8)
-                hipLaunchKernelGGL((k_solute_zl<8, F32>), dim3(ng), dim3(64, 8), 0, s, v, cur, nxt);
-            else
-                hipLaunchKernelGGL((k_solute_zl<4, F32>), dim3(ng), dim3(64, 4), 0, s, v, cur, nxt);
-        }
+            hipLaunchKernelGGL((k_solute_rw<2, F32, AM>), grid, wg, tlds, s, v, cur, nxt);
     }
     else if (diff && fsc)
         hipLaunchKernelGGL((k_solute<true, true, AM, F32>), dim3((unsigned) v.tot_cell), blk, 0, s, v, cur, nxt);
@@ -2316,22 +2289,22 @@ static void launch_solute_t(const View &v, int zm_by, int tf, int diff, int fsc,
                            nxt);
 }
 
-hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int tf, int diff, int fsc, int rec, int cur,
+hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int diff, int fsc, int rec, int cur,
                          int nxt, hipStream_t s)
 {
     if (am)
     {
         if (f32)
-            launch_solute_t<true, true>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<true, true>(v, zm_by, diff, fsc, rec, cur, nxt, s);
         else
-            launch_solute_t<true, false>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<true, false>(v, zm_by, diff, fsc, rec, cur, nxt, s);
     }
     else
     {
         if (f32)
-            launch_solute_t<false, true>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<false, true>(v, zm_by, diff, fsc, rec, cur, nxt, s);
         else
-            launch_solute_t<false, false>(v, zm_by, tf, diff, fsc, rec, cur, nxt, s);
+            launch_solute_t<false, false>(v, zm_by, diff, fsc, rec, cur, nxt, s);
     }
     return hipGetLastError();
 }
@@ -2420,9 +2393,18 @@ hipError_t launch_reduce(const DevBufs &b, const Consts &c, int cb, double *out2
     return hipGetLastError();
 }
 
+// temperature over the padded box (with beam_sep: of the halo cells, the
+// interior is the separable field)
 hipError_t launch_fill_temp(const DevBufs &b, const Consts &c, double *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fill_temp, dim3((unsigned) ((c.P + 255) / 256)), dim3(256), 0, s, b, c, out);
+    if (c.am)
+    {
+        const long long n = c.beam_sep ? 2 * c.sxy + 2ll * c.nz * c.sx + 2ll * c.ny * c.nz : c.P;
+        hipLaunchKernelGGL(k_beam_fill, dim3((unsigned) std::min<long long>((n + 255) / 256, 8192)), dim3(256), 0, s,
+                           b, c, c.beam_sep, out);
+    }
+    else
+        hipLaunchKernelGGL(k_fill_temp, dim3((unsigned) ((c.P + 255) / 256)), dim3(256), 0, s, b, c, out);
     return hipGetLastError();
 }
 
