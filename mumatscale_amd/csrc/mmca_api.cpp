@@ -37,6 +37,8 @@ long long zm_tiles(const Consts &c, int by);
 hipError_t launch_reduce(const DevBufs &b, const Consts &c, int cb, double *out2, hipStream_t s);
 hipError_t launch_fill_temp(const DevBufs &b, const Consts &c, double *out, hipStream_t s);
 hipError_t launch_grow_octahedra(const DevBufs &b, const Consts &c, int cb, hipStream_t s);
+hipError_t launch_widen(const float *in, double *out, double c0, long long n, hipStream_t s);
+hipError_t launch_narrow(const double *in, float *out, float *out2, double c0, long long n, hipStream_t s);
 hipError_t launch_gather_counters(const View &v, Counters *out, hipStream_t s);
 hipError_t launch_reset_new_grains(const View &v, hipStream_t s);
 hipError_t launch_fill_f64(double *p, long long n, double v, hipStream_t s);
@@ -107,7 +109,8 @@ struct mmca_ctx {
     long long time_n = 0;
     // grain records set by mmca_set_grains (ids below ext_grains.size())
     std::vector<mmca_grain> ext_grains;
-    // staging buffer of mmca_io_fields: 4 x P 32-bit values (allocated on first use)
+    // staging buffer of mmca_io_fields and of FP32-deviation fields on their way
+    // to or from the host: 4 x P 32-bit values (allocated on first use)
     float *io_buf = nullptr;
     // The random stream at the start of the orientation queue (before draw
     // q0).  mmca_rand draws from rng_now, the stream right after the
@@ -233,6 +236,15 @@ int ensure_d(mmca_ctx *ctx)
         ctx->view_dirty = true;
         HIPCHK(hipMemsetAsync(ctx->b.d, 0, (size_t) ctx->c.P * sizeof(double), ctx->stream));
     }
+    return MMCA_OK;
+}
+
+// staging buffer of mmca_io_fields, as P doubles
+int staging(mmca_ctx *ctx, double **out)
+{
+    if (!ctx->io_buf)
+        TRY(dev_alloc(&ctx->io_buf, 4 * (size_t) ctx->c.P));
+    *out = (double *) ctx->io_buf;
     return MMCA_OK;
 }
 
@@ -1055,16 +1067,14 @@ int mmca_upload_field(mmca_ctx *ctx, int field, const void *host)
     case MMCA_FIELD_CE:
     case MMCA_FIELD_CL:
         if (ctx->c.f32) {
-            const double *h = (const double *) host;
-            std::vector<float> tmp(P);
-            for (size_t i = 0; i < P; i++)
-                tmp[i] = (float) (h[i] - ctx->c.cinit);
-            if (field == MMCA_FIELD_CE) {
-                HIPCHK(hipMemcpy(b.ce32, tmp.data(), P * sizeof(float), hipMemcpyHostToDevice));
-            } else {
-                HIPCHK(hipMemcpy(b.cl32[0], tmp.data(), P * sizeof(float), hipMemcpyHostToDevice));
-                HIPCHK(hipMemcpy(b.cl32[1], tmp.data(), P * sizeof(float), hipMemcpyHostToDevice));
-            }
+            double *wide;
+            TRY(staging(ctx, &wide));
+            HIPCHK(hipMemcpyAsync(wide, host, P * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+            if (field == MMCA_FIELD_CE)
+                HIPCHK(launch_narrow(wide, b.ce32, nullptr, ctx->c.cinit, ctx->c.P, ctx->stream));
+            else
+                HIPCHK(launch_narrow(wide, b.cl32[0], b.cl32[1], ctx->c.cinit, ctx->c.P, ctx->stream));
+            HIPCHK(hipStreamSynchronize(ctx->stream));
         } else if (field == MMCA_FIELD_CE) {
             HIPCHK(hipMemcpy(b.ce, host, P * sizeof(double), hipMemcpyHostToDevice));
         } else {
@@ -1114,12 +1124,11 @@ int mmca_download_field(mmca_ctx *ctx, int field, void *host)
     case MMCA_FIELD_CE:
     case MMCA_FIELD_CL:
         if (c.f32) {
-            std::vector<float> tmp(P);
-            const float *src = (field == MMCA_FIELD_CE) ? b.ce32 : b.cl32[ctx->cur];
-            HIPCHK(hipMemcpy(tmp.data(), src, P * sizeof(float), hipMemcpyDeviceToHost));
-            double *h = (double *) host;
-            for (size_t i = 0; i < P; i++)
-                h[i] = c.cinit + (double) tmp[i];
+            double *wide;
+            TRY(staging(ctx, &wide));
+            HIPCHK(launch_widen((field == MMCA_FIELD_CE) ? b.ce32 : b.cl32[ctx->cur], wide, c.cinit, c.P, ctx->stream));
+            HIPCHK(hipMemcpyAsync(host, wide, P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(hipStreamSynchronize(ctx->stream));
         } else {
             const double *src = (field == MMCA_FIELD_CE) ? b.ce : b.cl[ctx->cur];
             HIPCHK(hipMemcpy(host, src, P * sizeof(double), hipMemcpyDeviceToHost));
