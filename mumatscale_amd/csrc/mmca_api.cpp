@@ -47,6 +47,9 @@ hipError_t launch_probe(int mix, long long n, double *a, double *b, double *f, f
                         hipStream_t s);
 long long list_words(const Consts &c);
 int list_blocks(const Consts &c);
+int count_blocks(const Consts &c);
+int list_unit(const Consts &c);
+int capture_blocks(const Consts &c);
 int reduce_blocks(const Consts &c);
 }  // namespace mmca
 
@@ -353,12 +356,13 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
         *desc = nullptr;
         *off = nullptr;
         TRY(dev_alloc(desc, (size_t) n));
-        TRY(dev_alloc(off, (size_t) 4 * (n + 1)));
+        TRY(dev_alloc(off, (size_t) 6 * (n + 1)));
         *cap = n;
     }
     std::vector<DomainDesc> h(n);
-    std::vector<long long> t((size_t) 4 * (n + 1), 0);
-    long long *on = &t[0], *oz = &t[n + 1], *oc = &t[2 * (n + 1)], *ol = &t[3 * (n + 1)];
+    std::vector<long long> t((size_t) 6 * (n + 1), 0);
+    long long *on = &t[0], *oz = &t[n + 1], *oc = &t[2 * (n + 1)], *ol = &t[3 * (n + 1)], *ok = &t[4 * (n + 1)],
+              *op = &t[5 * (n + 1)];
     for (int d = 0; d < n; d++) {
         h[d].b = ctxs[d]->b;
         h[d].c = ctxs[d]->c;
@@ -366,6 +370,8 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
         oz[d + 1] = oz[d] + (zm_by > 0 ? zm_tiles(ctxs[d]->c, zm_by) : 0);
         oc[d + 1] = oc[d] + cell_blocks(ctxs[d]->c);
         ol[d + 1] = ol[d] + list_blocks(ctxs[d]->c);
+        ok[d + 1] = ok[d] + count_blocks(ctxs[d]->c);
+        op[d + 1] = op[d] + capture_blocks(ctxs[d]->c);
     }
     HIPCHK(hipMemcpyAsync(*desc, h.data(), sizeof(DomainDesc) * (size_t) n, hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(*off, t.data(), sizeof(long long) * t.size(), hipMemcpyHostToDevice, s));
@@ -380,10 +386,14 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
     v->off_zm = *off + (n + 1);
     v->off_cell = *off + 2 * (n + 1);
     v->off_list = *off + 3 * (n + 1);
+    v->off_count = *off + 4 * (n + 1);
+    v->off_cap = *off + 5 * (n + 1);
     v->tot_nuc = on[n];
     v->tot_zm = oz[n];
     v->tot_cell = oc[n];
     v->tot_list = ol[n];
+    v->tot_count = ok[n];
+    v->tot_cap = op[n];
     return MMCA_OK;
 }
 
@@ -615,6 +625,7 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
     *out = ctx;     // destroy() frees partial allocations on failure
     HIPCHK(hipSetDevice(device));
     HIPCHK(hipStreamCreate(&ctx->stream));
+    ctx->c.list_w = list_unit(ctx->c);
     const Consts &c = ctx->c;
     DevBufs &b = ctx->b;
     const size_t P = (size_t) c.P;
@@ -647,6 +658,10 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
     b.nblk_list = list_blocks(c);
     TRY(dev_alloc(&b.blk_count, (size_t) b.nblk_list));
     TRY(dev_alloc(&b.row_first, (size_t) c.ny * c.nz));
+    TRY(dev_alloc(&b.list_done, 1));
+    TRY(dev_alloc(&b.nuc_done, 1));
+    HIPCHK(hipMemsetAsync(b.list_done, 0, sizeof(int), ctx->stream));
+    HIPCHK(hipMemsetAsync(b.nuc_done, 0, sizeof(int), ctx->stream));
     b.nblk_red = reduce_blocks(c);
     TRY(dev_alloc(&b.red_part, (size_t) 2 * b.nblk_red));
     TRY(dev_alloc(&ctx->d_red, 2));
@@ -711,7 +726,7 @@ int mmca_destroy(mmca_ctx *ctx)
         b.g_rot = nullptr, b.g_cell = nullptr, b.g_step = nullptr, b.g_src = nullptr, b.g_dom = nullptr;
     void *ptrs[] = { b.ce, b.cl[0], b.cl[1], b.ce32, b.cl32[0], b.cl32[1], b.ledger, b.fs[0], b.fs[1], b.gr, b.dc, b.mask,
                      b.xhalo,
-                     b.diff_id, b.nbr, b.dtx, b.dty, b.dtz, b.blk_count, b.row_first, b.site_idx, b.site_thr, b.site_fixed,
+                     b.diff_id, b.nbr, b.dtx, b.dty, b.dtz, b.blk_count, b.row_first, b.list_done, b.nuc_done, b.site_idx, b.site_thr, b.site_fixed,
                      b.site_ls, b.events, b.ev_blk, b.ev_cnt, b.g_rot, b.g_cell, b.g_step, b.g_src, b.g_dom, b.fixed_rot,
                      b.rand_rot,
                      b.oce, b.d, b.temp, b.temp32, b.beam_nodes, b.beam_zq, b.und, b.und_n,

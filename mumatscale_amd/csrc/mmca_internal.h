@@ -29,6 +29,7 @@ struct Consts {
     int zm_lds;             // MMCA_TUNE_ZM_LDS as set (both values run the same kernel)
     int capture_chunk;      // > 0: capture deals list slots in chunks of this many, pinned to XCDs
     int capture_band;       // > 0: capture works on units of this many rows of one plane, band q on XCD q % 8
+    int list_w;             // mask words per list workgroup (64 or 256)
     int track_d;            // 1: keep the reference's d array (stale values of cells no longer solid)
     int f32;                // 1: ce, cl stored as FP32 deviations from cinit
     // diffusion (growth.c:38-40)
@@ -94,6 +95,7 @@ struct DevBufs {
     int *blk_count;                  // per-block member counts -> offsets
     int *row_first;                  // per interior row (k-1) ny + (j-1): slot of its first list member
     int nblk_list;
+    int *list_done, *nuc_done;       // workgroups of the list count / of detection that have finished (0 between launches)
     // nucleation sites, sorted by padded index
     int *site_idx;
     float *site_thr;
@@ -161,8 +163,10 @@ struct View {
     const long long *off_nuc;    // k_nuc_detect workgroups
     const long long *off_zm;     // z-marching solute tiles
     const long long *off_cell;   // cell-parallel solute workgroups
-    const long long *off_list;   // list count / capture workgroups
-    long long tot_nuc, tot_zm, tot_cell, tot_list;
+    const long long *off_list;   // list writer workgroups
+    const long long *off_count;  // list count workgroups
+    const long long *off_cap;    // capture workgroups
+    long long tot_nuc, tot_zm, tot_cell, tot_list, tot_count, tot_cap;
 };
 
 }  // namespace mmca

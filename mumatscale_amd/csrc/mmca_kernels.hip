@@ -1,19 +1,23 @@
 // HIP kernels of the CA step for gfx950 (CDNA4, wave64).
 //
-// One step (doiteration, calculate.c:193-352) on one subblock is seven
+// One step (doiteration, calculate.c:193-352) on one subblock is five
 // launches on the context's stream:
 //   k_nuc_detect    cell_nucleation (grain.c:1222-1318) over the sorted site list
-//   k_nuc_activate  activateNewGrains (grain.c:841-916): ids in site order, one workgroup
+//                   and, in the workgroup that finishes last, activateNewGrains
+//                   (grain.c:841-916): ids in site order
 //   k_solute_rw     diffusion + partitioning (growth.c:30-170, 177-276),
 //                   fused, and a 1-bit "solid" mask of gr > 0
 //   k_list_count    interface-list membership counts from the mask
-//                   (grow_cell_reduction, growth.c:461-538)
-//   k_list_scan     exclusive scan of the counts -> raster-order slots
+//                   (grow_cell_reduction, growth.c:461-538) and, in the
+//                   workgroup that finishes last, their exclusive scan ->
+//                   raster-order slots
 //   k_list_write    the list itself (diff_id) in raster order
 //   k_capture       capture_octahedra_diffuse (growth.c:574-807) over the
 //                   list slots, dealt evenly over the whole grid, with the
 //                   octahedron half-diagonal of each candidate neighbour
 //                   computed on the fly (grow_octahedra, growth.c:339-407)
+// A Gaussian-beam block adds the approximate beam temperature before them
+// (k_beam_ax, k_beam_field) and k_beam_finish after the solute kernel.
 //
 // Arithmetic follows the reference's operation order and is compiled with
 // -ffp-contract=off: FP64 results are bit-identical with the reference CPU
@@ -154,6 +158,45 @@ block_exscan_int(int v, int *total, int *s_w)
     return off + incl - v;
 }
 
+// Values handed from the workgroups of a launch to the one that finishes last
+// (last_workgroup): stores and loads at agent scope go past the L2s, of which
+// every XCD has its own.
+template <typename T>
+__device__ __forceinline__ void
+st_agent(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename T>
+__device__ __forceinline__ T
+ld_agent(const T *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True in the workgroup, of n, that gets here last; all of its threads call it.
+// Every thread first waits until its st_agent stores have arrived, so that the
+// last workgroup's ld_agent loads see all of them; a __threadfence() instead
+// would write back and invalidate the whole L2 in every workgroup (it took
+// k_list_count of a 256 x 256 x 512 block from 7 to 150 us).  *done is 0
+// before and after.
+__device__ __forceinline__ bool
+last_workgroup(int *done, int n)
+{
+    __shared__ int s_last;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        s_last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+        if (s_last)
+            *done = 0;
+    }
+    __syncthreads();
+    return s_last != 0;
+}
+
 // Domain of workgroup w: the last d with off[d] <= w (domains without work
 // share their offset with the next domain).
 __device__ __forceinline__ int
@@ -172,115 +215,44 @@ find_dom(const long long *off, int ndom, long long w)
 }
 
 // ---------------------------------------------------------------------------
-// cell_nucleation (grain.c:1222-1318): one thread per site, sites sorted by
-// padded index; each workgroup compacts its events in site order.
+// ---------------------------------------------------------------------------
 constexpr int NUC_BS = 256;
-
-__global__ void __launch_bounds__(NUC_BS)
-k_nuc_detect(View V, int advance, int cur)
-{
-    __shared__ int s_w[NUC_BS / 64];
-    const int d = find_dom(V.off_nuc, V.ndom, blockIdx.x);
-    const long long blk = blockIdx.x - V.off_nuc[d];
-    const DevBufs b = V.dom[d].b;    // private copy: stores cannot alias it
-    const Consts c = V.dom[d].c;
-    const MMCA_GLOBAL Counters *cnt = G(b.cnt);
-    if (cnt->status != MMCA_OK)
-        return;
-    const unsigned long long ts = cnt->timestep + (advance ? 1ull : 0ull);
-    const double sim_time = ts * c.dt;
-    const int s = (int) blk * NUC_BS + threadIdx.x;
-    int flag = 0;
-    if (s < b.nsites)
-    {
-        int idx = G(b.site_idx)[s];
-        int z = (int) (idx / c.sxy);
-        int rem = (int) (idx - z * c.sxy);
-        int y = rem / c.sx;
-        int x = rem - y * c.sx;
-        double T;
-        if (c.am)
-        {
-            // The tests below read T only through comparisons (undercooling
-            // falls with T where the slope m is constant): where they all come
-            // out the same at both ends of the approximate temperature's
-            // interval, it will do.
-            T = (double) G(b.temp32)[idx];
-            const double d = beam_margin(c, T);
-            const double lo = T - d, hi = T + d;
-            const double cl = c.f32 ? ld_cl<true>(b, c, cur, idx) : ld_cl<false>(b, c, cur, idx);
-            const double add = c.mc * (cl - c.cinit), thr = (double) G(b.site_thr)[s];
-            const bool same = (lo > c.Tliq || hi <= c.Tliq) && (lo >= c.Tsol || hi < c.Tsol) &&
-                              ((c.Tliq - hi) + add > thr || (c.Tliq - lo) + add <= thr);
-            if (!(c.ma == 0.0 && c.mb == 0.0 && same))
-                T = temp_model<true>(c, sim_time, x, y, z);
-        }
-        else
-            T = temp_model<false>(c, sim_time, x, y, z);
-        int layerno = 1, initnuc = 1;
-        if (c.am)
-        {
-            // tempUpdateSB_int sets lsindex before nucleation (temperature.c:256-259)
-            if (T > c.Tliq)
-                G(b.site_ls)[s] = 1;
-            if (c.am_layers == 1)
-                layerno = 1;
-            else if (c.am_layers > 1 && G(b.site_ls)[s] == 1)
-                layerno = 1;
-            else
-                layerno = 0;
-            if (sim_time <= 1e-4)
-                initnuc = 1;
-            else if (T >= c.Tsol)
-                initnuc = 1;
-            else
-                initnuc = 0;
-        }
-        if (G(b.gr)[idx] <= 0 && layerno && initnuc)
-        {
-            double Tunder = c.Tliq - T;
-            double m_solute0 = c.ma * T * T + c.mb * T + c.mc;
-            Tunder += m_solute0 * ((c.f32 ? ld_cl<true>(b, c, cur, idx) : ld_cl<false>(b, c, cur, idx)) - c.cinit);
-            if (Tunder > (double) G(b.site_thr)[s])
-                flag = 1;
-        }
-    }
-    int tot;
-    int r = block_exscan_flag<NUC_BS / 64>(flag, &tot, s_w);
-    if (flag)
-        G(b.ev_blk)[blk * NUC_BS + r] = s;
-    if (threadIdx.x == 0)
-        G(b.ev_cnt)[blk] = tot;
-}
 
 // Event ordering and activateNewGrains/createGrains on one rank
 // (grain.c:841-916, 348-425), one workgroup.
-// mode: 1 = order the detected events, 2 = activate, 4 = advance the timestep.
-__global__ void __launch_bounds__(NUC_BS)
-k_nuc_activate(View V, int mode)
+// mode: 1 = order the detected events, 2 = activate, 4 = advance the timestep
+// (k_nuc_detect: 8 = detect at the next timestep without advancing).
+// nev1 >= 0: the number of events of a domain with one detecting workgroup,
+// already in order in `events`.
+__device__ __forceinline__ void
+nuc_activate(const DevBufs &b, const Consts &c, int mode, int nev1)
 {
     __shared__ int s_w[NUC_BS / 64];
     __shared__ int s_nev;
-    const DevBufs b = V.dom[blockIdx.x].b;    // private copy: stores cannot alias it
-    const Consts c = V.dom[blockIdx.x].c;
     const int nblk = (b.nsites + NUC_BS - 1) / NUC_BS;
     Counters *cnt = b.cnt;
-    if (cnt->status != MMCA_OK)
-        return;
     const int tid = threadIdx.x;
     const unsigned long long ts = cnt->timestep + ((mode & 4) ? 1ull : 0ull);
-    if (mode & 1)
+    if (nev1 >= 0)
+    {
+        if (tid == 0)
+        {
+            s_nev = nev1;
+            cnt->n_events = nev1;
+        }
+    }
+    else if (mode & 1)
     {
         // exclusive scan of the per-workgroup counts, then concatenate
         int carry = 0;
         for (int base = 0; base < nblk; base += NUC_BS)
         {
             int blk = base + tid;
-            int v = (blk < nblk) ? G(b.ev_cnt)[blk] : 0;
+            int v = (blk < nblk) ? ld_agent(&b.ev_cnt[blk]) : 0;
             int tot;
             int off = carry + block_exscan_int<NUC_BS / 64>(v, &tot, s_w);
             for (int i = 0; i < v; ++i)
-                G(b.events)[off + i] = G(b.ev_blk)[blk * NUC_BS + i];
+                G(b.events)[off + i] = ld_agent(&b.ev_blk[blk * NUC_BS + i]);
             carry += tot;
         }
         if (tid == 0)
@@ -363,6 +335,111 @@ k_nuc_activate(View V, int mode)
     if ((mode & 4) && tid == 0)
         cnt->timestep = ts;
 }
+
+// activation on its own (mmca_activate_new_grains)
+__global__ void __launch_bounds__(NUC_BS)
+k_nuc_activate(View V, int mode)
+{
+    const DevBufs b = V.dom[blockIdx.x].b;    // private copy: stores cannot alias it
+    const Consts c = V.dom[blockIdx.x].c;
+    if (b.cnt->status != MMCA_OK)
+        return;
+    nuc_activate(b, c, mode, -1);
+}
+
+// cell_nucleation (grain.c:1222-1318): one thread per site, sites sorted by
+// padded index; each workgroup compacts its events in site order.  The
+// workgroup of a domain that finishes last orders them and, by `mode`,
+// activates the grains (nuc_activate): one launch where detection and
+// activation took two of 4.6 us each, nearly all of it launch latency.
+__global__ void __launch_bounds__(NUC_BS)
+k_nuc_detect(View V, int mode, int cur)
+{
+    __shared__ int s_w[NUC_BS / 64];
+    const int d = find_dom(V.off_nuc, V.ndom, blockIdx.x);
+    const long long blk = blockIdx.x - V.off_nuc[d];
+    const DevBufs b = V.dom[d].b;    // private copy: stores cannot alias it
+    const Consts c = V.dom[d].c;
+    const MMCA_GLOBAL Counters *cnt = G(b.cnt);
+    if (cnt->status != MMCA_OK)
+        return;
+    const unsigned long long ts = cnt->timestep + ((mode & 12) ? 1ull : 0ull);
+    const double sim_time = ts * c.dt;
+    const int s = (int) blk * NUC_BS + threadIdx.x;
+    int flag = 0;
+    if (s < b.nsites)
+    {
+        int idx = G(b.site_idx)[s];
+        int z = (int) (idx / c.sxy);
+        int rem = (int) (idx - z * c.sxy);
+        int y = rem / c.sx;
+        int x = rem - y * c.sx;
+        double T;
+        if (c.am)
+        {
+            // The tests below read T only through comparisons (undercooling
+            // falls with T where the slope m is constant): where they all come
+            // out the same at both ends of the approximate temperature's
+            // interval, it will do.
+            T = (double) G(b.temp32)[idx];
+            const double d = beam_margin(c, T);
+            const double lo = T - d, hi = T + d;
+            const double cl = c.f32 ? ld_cl<true>(b, c, cur, idx) : ld_cl<false>(b, c, cur, idx);
+            const double add = c.mc * (cl - c.cinit), thr = (double) G(b.site_thr)[s];
+            const bool same = (lo > c.Tliq || hi <= c.Tliq) && (lo >= c.Tsol || hi < c.Tsol) &&
+                              ((c.Tliq - hi) + add > thr || (c.Tliq - lo) + add <= thr);
+            if (!(c.ma == 0.0 && c.mb == 0.0 && same))
+                T = temp_model<true>(c, sim_time, x, y, z);
+        }
+        else
+            T = temp_model<false>(c, sim_time, x, y, z);
+        int layerno = 1, initnuc = 1;
+        if (c.am)
+        {
+            // tempUpdateSB_int sets lsindex before nucleation (temperature.c:256-259)
+            if (T > c.Tliq)
+                G(b.site_ls)[s] = 1;
+            if (c.am_layers == 1)
+                layerno = 1;
+            else if (c.am_layers > 1 && G(b.site_ls)[s] == 1)
+                layerno = 1;
+            else
+                layerno = 0;
+            if (sim_time <= 1e-4)
+                initnuc = 1;
+            else if (T >= c.Tsol)
+                initnuc = 1;
+            else
+                initnuc = 0;
+        }
+        if (G(b.gr)[idx] <= 0 && layerno && initnuc)
+        {
+            double Tunder = c.Tliq - T;
+            double m_solute0 = c.ma * T * T + c.mb * T + c.mc;
+            Tunder += m_solute0 * ((c.f32 ? ld_cl<true>(b, c, cur, idx) : ld_cl<false>(b, c, cur, idx)) - c.cinit);
+            if (Tunder > (double) G(b.site_thr)[s])
+                flag = 1;
+        }
+    }
+    int tot;
+    int r = block_exscan_flag<NUC_BS / 64>(flag, &tot, s_w);
+    const int nwg = (int) (V.off_nuc[d + 1] - V.off_nuc[d]);
+    if (nwg == 1)
+    {
+        // nothing to wait for or to order
+        if (flag)
+            G(b.events)[r] = s;
+        nuc_activate(b, c, mode, tot);
+        return;
+    }
+    if (flag)
+        st_agent(&b.ev_blk[blk * NUC_BS + r], s);
+    if (threadIdx.x == 0)
+        st_agent(&b.ev_cnt[blk], tot);
+    if (last_workgroup(b.nuc_done, nwg))
+        nuc_activate(b, c, mode, -1);
+}
+
 
 // activateNewGrains over the ranks of a coupled batch (grain.c:841-916), one
 // workgroup: each domain's ordered events (k_nuc_activate mode 1) get ids
@@ -1252,6 +1329,13 @@ list_words_d(const Consts &c)
     return (long long) c.nz * c.ny * c.w64;
 }
 
+// workgroups of the list writer: list_w mask words each
+__host__ __device__ __forceinline__ int
+list_blocks_d(const Consts &c)
+{
+    return (int) ((list_words_d(c) + c.list_w - 1) / c.list_w);
+}
+
 __device__ __forceinline__ unsigned long long
 mask_word(const DevBufs &b, const Consts &c, int k, int j, int w)
 {
@@ -1310,69 +1394,108 @@ member_bits(const DevBufs &b, const Consts &c, long long wi, int *pk, int *pj, i
     return ~own & (left | right | yz) & inter;
 }
 
+// Offsets of the list workgroups from their counts, by one workgroup of BS
+// threads, and, when decide_realloc is set, the dc_tmp growth rule of
+// growth.c:644-660.  AGENT: the counts come from workgroups of this launch.
+template <int BS, bool AGENT>
+__device__ __forceinline__ void
+list_scan(const DevBufs &b, const Consts &c, int decide_realloc)
+{
+    __shared__ int s_w[BS / 64];
+    const int tid = threadIdx.x, nblk = list_blocks_d(c);
+    int tot = 0;
+    for (int base = 0; base < nblk; base += BS)
+    {
+        const int i = base + tid;
+        int v = 0, n;
+        if (i < nblk)
+            v = AGENT ? ld_agent(&b.blk_count[i]) : G(b.blk_count)[i];
+        const int ex = block_exscan_int<BS / 64>(v, &n, s_w);
+        if (i < nblk)
+            G(b.blk_count)[i] = tot + ex;
+        tot += n;
+    }
+    if (tid == 0)
+    {
+        Counters *cnt = b.cnt;
+        cnt->gindex = tot;
+        if (decide_realloc)
+        {
+            if (tot > cnt->dc_tmp_size)
+            {
+                cnt->realloc_old = cnt->dc_tmp_size;
+                cnt->dc_tmp_size = tot + 100;
+            }
+            else
+                cnt->realloc_old = -1;
+        }
+    }
+}
+
+// Counts the members of every list workgroup (c.list_w words of k_list_write).
+// FUSED: the workgroup of a domain that finishes last also scans the counts,
+// which takes k_list_scan's launch (4.7 us) out of the step of small blocks.
+template <bool FUSED>
 __global__ void __launch_bounds__(LIST_BS)
-k_list_count(View V)
+k_list_count(View V, int decide_realloc)
 {
     __shared__ int s_w[LIST_BS / 64];
-    const int dm = find_dom(V.off_list, V.ndom, blockIdx.x);
-    const long long blk = blockIdx.x - V.off_list[dm];
+    const int dm = find_dom(V.off_count, V.ndom, blockIdx.x);
+    const long long blk = blockIdx.x - V.off_count[dm];
     const DevBufs b = V.dom[dm].b;    // private copy: stores cannot alias it
     const Consts c = V.dom[dm].c;
     const long long nwords = list_words_d(c);
     if (G(b.cnt)->status != MMCA_OK)
         return;
-    const long long wi = blk * LIST_BS + threadIdx.x;
+    const int tid = threadIdx.x;
+    const long long wi = blk * LIST_BS + tid;
     int v = 0;
     if (wi < nwords)
     {
         int k, j, w;
         v = __popcll(member_bits(b, c, wi, &k, &j, &w));
     }
-    int tot;
-    block_exscan_int<LIST_BS / 64>(v, &tot, s_w);
-    if (threadIdx.x == 0)
-        G(b.blk_count)[blk] = tot;
+    if (c.list_w == 64)
+    {
+        // one count per wave
+        for (int d = 32; d > 0; d >>= 1)
+            v += __shfl_xor(v, d, 64);
+        const long long q = blk * (LIST_BS / 64) + (tid >> 6);
+        if ((tid & 63) == 0 && q < list_blocks_d(c))
+        {
+            if (FUSED)
+                st_agent(&b.blk_count[q], v);
+            else
+                G(b.blk_count)[q] = v;
+        }
+    }
+    else
+    {
+        int tot;
+        block_exscan_int<LIST_BS / 64>(v, &tot, s_w);
+        if (tid == 0)
+        {
+            if (FUSED)
+                st_agent(&b.blk_count[blk], tot);
+            else
+                G(b.blk_count)[blk] = tot;
+        }
+    }
+    if constexpr (FUSED)
+        if (last_workgroup(b.list_done, (int) (V.off_count[dm + 1] - V.off_count[dm])))
+            list_scan<LIST_BS, true>(b, c, decide_realloc);
 }
 
-// Exclusive scan of the block counts (one workgroup).  When decide_realloc
-// is set, also applies the dc_tmp growth rule of growth.c:644-660.
 constexpr int SCAN_BS = 1024;
 
 __global__ void __launch_bounds__(SCAN_BS)
 k_list_scan(View V, int decide_realloc)
 {
-    __shared__ int s_w[SCAN_BS / 64];
     const DevBufs b = V.dom[blockIdx.x].b;    // private copy: stores cannot alias it
     const Consts c = V.dom[blockIdx.x].c;
-    const int nblk = (int) ((list_words_d(c) + LIST_BS - 1) / LIST_BS);
-    Counters *cnt = b.cnt;
-    if (cnt->status != MMCA_OK)
+    if (b.cnt->status != MMCA_OK)
         return;
-    int carry = 0;
-    for (int base = 0; base < nblk; base += SCAN_BS)
-    {
-        int i = base + threadIdx.x;
-        int v = (i < nblk) ? G(b.blk_count)[i] : 0;
-        int tot;
-        int ex = block_exscan_int<SCAN_BS / 64>(v, &tot, s_w);
-        if (i < nblk)
-            G(b.blk_count)[i] = carry + ex;
-        carry += tot;
-    }
-    if (threadIdx.x == 0)
-    {
-        cnt->gindex = carry;
-        if (decide_realloc)
-        {
-            if (carry > cnt->dc_tmp_size)
-            {
-                cnt->realloc_old = cnt->dc_tmp_size;
-                cnt->dc_tmp_size = carry + 100;
-            }
-            else
-                cnt->realloc_old = -1;
-        }
-    }
+    list_scan<SCAN_BS, false>(b, c, decide_realloc);
 }
 
 __global__ void
@@ -1430,11 +1553,17 @@ k_list_write(View V)
     const long long nwords = list_words_d(c);
     if (G(b.cnt)->status != MMCA_OK)
         return;
-    const long long wi0 = blk * LIST_BS;
+    const int base = G(b.blk_count)[blk];            // members before this workgroup
+    const int next = blk + 1 < list_blocks_d(c) ? G(b.blk_count)[blk + 1] : G(b.cnt)->gindex;
+    if (next == base && c.capture_band == 0)
+        return;                                      // no members (the bands need every row's slot)
+    const int W = c.list_w;                          // words of a workgroup: 64 or LIST_BS
+    const long long wi0 = blk * W;
     const long long wi = wi0 + threadIdx.x;
+    const bool mine = (int) threadIdx.x < W && wi < nwords;
     unsigned long long mem = 0;
     unsigned long long nb[6] = { 0, 0, 0, 0, 0, 0 };
-    if (wi < nwords)
+    if (mine)
     {
         int k, j, w;
         word_pos(c, wi, &k, &j, &w);
@@ -1458,8 +1587,7 @@ k_list_write(View V)
         s_nb[n][threadIdx.x] = nb[n];
     s_ex[threadIdx.x] = ex;
     __syncthreads();
-    const int base = G(b.blk_count)[blk];            // members before this workgroup
-    if (wi < nwords)
+    if (mine)
     {
         // slot of the first member of each row (of the next member after the
         // row's start when the row has none), for capture's row bands
@@ -1471,7 +1599,7 @@ k_list_write(View V)
     for (int i = threadIdx.x; i < tot; i += LIST_BS)
     {
         // word of member i: the last word whose prefix count is <= i
-        int lo = 0, hi = LIST_BS - 1;
+        int lo = 0, hi = W - 1;
         while (lo < hi)
         {
             int mid = (lo + hi + 1) >> 1;
@@ -1502,9 +1630,9 @@ k_list_write(View V)
 __global__ void __launch_bounds__(LIST_BS)
 k_capture(View V, int cb, int rows)
 {
-    const int dm = find_dom(V.off_list, V.ndom, blockIdx.x);
-    const long long blk = blockIdx.x - V.off_list[dm];
-    const long long nwg = V.off_list[dm + 1] - V.off_list[dm];
+    const int dm = find_dom(V.off_cap, V.ndom, blockIdx.x);
+    const long long blk = blockIdx.x - V.off_cap[dm];
+    const long long nwg = V.off_cap[dm + 1] - V.off_cap[dm];
     const long long nthr = nwg * LIST_BS;
     const DevBufs b = V.dom[dm].b;    // private copy: stores cannot alias it
     const Consts c = V.dom[dm].c;
@@ -1643,7 +1771,7 @@ k_capture(View V, int cb, int rows)
         // neighbours lie in its own row, in the rows next to it (mostly in
         // the same unit: one workgroup, one L1) and in the planes next to it
         // (units of the same XCD in flight together: one L2).
-        const long long o = V.off_list[dm];
+        const long long o = V.off_cap[dm];
         const int xcd = (int) (blockIdx.x % 8);
         const long long first = o + ((xcd - (int) (o % 8)) + 8) % 8;
         const long long rank = (blockIdx.x - first) / 8;
@@ -1672,7 +1800,7 @@ k_capture(View V, int cb, int rows)
         // w % 8; the workgroups of this domain on one XCD stride over the
         // 256-slot groups of that XCD's chunks.
         const int S = chunk / LIST_BS;
-        const long long o = V.off_list[dm];
+        const long long o = V.off_cap[dm];
         const int xcd = (int) (blockIdx.x % 8);
         const long long first = o + ((xcd - (int) (o % 8)) + 8) % 8;
         const long long rank = (blockIdx.x - first) / 8;
@@ -2135,7 +2263,7 @@ hipError_t launch_beam_field(const DevBufs &b, const Consts &c, const BeamSet &p
 // at most 1024 workgroups per domain: four waves per SIMD of the whole chip
 hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStream_t s)
 {
-    const long long per = (v.tot_list * LIST_BS * 64 / v.ndom + 1023) / 1024;     // cells per domain / 1024, about
+    const long long per = (v.tot_count * LIST_BS * 64 / v.ndom + 1023) / 1024;     // cells per domain / 1024, about
     const dim3 grid((unsigned) std::max<long long>(1, std::min<long long>(1024, per)), (unsigned) v.ndom);
     if (f32)
         hipLaunchKernelGGL(k_beam_finish<true>, grid, dim3(256), 0, s, v, cur, nxt);
@@ -2226,20 +2354,19 @@ k_grow_octahedra(DevBufs b, Consts c, int cb)
 // Launch wrappers (host side).
 hipError_t launch_nucleate(const View &v, int mode, int cur, hipStream_t s)
 {
-    if ((mode & 1) && v.tot_nuc > 0)
-        hipLaunchKernelGGL(k_nuc_detect, dim3((unsigned) v.tot_nuc), dim3(NUC_BS), 0, s, v,
-                           (mode & 4) ? 1 : 0, cur);
-    hipLaunchKernelGGL(k_nuc_activate, dim3(v.ndom), dim3(NUC_BS), 0, s, v, mode);
+    if (mode & 1)
+        hipLaunchKernelGGL(k_nuc_detect, dim3((unsigned) v.tot_nuc), dim3(NUC_BS), 0, s, v, mode, cur);
+    else
+        hipLaunchKernelGGL(k_nuc_activate, dim3(v.ndom), dim3(NUC_BS), 0, s, v, mode);
     return hipGetLastError();
 }
 
 // Nucleation of a coupled batch: detection and event order per domain, then
-// activation across the domains in rank order.
+// activation across the domains in rank order (which advances the timestep:
+// detection works at the next one).
 hipError_t launch_nucleate_coupled(const View &v, int cur, hipStream_t s)
 {
-    if (v.tot_nuc > 0)
-        hipLaunchKernelGGL(k_nuc_detect, dim3((unsigned) v.tot_nuc), dim3(NUC_BS), 0, s, v, 1, cur);
-    hipLaunchKernelGGL(k_nuc_activate, dim3(v.ndom), dim3(NUC_BS), 0, s, v, 1);
+    hipLaunchKernelGGL(k_nuc_detect, dim3((unsigned) v.tot_nuc), dim3(NUC_BS), 0, s, v, 1 | 8, cur);
     hipLaunchKernelGGL(k_nuc_activate_coupled, dim3(1), dim3(NUC_BS), 0, s, v);
     return hipGetLastError();
 }
@@ -2316,8 +2443,23 @@ hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s)
 }
 
 long long list_words(const Consts &c) { return list_words_d(c); }
-int list_blocks(const Consts &c) { return (int) ((list_words(c) + LIST_BS - 1) / LIST_BS); }
-int nuc_blocks(int nsites) { return (nsites + NUC_BS - 1) / NUC_BS; }
+int list_blocks(const Consts &c) { return list_blocks_d(c); }
+int count_blocks(const Consts &c) { return (int) ((list_words(c) + LIST_BS - 1) / LIST_BS); }
+// The list writer takes 64 words per workgroup while that gives at most 2048
+// workgroups (15.4 -> 7.7 us for the 65536 words and 450 000 members of 128 x
+// 128 x 256, which gave 256 workgroups), and 256 in larger blocks: with 8192
+// workgroups of 64 words, 256 x 256 x 512 takes 22.6 us to write and 10.3 to
+// scan, against 16.5 and 4.7.
+int list_unit(const Consts &c) { return list_words(c) <= 64 * 2048 ? 64 : LIST_BS; }
+// Capture's workgroups: the list's slots are dealt to their threads, so a small
+// block needs more of them than its mask has words (40 x 36 x 44: 7 workgroups
+// took 19.5 us for 13 000 slots, 62 take 6.5).
+int capture_blocks(const Consts &c)
+{
+    const long long cells = (long long) c.nx * c.ny * c.nz;
+    return (int) std::max<long long>((list_words(c) + LIST_BS - 1) / LIST_BS, std::min<long long>(1024, (cells + 1023) / 1024));
+}
+int nuc_blocks(int nsites) { return std::max(1, (nsites + NUC_BS - 1) / NUC_BS); }   // at least the one that activates
 long long cell_blocks(const Consts &c)
 {
     return (long long) ((c.nx + SOL_BX - 1) / SOL_BX) * ((c.ny + SOL_BY - 1) / SOL_BY) *
@@ -2328,23 +2470,35 @@ long long zm_tiles(const Consts &c, int by)
     return (long long) ((c.nx + 63) / 64) * ((c.ny + by - 1) / by) * ((c.nz + c.zm_planes - 1) / c.zm_planes);
 }
 
+// Up to this many list-count workgroups the scan runs in their launch: a 40 x
+// 36 x 44 block (7 workgroups) steps in 28.3 instead of 29.4 us, a 99 x 130 x
+// 121 one (123) in 47.8 instead of 48.2; 150 x 140 x 165 (271) takes 65.9 against
+// 63.8 us with a launch of its own, 256 x 256 x 512 (8192) 603 against 571: the
+// counter that orders the workgroups is one address for all XCDs.
+constexpr long long LIST_FUSED = 192;
+
 hipError_t launch_list(const View &v, int cb, int capture, int decide_realloc, hipStream_t s)
 {
-    if (v.tot_list > 0)
-        hipLaunchKernelGGL(k_list_count, dim3((unsigned) v.tot_list), dim3(LIST_BS), 0, s, v);
-    hipLaunchKernelGGL(k_list_scan, dim3(v.ndom), dim3(SCAN_BS), 0, s, v, decide_realloc);
-    if (capture >= 0 && v.tot_list > 0)
+    const dim3 grid((unsigned) v.tot_count);
+    if (v.tot_count <= LIST_FUSED)
+        hipLaunchKernelGGL(k_list_count<true>, grid, dim3(LIST_BS), 0, s, v, decide_realloc);
+    else
+    {
+        hipLaunchKernelGGL(k_list_count<false>, grid, dim3(LIST_BS), 0, s, v, decide_realloc);
+        hipLaunchKernelGGL(k_list_scan, dim3(v.ndom), dim3(SCAN_BS), 0, s, v, decide_realloc);
+    }
+    if (capture >= 0)
         hipLaunchKernelGGL(k_list_write, dim3((unsigned) v.tot_list), dim3(LIST_BS), 0, s, v);
-    if (capture > 0 && v.tot_list > 0)
-        hipLaunchKernelGGL(k_capture, dim3((unsigned) v.tot_list), dim3(LIST_BS), 0, s, v, cb, 1);
+    if (capture > 0)
+        hipLaunchKernelGGL(k_capture, dim3((unsigned) v.tot_cap), dim3(LIST_BS), 0, s, v, cb, 1);
     return hipGetLastError();
 }
 
 hipError_t launch_capture_only(const View &v, const DevBufs &b, int cb, hipStream_t s)
 {
     hipLaunchKernelGGL(k_realloc_decide, dim3(1), dim3(1), 0, s, b);
-    if (v.tot_list > 0)   // the list may come from a state image, which holds no row_first
-        hipLaunchKernelGGL(k_capture, dim3((unsigned) v.tot_list), dim3(LIST_BS), 0, s, v, cb, 0);
+    // the list may come from a state image, which holds no row_first
+    hipLaunchKernelGGL(k_capture, dim3((unsigned) v.tot_cap), dim3(LIST_BS), 0, s, v, cb, 0);
     return hipGetLastError();
 }
 
