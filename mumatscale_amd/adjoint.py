@@ -152,26 +152,26 @@ def backward(traj, params, checkpoints, K, g_ce, g_cl=None, g_fs=None):
     g = [g_ce.clone(),
          torch.zeros_like(g_ce) if g_cl is None else g_cl.clone(),
          torch.zeros_like(g_ce) if g_fs is None else g_fs.clone()]
+    g_in = [t.clone() for t in g]           # a step out of place is one pass (halo cells are never written)
     g_param = torch.zeros(3, dtype=torch.float64, device=dev)
     T = traj.nsteps
     nseg = (T + K - 1) // K
+    # states of a segment after its checkpoint: the halo cells, which no step
+    # writes, hold the same values in every state
+    seg_states = [tuple(t.clone() for t in checkpoints[0]) for _ in range(min(T, K) - 1)]
     for seg in range(nseg - 1, -1, -1):
         s0 = seg * K
         s1 = min(T, s0 + K)
-        states = [checkpoints[seg]]
+        states = [checkpoints[seg]] + seg_states
         for s in range(s0, s1 - 1):
-            out = tuple(torch.empty_like(t) for t in states[-1])
-            for o, i in zip(out, states[-1]):
-                o.copy_(i)                      # halo cells are never written
-            replay_step(params, traj.t0 + s + 1, traj.codes[s], states[-1], out)
-            states.append(out)
+            replay_step(params, traj.t0 + s + 1, traj.codes[s], states[s - s0], states[s - s0 + 1])
         for s in range(s1 - 1, s0 - 1, -1):
             st = states[s - s0]
             _check(L.mmca_adjoint_step(C.byref(params), traj.t0 + s + 1, _ptr(traj.codes[s]), _ptr(st[0]),
-                                       _ptr(st[1]), _ptr(st[2]), _ptr(g[0]), _ptr(g[1]), _ptr(g[2]), _ptr(g[0]),
-                                       _ptr(g[1]), _ptr(g[2]), _ptr(g_param), _ptr(ws), _stream()),
+                                       _ptr(st[1]), _ptr(st[2]), _ptr(g[0]), _ptr(g[1]), _ptr(g[2]), _ptr(g_in[0]),
+                                       _ptr(g_in[1]), _ptr(g_in[2]), _ptr(g_param), _ptr(ws), _stream()),
                    "mmca_adjoint_step")
-        del states
+            g, g_in = g_in, g
     return g, g_param
 
 

@@ -14,17 +14,18 @@
 //   A = 1 - km fs,  dce = ce' - ce,  c_int = c0 + m_inv (T - T_liq)
 // k_replay evaluates it with the forward kernel's expressions (bit-identical
 // with the recorded run at the recorded parameters).  The adjoint of one
-// step is two kernels:
-//   k_adj_part  per cell: recomputes ce', back-propagates the branch to
-//               lam = dL/dce' and to the direct dependence on (ce, cl, fs)
-//   k_adj_diff  per cell: gathers lam of the 6 neighbours through the
-//               diffusion stencil
-// and a one-workgroup sum of the parameter partials (fixed order, so the
-// gradients are reproducible run to run).
+// step back-propagates the branch of each cell to lam = dL/dce' and to the
+// direct dependence on (ce, cl, fs), gathers lam of the 6 neighbours through
+// the diffusion stencil, and sums the parameter partials in fixed order, so
+// that the gradients are reproducible run to run:
+//   k_adj_fused            all of it in one pass, outputs apart from inputs
+//   k_adj_part, _diff, _sum  the same in place
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
+#include <initializer_list>
 #include <mutex>
 
 #include "host_init.h"
@@ -171,9 +172,383 @@ k_replay(Consts c, const unsigned char *code, double sim_time, const double *ce,
     fs_o[q.idx] = fsv;
 }
 
-// Per-cell adjoint of the branch.  Writes lam = dL/dce' and the direct
-// derivatives with respect to the cell's own (ce, cl, fs); partials of
-// (d_liq, part_coef) per workgroup into part[2 * blk].
+// What the branch of a cell passes back: lam = dL/dce', the direct
+// derivatives with respect to its own (ce, cl, fs), and its terms of the
+// derivatives with respect to d_liq and part_coef.
+struct BranchAdj {
+    double lam, ce, cl, fs, dl, k;
+};
+
+// `diffused` gives ce': most waves are in the liquid throughout, where
+// nothing depends on it, and a cell for which only lam is wanted (!own) needs
+// it where the cell grows.
+template <bool AM, typename Diffused>
+__device__ __forceinline__ BranchAdj
+branch_adjoint(const Consts &c, const Deriv &dv, int br, double sim_time, int x, int j, int k, double ce_old,
+               double conc, double lspfs, Diffused diffused, bool own, double ga, double gb, double ge)
+{
+    BranchAdj r = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    if (br == MMCA_BRANCH_SOLID)
+    {
+        // cl' = ce' k_inv, fs' = fs
+        r.lam = ga + gb * c.k_inv;
+        r.fs = ge;
+        if (own)
+            r.k = -gb * diffused() * c.k_inv * c.k_inv;
+    }
+    else if (br == MMCA_BRANCH_GROW || br == MMCA_BRANCH_FULL)
+    {
+        const double Tcell = temp_model<AM>(c, sim_time, x, j, k);
+        const double c_int = c.cinit + c.m_inv * (Tcell - c.Tliq);
+        const double A = 1 - c.km * lspfs;
+        const double dce = diffused() - ce_old;
+        const double D2 = c.D_xt * 2;
+        const double dcl = (c_int - conc) * D2 + dce / A;
+        const double u = dcl * A - dce;
+        const double gdfs = (br == MMCA_BRANCH_GROW) ? ge : 0.0;   // FULL: fs' = 1
+        // dfs = u km_inv / cl
+        const double gu = gdfs * c.km_inv / conc;
+        double gq = -gdfs * u * c.km_inv / (conc * conc);
+        const double gkminv = gdfs * u / conc;
+        // u = dcl A - dce ; cl' = cl + dcl
+        const double gdcl = gb + gu * A;
+        const double gA = gu * dcl - gdcl * dce / (A * A);
+        const double gdce = -gu + gdcl / A;
+        // dcl = (c_int - cl) D2 + dce / A
+        gq += gb - gdcl * D2;
+        const double gD2 = gdcl * (c_int - conc);
+        // A = 1 - km fs ; fs' = fs + dfs
+        const double gs = gdfs - gA * c.km;
+        const double gkm = -gA * lspfs - gkminv * c.km_inv * c.km_inv;
+        r.lam = ga + gdce;
+        r.ce = -gdce;           // dce = ce' - ce
+        r.cl = gq;
+        r.fs = gs;
+        r.k = -gkm;             // km = 1 - k
+        r.dl = gD2 * 2 * dv.dDxt;
+    }
+    else
+    {
+        // LIQUID, REMELT: cl' = ce', fs' = 0
+        r.lam = ga + gb;
+    }
+    return r;
+}
+
+// The sums of N values over the workgroup, valid in thread 0; s_red holds
+// N * (BS / 64) doubles.
+template <int BS, int N>
+__device__ __forceinline__ void
+block_sums(double *t, double *s_red)
+{
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+        for (int d = 32; d > 0; d >>= 1)
+            t[n] += __shfl_xor(t[n], d, 64);
+    const int tid = threadIdx.x;
+    if ((tid & 63) == 0)
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            s_red[n * (BS / 64) + (tid >> 6)] = t[n];
+    __syncthreads();
+    if (tid == 0)
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+        {
+            t[n] = 0.0;
+            for (int i = 0; i < BS / 64; ++i)
+                t[n] += s_red[n * (BS / 64) + i];
+        }
+    __syncthreads();
+}
+
+// lam's pull-back through a cell's diffusion stencil, as sums over its
+// neighbours of r (lam_n - lam), of d (lam_n - lam), of f d and of (1 - f) d,
+// with d = cl_n - cl, f = (fs + fs_n) / 2 and r = rs f + rl (1 - f): the
+// factors that do not depend on the neighbour stay outside, 11 FP64 operations
+// a neighbour (22 with each of the four derivatives formed term by term).  r
+// as rl + (rs - rl) f would take one less, but in the solid, where r = rs =
+// rl / 3000, it loses 3 digits (9.6e-15 instead of 1e-15 of error in the
+// derivatives with respect to the diffusivities over 81 steps).
+struct DiffSums {
+    double rl, dl, fd, gd;
+};
+
+__device__ __forceinline__ void
+diff_term(const Consts &c, double lc, double clc, double fsc, double ln, double cln, double fsn, int mo, DiffSums &q)
+{
+    const double f = 0.5 * (fsc + fsn), g = 1.0 - f;
+    const double r = mo ? 0.0 : __builtin_fma(c.rs, f, c.rl * g);
+    const double d = mo ? 0.0 : cln - clc;
+    const double l = ln - lc;
+    q.rl = __builtin_fma(r, l, q.rl);
+    q.dl = __builtin_fma(d, l, q.dl);
+    q.fd = __builtin_fma(f, d, q.fd);
+    q.gd = __builtin_fma(g, d, q.gd);
+}
+
+// The derivatives with respect to cl, fs, rl and rs from the sums.
+struct DiffAdj {
+    double cl, fs, rl, rs;
+};
+
+__device__ __forceinline__ DiffAdj
+diff_adjoint(const Consts &c, double lc, const DiffSums &q)
+{
+    return { q.rl, -0.5 * (c.rs - c.rl) * q.dl, lc * q.gd, lc * q.fd };
+}
+
+// One adjoint step in one pass over the fields.  A workgroup walks a tile of
+// ADJ_TX x TY cells up its planes: at plane kk it forms lam there, for the
+// tile and the ring of cells around it (their lam is formed again by the
+// neighbouring tiles, by waves of their own), and finishes plane kk - 1, whose
+// neighbours' lam are then known.  cl, fs and lam of the planes at hand are in
+// LDS, and the loads of a plane are issued a plane ahead.  lam and the direct
+// derivatives, 7 of the 19 passes over a field that two kernels make, stay out
+// of memory.  The outputs must not overlap the inputs: neighbouring tiles read
+// the inputs again.
+// Partials of (d_liq, d_sol, part_coef) go to part[3 * blk]; the workgroup
+// that finishes last adds their sums, in fixed order, to g_param.
+// 128 x 120 x 104: 51 us against 31 + 33 + 10 of the two passes and their sum;
+// 48 x 41 x 56: 17 against 6 + 6 + 3 and two launches more.  A liquid block
+// stepped again and again, in one pass and in two: 24 x 20 x 22 11.9 and 12.0
+// us, 64^3 16.3 and 16.5, 256^3 283 and 735.  It is bound by
+// memory latency: the rings and the planes at the ends of the walks bring the
+// 121 MB to some 200, and LDS and registers hold one workgroup per CU (tiles
+// of 4, 5, 12 and 13 rows, two workgroups per CU: 49 to 53 us).
+constexpr int ADJ_TX = 64;
+using u32x2 = unsigned __attribute__((ext_vector_type(2)));
+
+// threads of a workgroup: the tile's, and whole waves for the ring and its corners
+constexpr int adj_threads(int ty) { return ADJ_TX * ty + (2 * ADJ_TX + 2 * ty + 4 + 63) / 64 * 64; }
+
+template <bool AM, int TY>
+__global__ void __launch_bounds__(adj_threads(TY))
+k_adj_fused(Consts c, Deriv dv, int kz, const unsigned char *code, double sim_time, const double *ce,
+            const double *cl, const double *fs, const double *g_ce, const double *g_cl, const double *g_fs,
+            double *o_ce, double *o_cl, double *o_fs, double *part, int *done, double *g_param)
+{
+    constexpr int BS = adj_threads(TY);
+    constexpr int CW = ADJ_TX + 4, CN = CW * (TY + 4);    // cl, fs: two cells around the tile
+    constexpr int LW = ADJ_TX + 2, LN = LW * (TY + 2);    // lam: one cell around it
+    constexpr int RING = 2 * ADJ_TX + 2 * TY, OUTER = RING + 4;
+    static_assert(OUTER <= BS - ADJ_TX * TY, "one ring and one outer cell per thread");
+    __shared__ double s_cl[4][CN], s_fs[4][CN], s_lam[2][LN];
+    __shared__ double s_red[3 * (BS / 64)];
+
+    const int tid = threadIdx.x;
+    const int gbx = (c.nx + ADJ_TX - 1) / ADJ_TX, gby = (c.ny + TY - 1) / TY;
+    // workgroups go to the 8 XCDs in turn: neighbouring tiles, which share
+    // their rings, to the same one
+    const int per = gridDim.x / 8;
+    const int w = (int) blockIdx.x < 8 * per ? (blockIdx.x % 8) * per + blockIdx.x / 8 : blockIdx.x;
+    const int x0 = (w % gbx) * ADJ_TX + 1, j0 = ((w / gbx) % gby) * TY + 1, z0 = (w / (gbx * gby)) * kz + 1;
+    const int z1 = min(z0 + kz - 1, c.nz);
+
+    // Cell t of the cells at distance d around the tile, in tile coordinates:
+    // the row below, the row above, the columns left and right.
+    auto around = [&](int t, int d, int &ex, int &ey) {
+        if (t < 2 * ADJ_TX)
+        {
+            ex = t & (ADJ_TX - 1);
+            ey = (t < ADJ_TX) ? -d : TY - 1 + d;
+        }
+        else
+        {
+            t -= 2 * ADJ_TX;
+            ex = (t < TY) ? -d : ADJ_TX - 1 + d;
+            ey = (t < TY) ? t : t - TY;
+        }
+    };
+    // The first ADJ_TX * TY threads have a cell of the tile, the others one of
+    // the ring and load one of the cells around it (cl and fs only).
+    const bool tile = tid < ADJ_TX * TY;
+    const int r = tid - ADJ_TX * TY;
+    int ex = tid & (ADJ_TX - 1), ey = tid / ADJ_TX, ox = 0, oy = 0;
+    if (!tile)
+    {
+        around(min(r, RING - 1), 1, ex, ey);
+        if (r < RING)
+            around(r, 2, ox, oy);
+        else
+        {
+            ox = (r & 1) ? ADJ_TX : -1;                  // the corners of the ring
+            oy = (r & 2) ? TY : -1;
+        }
+    }
+    auto inside = [&](int x, int j, int h) { return x >= 1 - h && x <= c.nx + h && j >= 1 - h && j <= c.ny + h; };
+    const int x = x0 + ex, j = j0 + ey;
+    const bool used = tile || r < RING, outer = !tile && r < OUTER;
+    const bool in = used && inside(x, j, 0);
+    // Byte offsets in a plane, whose address stays in scalar registers.  Every
+    // lane loads at every plane, lanes and planes outside the box from its
+    // edge (no cell inside reads what they get), and stores go through a
+    // buffer descriptor that drops the lanes without a cell: with no branch
+    // around a memory access the compiler knows how many are in flight and
+    // waits for the oldest ones only.
+    const unsigned po = used && inside(x, j, 1) ? 8u * (unsigned) (j * c.sx + x) : 0u;
+    const unsigned pq = outer && inside(x0 + ox, j0 + oy, 1) ? 8u * (unsigned) ((j0 + oy) * c.sx + x0 + ox) : 0u;
+    const unsigned co = in ? 4u * (unsigned) (6 * (j * c.w64 + ((x - 1) >> 6)) + (((x - 1) >> 5) & 1)) : 0u;
+    const unsigned ps = tile && in ? po : ~0u;
+    const int so = (ey + 2) * CW + ex + 2, sq = (oy + 2) * CW + ox + 2, lo = (ey + 1) * LW + ex + 1;
+    const long long cpitch = 24ll * c.w64 * (c.ny + 2);  // bytes of a plane's codes
+    auto ld = [](const double *plane, unsigned off) { return *(const double *) ((const char *) plane + off); };
+    auto st = [&](double *plane, unsigned off, double v) {
+        auto d = __builtin_amdgcn_make_buffer_rsrc(plane, 0, (int) (8u * (unsigned) c.sxy), 0x00027000);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), d, off, 0, 0);
+    };
+    // loads under way: cl and fs of a plane, for the thread's cell and for the
+    // one around the ring; ce, the incoming derivatives and the branch code
+    // (the half word of each bit plane that holds the cell's bit)
+    double cl_n, fs_n, ocl_n, ofs_n, ce_n, gce_n, gcl_n, gfs_n;
+    unsigned w0, w1, w2;
+    auto ld_plane = [&](int k) {
+        const long long p = min(max(k, 0), c.nz + 1) * c.sxy;
+        cl_n = ld(cl + p, po);
+        fs_n = ld(fs + p, po);
+        ocl_n = ld(cl + p, pq);
+        ofs_n = ld(fs + p, pq);
+    };
+    auto ld_cell = [&](int k) {
+        const int kc = min(max(k, 1), c.nz);
+        const long long p = kc * c.sxy;
+        ce_n = ld(ce + p, po);
+        gce_n = ld(g_ce + p, po);
+        gcl_n = ld(g_cl + p, po);
+        gfs_n = ld(g_fs + p, po);
+        const unsigned char *q = code + kc * cpitch;
+        w0 = *(const unsigned *) (q + co);
+        w1 = *(const unsigned *) (q + (co + 8u));
+        w2 = *(const unsigned *) (q + (co + 16u));
+    };
+    auto put_plane = [&](int k) {
+        if (used)
+        {
+            s_cl[k & 3][so] = cl_n;
+            s_fs[k & 3][so] = fs_n;
+        }
+        if (outer)
+        {
+            s_cl[k & 3][sq] = ocl_n;
+            s_fs[k & 3][sq] = ofs_n;
+        }
+    };
+    const int mx1 = (x == c.nx) ? c.pad_hi[0] : 0, mx0 = (x == 1) ? c.pad_lo[0] : 0;
+    const int my1 = (j == c.ny) ? c.pad_hi[1] : 0, my0 = (j == 1) ? c.pad_lo[1] : 0;
+
+    double lam2 = 0.0, lam1 = 0.0;                       // own lam of kk-2 and kk-1
+    double dce = 0.0, dcl = 0.0, dfs = 0.0;              // direct derivatives of kk-1
+    double p_dl = 0.0, p_ds = 0.0, p_k = 0.0;
+    ld_plane(z0 - 2);
+    put_plane(z0 - 2);
+    ld_plane(z0 - 1);
+    put_plane(z0 - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    ld_plane(z0);
+    __builtin_amdgcn_sched_barrier(0);
+    ld_cell(z0 - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // as many stores in flight behind the loads as in every later turn (no
+    // lane takes part), for the count that the loop waits for
+    st(o_ce + c.sxy, ~0u, 0.0);
+    st(o_cl + c.sxy, ~0u, 0.0);
+    st(o_fs + c.sxy, ~0u, 0.0);
+    for (int kk = z0 - 1; kk <= z1 + 1; ++kk)
+    {
+        put_plane(kk + 1);                               // over plane kk - 3
+        __builtin_amdgcn_sched_barrier(0);
+        ld_plane(kk + 2);
+        __syncthreads();
+
+        // of planes kk - 2 and kk + 1 only the thread's own words are read
+        const double *C = s_cl[kk & 3] + so, *F = s_fs[kk & 3] + so;
+        const double *Cu = s_cl[(kk + 1) & 3] + so, *Fu = s_fs[(kk + 1) & 3] + so;
+        const double *Cd = s_cl[(kk + 3) & 3] + so, *Fd = s_fs[(kk + 3) & 3] + so;
+        double lam0 = 0.0, ece = 0.0, ecl = 0.0, efs = 0.0;
+        const bool here = kk >= z0 && kk <= z1;
+        if (in && (here || (tile && kk >= 1 && kk <= c.nz)))
+        {
+            auto diffused = [&]() {
+                const int mo[6] = { mx1, mx0, my1, my0, (kk == c.nz) ? c.pad_hi[2] : 0, (kk == 1) ? c.pad_lo[2] : 0 };
+                const double cn[6] = { C[1], C[-1], C[CW], C[-CW], Cu[0], Cd[0] };
+                const double fn[6] = { F[1], F[-1], F[CW], F[-CW], Fu[0], Fd[0] };
+                return diffuse_cell(c, ce_n, C[0], F[0], cn, fn, mo);
+            };
+            const int bit = (x - 1) & 31;
+            const int br = (int) ((w0 >> bit) & 1u) | (int) (((w1 >> bit) & 1u) << 1) | (int) (((w2 >> bit) & 1u) << 2);
+            const BranchAdj d = branch_adjoint<AM>(c, dv, br, sim_time, x, j, kk, ce_n, C[0], F[0], diffused,
+                                                   here && tile, gce_n, gcl_n, gfs_n);
+            lam0 = d.lam;
+            ece = d.ce;
+            ecl = d.cl;
+            efs = d.fs;
+            if (here && tile)
+            {
+                p_dl += d.dl;
+                p_k += d.k;
+            }
+        }
+        if (used)
+            s_lam[kk & 1][lo] = lam0;
+        __builtin_amdgcn_sched_barrier(0);
+        ld_cell(kk + 1);
+        __builtin_amdgcn_sched_barrier(0);
+
+        const int m = kk - 1;
+        double vce = 0.0, vcl = 0.0, vfs = 0.0;
+        if (m >= z0 && tile && in)
+        {
+            const double *L = s_lam[m & 1] + lo;
+            const double clc = Cd[0], fsc = Fd[0];
+            DiffSums u = { 0.0, 0.0, 0.0, 0.0 };
+            diff_term(c, lam1, clc, fsc, L[1], Cd[1], Fd[1], mx1, u);
+            diff_term(c, lam1, clc, fsc, L[-1], Cd[-1], Fd[-1], mx0, u);
+            diff_term(c, lam1, clc, fsc, L[LW], Cd[CW], Fd[CW], my1, u);
+            diff_term(c, lam1, clc, fsc, L[-LW], Cd[-CW], Fd[-CW], my0, u);
+            diff_term(c, lam1, clc, fsc, lam0, C[0], F[0], (m == c.nz) ? c.pad_hi[2] : 0, u);
+            diff_term(c, lam1, clc, fsc, lam2, s_cl[(kk + 2) & 3][so], s_fs[(kk + 2) & 3][so], (m == 1) ? c.pad_lo[2] : 0, u);
+            const DiffAdj q = diff_adjoint(c, lam1, u);
+            vce = dce + lam1;
+            vcl = dcl + q.cl;
+            vfs = dfs + q.fs;
+            p_dl += q.rl * dv.dtx;
+            p_ds += q.rs * dv.dtx;
+        }
+        const long long p = max(m, 1) * c.sxy;
+        const unsigned off = m >= z0 ? ps : ~0u;
+        st(o_ce + p, off, vce);
+        st(o_cl + p, off, vcl);
+        st(o_fs + p, off, vfs);
+
+        lam2 = lam1, lam1 = lam0;
+        dce = ece, dcl = ecl, dfs = efs;
+    }
+
+    double t[3] = { p_dl, p_ds, p_k };
+    block_sums<BS, 3>(t, s_red);
+    if (tid == 0)
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+            st_agent(&part[3 * (long long) blockIdx.x + n], t[n]);
+    const int nblk = gridDim.x;
+    if (!last_workgroup(done, nblk))
+        return;
+    t[0] = t[1] = t[2] = 0.0;
+    for (int i = tid; i < nblk; i += BS)
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+            t[n] += ld_agent(&part[3 * (long long) i + n]);
+    block_sums<BS, 3>(t, s_red);
+    if (tid == 0)
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+            g_param[n] += t[n];
+}
+
+// The same step in place, in two passes: the outputs may be the incoming
+// derivatives, which only the cell itself reads in each pass.
+// First the branch: lam, and the direct derivatives; partials of (d_liq,
+// part_coef) per workgroup into part[2 * blk].
 template <bool AM>
 __global__ void __launch_bounds__(ADJ_BS)
 k_adj_part(Consts c, Deriv dv, const unsigned char *code, double sim_time, const double *ce,
@@ -185,68 +560,29 @@ k_adj_part(Consts c, Deriv dv, const unsigned char *code, double sim_time, const
     double p_dl = 0.0, p_k = 0.0;
     if (q.active)
     {
-        long long nb[6];
-        int mo[6];
-        stencil(c, q, nb, mo);
-        double cln[6], fsn[6];
-#pragma unroll
-        for (int n = 0; n < 6; ++n)
-        {
-            cln[n] = cl[nb[n]];
-            fsn[n] = fs[nb[n]];
-        }
         const double ce_old = ce[q.idx], conc = cl[q.idx], lspfs = fs[q.idx];
-        const double ce_new = diffuse_cell(c, ce_old, conc, lspfs, cln, fsn, mo);
-        const double ga = g_ce[q.idx], gb = g_cl[q.idx], ge = g_fs[q.idx];
+        auto diffused = [&]() {
+            long long nb[6];
+            int mo[6];
+            stencil(c, q, nb, mo);
+            double cln[6], fsn[6];
+#pragma unroll
+            for (int n = 0; n < 6; ++n)
+            {
+                cln[n] = cl[nb[n]];
+                fsn[n] = fs[nb[n]];
+            }
+            return diffuse_cell(c, ce_old, conc, lspfs, cln, fsn, mo);
+        };
         const int br = rec_code(c, code, q.x, q.j, q.k);
-        double lamv, gce_d = 0.0, gcl_d = 0.0, gfs_d = 0.0;
-        if (br == MMCA_BRANCH_SOLID)
-        {
-            // cl' = ce' k_inv, fs' = fs
-            lamv = ga + gb * c.k_inv;
-            gfs_d = ge;
-            p_k = -gb * ce_new * c.k_inv * c.k_inv;
-        }
-        else if (br == MMCA_BRANCH_GROW || br == MMCA_BRANCH_FULL)
-        {
-            const double Tcell = temp_model<AM>(c, sim_time, q.x, q.j, q.k);
-            const double c_int = c.cinit + c.m_inv * (Tcell - c.Tliq);
-            const double A = 1 - c.km * lspfs;
-            const double dce = ce_new - ce_old;
-            const double D2 = c.D_xt * 2;
-            const double dcl = (c_int - conc) * D2 + dce / A;
-            const double u = dcl * A - dce;
-            const double gdfs = (br == MMCA_BRANCH_GROW) ? ge : 0.0;   // FULL: fs' = 1
-            // dfs = u km_inv / cl
-            const double gu = gdfs * c.km_inv / conc;
-            double gq = -gdfs * u * c.km_inv / (conc * conc);
-            const double gkminv = gdfs * u / conc;
-            // u = dcl A - dce ; cl' = cl + dcl
-            const double gdcl = gb + gu * A;
-            const double gA = gu * dcl - gdcl * dce / (A * A);
-            const double gdce = -gu + gdcl / A;
-            // dcl = (c_int - cl) D2 + dce / A
-            gq += gb - gdcl * D2;
-            const double gD2 = gdcl * (c_int - conc);
-            // A = 1 - km fs ; fs' = fs + dfs
-            const double gs = gdfs - gA * c.km;
-            const double gkm = -gA * lspfs - gkminv * c.km_inv * c.km_inv;
-            lamv = ga + gdce;
-            gce_d = -gdce;          // dce = ce' - ce
-            gcl_d = gq;
-            gfs_d = gs;
-            p_k = -gkm;             // km = 1 - k
-            p_dl = gD2 * 2 * dv.dDxt;
-        }
-        else
-        {
-            // LIQUID, REMELT: cl' = ce', fs' = 0
-            lamv = ga + gb;
-        }
-        lam[q.idx] = lamv;
-        gce_in[q.idx] = gce_d;
-        gcl_in[q.idx] = gcl_d;
-        gfs_in[q.idx] = gfs_d;
+        const BranchAdj r = branch_adjoint<AM>(c, dv, br, sim_time, q.x, q.j, q.k, ce_old, conc, lspfs, diffused, true,
+                                               g_ce[q.idx], g_cl[q.idx], g_fs[q.idx]);
+        lam[q.idx] = r.lam;
+        gce_in[q.idx] = r.ce;
+        gcl_in[q.idx] = r.cl;
+        gfs_in[q.idx] = r.fs;
+        p_dl = r.dl;
+        p_k = r.k;
     }
     const double s_dl = block_sum<ADJ_BS>(p_dl, s_red);
     __syncthreads();
@@ -258,9 +594,9 @@ k_adj_part(Consts c, Deriv dv, const unsigned char *code, double sim_time, const
     }
 }
 
-// Adjoint of the diffusion stencil: adds lam's pull-back to (ce, cl, fs) and
-// the (d_liq, d_sol) partials per workgroup into part[2 * blk].  lam is zero
-// on the halo (halo cells are never updated).
+// Then the stencil: adds lam's pull-back to (ce, cl, fs); partials of (d_liq,
+// d_sol) per workgroup into part[2 * blk].  lam is zero on the halo (halo
+// cells are never updated).
 __global__ void __launch_bounds__(ADJ_BS)
 k_adj_diff(Consts c, Deriv dv, const double *cl, const double *fs, const double *lam, double *gce_in,
            double *gcl_in, double *gfs_in, double *part)
@@ -273,27 +609,26 @@ k_adj_diff(Consts c, Deriv dv, const double *cl, const double *fs, const double 
         long long nb[6];
         int mo[6];
         stencil(c, q, nb, mo);
-        const double lc = lam[q.idx], clc = cl[q.idx], fsc = fs[q.idx];
-        const double hd = 0.5 * (c.rs - c.rl);
-        double gcl = 0.0, gfs = 0.0, grs = 0.0, grl = 0.0;
+        double ln[6], cln[6], fsn[6];
 #pragma unroll
         for (int n = 0; n < 6; ++n)
         {
-            const double ln = lam[nb[n]];
-            const double f = 0.5 * (fsc + fs[nb[n]]);
-            const double w = 1 - mo[n];
-            const double r = (c.rs * f + c.rl * (1 - f)) * w;
-            const double d = cl[nb[n]] - clc;
-            gcl += r * (ln - lc);
-            gfs += hd * w * d * (lc - ln);
-            grs += lc * f * w * d;
-            grl += lc * (1 - f) * w * d;
+            ln[n] = lam[nb[n]];
+            cln[n] = cl[nb[n]];
+            fsn[n] = fs[nb[n]];
         }
+        const double lc = lam[q.idx];
+        const double clc = cl[q.idx], fsc = fs[q.idx];
+        DiffSums u = { 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+        for (int n = 0; n < 6; ++n)
+            diff_term(c, lc, clc, fsc, ln[n], cln[n], fsn[n], mo[n], u);
+        const DiffAdj r = diff_adjoint(c, lc, u);
         gce_in[q.idx] += lc;
-        gcl_in[q.idx] += gcl;
-        gfs_in[q.idx] += gfs;
-        p_dl = grl * dv.dtx;
-        p_ds = grs * dv.dtx;
+        gcl_in[q.idx] += r.cl;
+        gfs_in[q.idx] += r.fs;
+        p_dl = r.rl * dv.dtx;
+        p_ds = r.rs * dv.dtx;
     }
     const double s_dl = block_sum<ADJ_BS>(p_dl, s_red);
     __syncthreads();
@@ -350,6 +685,54 @@ k_zero_halo(Consts c, double *lam)
         lam[i] = 0.0;
 }
 
+constexpr int ADJ_TY = 8;
+
+long long adj_tiles(const Consts &c)
+{
+    return (long long) ((c.nx + ADJ_TX - 1) / ADJ_TX) * ((c.ny + ADJ_TY - 1) / ADJ_TY);
+}
+
+// Planes that a workgroup of k_adj_fused walks.  One workgroup fits a CU, and
+// a walk takes two planes more than it finishes: the fewest rounds of the
+// chip's 256 CUs times the planes of a walk.  128 x 120 x 104 (30 tiles): 13
+// planes (240 workgroups) 50 us, 7 (450) 59, 15 (210) 55, 4 (780) 68.
+int adj_planes(const Consts &c)
+{
+    const long long t = adj_tiles(c);
+    int best = 1;
+    long long cost = -1;
+    for (int kz = 1; kz <= std::min(64, c.nz); ++kz)
+    {
+        const long long rounds = (t * ((c.nz + kz - 1) / kz) + 255) / 256;
+        if (cost < 0 || rounds * (kz + 2) < cost)
+        {
+            best = kz;
+            cost = rounds * (kz + 2);
+        }
+    }
+    return best;
+}
+
+// True when none of the outputs overlaps an input or another output.
+bool adj_separate(const Consts &c, std::initializer_list<const double *> out, std::initializer_list<const double *> in)
+{
+    const uintptr_t n = (uintptr_t) c.P * sizeof(double);
+    auto apart = [&](const double *a, const double *b) {
+        const uintptr_t p = (uintptr_t) a, q = (uintptr_t) b;
+        return p + n <= q || q + n <= p;
+    };
+    for (auto o = out.begin(); o != out.end(); ++o)
+    {
+        for (const double *i : in)
+            if (!apart(*o, i))
+                return false;
+        for (auto p = o + 1; p != out.end(); ++p)
+            if (!apart(*o, *p))
+                return false;
+    }
+    return true;
+}
+
 // The launches of one adjoint step; lam holds P doubles, pa and pb 2 * nblk each.
 hipError_t
 adjoint_launch(const Consts &c, const Deriv &dv, uint64_t timestep, const uint8_t *codes, const double *ce,
@@ -359,6 +742,23 @@ adjoint_launch(const Consts &c, const Deriv &dv, uint64_t timestep, const uint8_
 {
     const long long nblk = adj_blocks(c);
     const double sim_time = timestep * c.dt;
+    // one pass where no output is an input, and a plane's byte offsets fit 31 bits
+    if (c.sxy <= (1ll << 28) - 1 && adj_separate(c, { g_ce_in, g_cl_in, g_fs_in }, { ce, cl, fs, g_ce, g_cl, g_fs }))
+    {
+        const int kz = adj_planes(c);
+        const dim3 fgrid((unsigned) (adj_tiles(c) * ((c.nz + kz - 1) / kz)));
+        // the first cell of lam is a halo cell, 0 between the calls
+        int *done = (int *) lam;
+        if (c.am)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_fused<true, ADJ_TY>), fgrid, dim3(adj_threads(ADJ_TY)), 0, s, c, dv, kz,
+                               codes, sim_time, ce, cl, fs, g_ce, g_cl, g_fs, g_ce_in, g_cl_in, g_fs_in, pa, done,
+                               g_param);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_fused<false, ADJ_TY>), fgrid, dim3(adj_threads(ADJ_TY)), 0, s, c, dv, kz,
+                               codes, sim_time, ce, cl, fs, g_ce, g_cl, g_fs, g_ce_in, g_cl_in, g_fs_in, pa, done,
+                               g_param);
+        return hipGetLastError();
+    }
     const dim3 grid((unsigned) nblk), blk(ADJ_BX, ADJ_BY);
     if (c.am)
         hipLaunchKernelGGL(k_adj_part<true>, grid, blk, 0, s, c, dv, codes, sim_time, ce, cl, fs, g_ce, g_cl, g_fs,

@@ -158,45 +158,6 @@ block_exscan_int(int v, int *total, int *s_w)
     return off + incl - v;
 }
 
-// Values handed from the workgroups of a launch to the one that finishes last
-// (last_workgroup): stores and loads at agent scope go past the L2s, of which
-// every XCD has its own.
-template <typename T>
-__device__ __forceinline__ void
-st_agent(T *p, T v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <typename T>
-__device__ __forceinline__ T
-ld_agent(const T *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// True in the workgroup, of n, that gets here last; all of its threads call it.
-// Every thread first waits until its st_agent stores have arrived, so that the
-// last workgroup's ld_agent loads see all of them; a __threadfence() instead
-// would write back and invalidate the whole L2 in every workgroup (it took
-// k_list_count of a 256 x 256 x 512 block from 7 to 150 us).  *done is 0
-// before and after.
-__device__ __forceinline__ bool
-last_workgroup(int *done, int n)
-{
-    __shared__ int s_last;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        s_last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
-        if (s_last)
-            *done = 0;
-    }
-    __syncthreads();
-    return s_last != 0;
-}
-
 // Domain of workgroup w: the last d with off[d] <= w (domains without work
 // share their offset with the next domain).
 __device__ __forceinline__ int
