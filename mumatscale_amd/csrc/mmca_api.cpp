@@ -25,6 +25,9 @@ hipError_t launch_beam_field(const DevBufs &b, const Consts &c, const BeamSet &p
                              hipStream_t s);
 hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStream_t s);
 hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s);
+long long tile_slots(const Consts &c);
+hipError_t launch_wake_all(const View &v, hipStream_t s);
+hipError_t launch_settle(const DevBufs &b, const Consts &c, int cur, unsigned failed, hipStream_t s);
 hipError_t launch_list(const View &v, int cb, int capture, int decide_realloc, hipStream_t s);
 hipError_t launch_nucleate_coupled(const View &v, int cur, hipStream_t s);
 hipError_t launch_halo_exchange(const View &v, int phase, int cb, long long max_face, hipStream_t s);
@@ -426,11 +429,36 @@ int read_ledger(mmca_ctx *ctx, double *out)
     return MMCA_OK;
 }
 
+// Whether the steps of a call are lean (View::lean).  The call then starts
+// with one more launch (5 us), which clears what is known of the cells, so a
+// call of a few steps does without.  FP32 storage and beams do without too:
+// the solute kernel is not bound by what it writes there, and testing for it
+// takes longer than it saves (FP32 205 x 251 x 303, 45 % of the words liquid:
+// 177 us a step against 173; FP32 beam 500 x 256 x 128: 187 against 170).
+// Nor do blocks whose fields (56 bytes a cell) the 256 MB of last-level cache
+// hold: 40 x 36 x 44 8.49 ms a pass against 8.27, 8 x 64 x 60 x 96 35.0 against
+// 34.6; above, 150 x 140 x 165 22.7 against 24.2, 256 x 256 x 512 147 against 160.
+constexpr int LEAN_STEPS = 8;
+constexpr long long LEAN_CELLS = 3ll << 20;
+
+bool lean_call(mmca_ctx *const *ctxs, size_t n, int nsteps, bool tiles)
+{
+    long long cells = 0;
+    for (size_t d = 0; d < n; d++)
+        cells += (long long) ctxs[d]->c.nx * ctxs[d]->c.ny * ctxs[d]->c.nz;
+    const Consts &c = ctxs[0]->c;
+    return nsteps >= LEAN_STEPS && tiles && !c.f32 && !c.am && cells >= LEAN_CELLS;
+}
+
+// View::lean of step n (from 0) of a call
+int lean_mode(bool lean, int n, int nsteps) { return !lean ? 0 : n == 0 ? 3 : n + 1 < nsteps ? 1 : 2; }
+
 // one doiteration() on the device (calculate.c:193-352)
-int enqueue_iteration(mmca_ctx *ctx, bool advance)
+int enqueue_iteration(mmca_ctx *ctx, bool advance, int lean)
 {
     const int nxt = ctx->cur ^ 1;
     TRY(ensure_view(ctx));
+    ctx->view.lean = lean;
     TRY(refresh_beam(ctx, advance ? 1 : 0, ctx->stream));
     HIPCHK(launch_nucleate(ctx->view, advance ? 7 : 3, ctx->cur, ctx->stream));
     const size_t ev0 = ctx->ev_used;
@@ -452,6 +480,7 @@ int enqueue_iteration(mmca_ctx *ctx, bool advance)
         ctx->ev_used = ev0 + 2;
     }
     HIPCHK(launch_list(ctx->view, nxt, 1, 1, ctx->stream));
+    ctx->view.lean = 0;
     ctx->cur = nxt;
     return MMCA_OK;
 }
@@ -634,7 +663,7 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
         TRY(dev_alloc(&b.ce32, P));
         TRY(dev_alloc(&b.cl32[0], P));
         TRY(dev_alloc(&b.cl32[1], P));
-        b.nledger = (long long) ((c.nx + 63) / 64) * ((c.ny + 3) / 4) * c.nz;
+        b.nledger = tile_slots(c);
         TRY(dev_alloc(&b.ledger, (size_t) (2 * b.nledger)));
     } else {
         TRY(dev_alloc(&b.ce, P));
@@ -647,6 +676,9 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
     TRY(dev_alloc(&b.dc, 3 * P));
     const size_t mask_words = (size_t) (c.ny + 2) * (c.nz + 2) * c.w64;
     TRY(dev_alloc(&b.mask, mask_words));
+    for (int i = 0; i < 2; i++)
+        TRY(dev_alloc(&b.act[i], mask_words));
+    TRY(dev_alloc(&b.stamp, (size_t) tile_slots(c)));
     const size_t xhalo_bytes = (size_t) 2 * (c.ny + 2) * (c.nz + 2);
     TRY(dev_alloc(&b.xhalo, xhalo_bytes));
     TRY(dev_alloc(&b.diff_id, N + 2));
@@ -725,7 +757,7 @@ int mmca_destroy(mmca_ctx *ctx)
     if (ctx->shares_grains)
         b.g_rot = nullptr, b.g_cell = nullptr, b.g_step = nullptr, b.g_src = nullptr, b.g_dom = nullptr;
     void *ptrs[] = { b.ce, b.cl[0], b.cl[1], b.ce32, b.cl32[0], b.cl32[1], b.ledger, b.fs[0], b.fs[1], b.gr, b.dc, b.mask,
-                     b.xhalo,
+                     b.act[0], b.act[1], b.stamp, b.xhalo,
                      b.diff_id, b.nbr, b.dtx, b.dty, b.dtz, b.blk_count, b.row_first, b.list_done, b.nuc_done, b.site_idx, b.site_thr, b.site_fixed,
                      b.site_ls, b.events, b.ev_blk, b.ev_cnt, b.g_rot, b.g_cell, b.g_step, b.g_src, b.g_dom, b.fixed_rot,
                      b.rand_rot,
@@ -831,6 +863,11 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
         const long long ns = ctx->b.nsites, ch = chunk_steps(ctx);
         long long used = ctx->hc.random_used, flight[2] = { 0, 0 };
         int done = 0, first = 0, nflight = 0;
+        const bool lean = lean_call(&ctx, 1, nsteps, !ctx->b.rec && zm_rows(ctx->c) > 0);
+        if (lean) {
+            TRY(ensure_view(ctx));
+            HIPCHK(launch_wake_all(ctx->view, ctx->stream));
+        }
         while (done < nsteps && ctx->hc.status == MMCA_OK) {
             long long k = nsteps - done;
             if (ns > 0 && ctx->rand_filled < ctx->rand_capacity) {
@@ -855,7 +892,7 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
             if (k < 1)
                 return MMCA_ERR_STATE;
             for (long long n = 0; n < k; n++)
-                TRY(enqueue_iteration(ctx, true));
+                TRY(enqueue_iteration(ctx, true, lean_mode(lean, done + (int) n, nsteps)));
             done += (int) k;
             if (done < nsteps) {
                 const int slot = (first + nflight) & 1;
@@ -871,8 +908,13 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
         TRY(sync_counters(ctx));
         // stopped on an error: the buffers of the failed step stay current
         // (the steps issued after it skipped every kernel)
-        if (ctx->hc.status != MMCA_OK)
+        if (ctx->hc.status != MMCA_OK) {
             ctx->cur = cur0 ^ (int) ((ctx->hc.timestep - t0) & 1);
+            if (lean && ctx->hc.failed_step > t0 + 1) {
+                HIPCHK(launch_settle(ctx->b, ctx->c, ctx->cur, (unsigned) ctx->hc.failed_step, ctx->stream));
+                HIPCHK(hipStreamSynchronize(ctx->stream));
+            }
+        }
         if (ctx->timing)
             TRY(collect_timing(ctx));
     }
@@ -1051,7 +1093,7 @@ int mmca_doiteration(mmca_ctx *ctx)
         return st;
     TRY(replan_random(ctx));
     TRY(ensure_random(ctx, (long long) ctx->hc.random_used + ctx->b.nsites));
-    TRY(enqueue_iteration(ctx, false));
+    TRY(enqueue_iteration(ctx, false, 0));
     TRY(check_status(ctx));
     if (ctx->timing)
         TRY(collect_timing(ctx));
@@ -1840,7 +1882,7 @@ struct mmca_batch {
     double time_ms = 0.0;
     long long time_n = 0;
     bool use_graph = false;
-    hipGraphExec_t graph[2] = { nullptr, nullptr };
+    hipGraphExec_t graph[6] = {};    // pairs of steps: buffer + 2 * (not lean, lean, the call's last lean ones)
     // the domains are the subblocks of one global domain (mmca_batch_couple)
     bool coupled = false;
     long long max_face = 0;      // largest face (cells) or halo-row word count
@@ -1864,7 +1906,7 @@ int batch_view(mmca_batch *bt)
     }
     TRY(build_view(bt->dom.data(), (int) bt->dom.size(), bt->xcd_remap, bt->zm_planes > 0 ? bt->zm_by : 0,
                    &bt->d_desc, &bt->d_off, &bt->cap, &bt->view, bt->stream));
-    for (int p = 0; p < 2; p++)
+    for (int p = 0; p < 6; p++)
         if (bt->graph[p]) {
             (void) hipGraphExecDestroy(bt->graph[p]);
             bt->graph[p] = nullptr;
@@ -1899,8 +1941,9 @@ long long batch_chunk_steps(const mmca_batch *bt)
 
 // one doiteration() of every domain: seven launches whatever the batch size
 // (ten for a coupled batch: two halo exchanges and the cross-rank activation)
-int batch_enqueue(mmca_batch *bt, int cur)
+int batch_enqueue(mmca_batch *bt, int cur, int lean)
 {
+    bt->view.lean = lean;
     const Consts &c0 = bt->dom[0]->c;
     const int nxt = cur ^ 1;
     for (mmca_ctx *c : bt->dom)
@@ -1932,23 +1975,25 @@ int batch_enqueue(mmca_batch *bt, int cur)
     return MMCA_OK;
 }
 
-// a pair of steps starting from buffer `cur`, captured once into a graph
-int batch_graph_pair(mmca_batch *bt, int cur)
+// a pair of steps starting from buffer `cur`, captured once into a graph;
+// `lean` of the two are 0 0, 1 1 or 1 2
+int batch_graph_pair(mmca_batch *bt, int cur, int lean)
 {
-    if (!bt->graph[cur]) {
+    hipGraphExec_t &graph = bt->graph[cur + 2 * lean];
+    if (!graph) {
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(bt->stream, hipStreamCaptureModeThreadLocal));
-        int st = batch_enqueue(bt, cur);
+        int st = batch_enqueue(bt, cur, lean ? 1 : 0);
         if (st == MMCA_OK)
-            st = batch_enqueue(bt, cur ^ 1);
+            st = batch_enqueue(bt, cur ^ 1, lean);
         hipError_t e = hipStreamEndCapture(bt->stream, &g);
         if (st != MMCA_OK)
             return st;
         HIPCHK(e);
-        HIPCHK(hipGraphInstantiate(&bt->graph[cur], g, nullptr, nullptr, 0));
+        HIPCHK(hipGraphInstantiate(&graph, g, nullptr, nullptr, 0));
         (void) hipGraphDestroy(g);
     }
-    HIPCHK(hipGraphLaunch(bt->graph[cur], bt->stream));
+    HIPCHK(hipGraphLaunch(graph, bt->stream));
     return MMCA_OK;
 }
 
@@ -2142,7 +2187,7 @@ int mmca_batch_destroy(mmca_batch *bt)
     (void) hipSetDevice(bt->device);
     if (bt->stream)
         (void) hipStreamSynchronize(bt->stream);
-    for (int p = 0; p < 2; p++)
+    for (int p = 0; p < 6; p++)
         if (bt->graph[p])
             (void) hipGraphExecDestroy(bt->graph[p]);
     for (auto e : bt->ev)
@@ -2275,6 +2320,9 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
     for (size_t d = 0; d < bt->dom.size(); d++)
         start[d] = { bt->dom[d]->cur, bt->dom[d]->hc.timestep };
     const long long ch = batch_chunk_steps(bt);
+    const bool lean = lean_call(bt->dom.data(), bt->dom.size(), nsteps, bt->zm_planes > 0);
+    if (lean)
+        HIPCHK(launch_wake_all(bt->view, bt->stream));
     int done = 0;
     while (done < nsteps) {
         // chunk bound: drawn orientations cover every grain the chunk can create
@@ -2294,11 +2342,18 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
         if (k < 1)
             return MMCA_ERR_STATE;
         long long n = 0;
-        if (bt->use_graph && !bt->timing)
+        if (bt->use_graph && !bt->timing) {
+            if (lean && done == 0) {                 // the first step is like no other
+                TRY(batch_enqueue(bt, bt->cur, lean_mode(lean, 0, nsteps)));
+                bt->cur ^= 1;
+                n = 1;
+            }
             for (; n + 2 <= k; n += 2)
-                TRY(batch_graph_pair(bt, bt->cur));   // two steps: cur returns to itself
+                TRY(batch_graph_pair(bt, bt->cur,    // two steps: cur returns to itself
+                                     lean_mode(lean, done + (int) n + 1, nsteps)));
+        }
         for (; n < k; n++) {
-            TRY(batch_enqueue(bt, bt->cur));
+            TRY(batch_enqueue(bt, bt->cur, lean_mode(lean, done + (int) n, nsteps)));
             bt->cur ^= 1;
         }
         done += (int) k;
@@ -2309,6 +2364,8 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
     for (size_t d = 0; d < bt->dom.size(); d++) {
         mmca_ctx *c = bt->dom[d];
         c->cur = c->hc.status == MMCA_OK ? bt->cur : start[d].first ^ (int) ((c->hc.timestep - start[d].second) & 1);
+        if (lean && c->hc.status != MMCA_OK && c->hc.failed_step > start[d].second + 1)
+            HIPCHK(launch_settle(c->b, c->c, c->cur, (unsigned) c->hc.failed_step, bt->stream));
         if (want_sums)
             HIPCHK(launch_reduce(c->b, c->c, c->cur, bt->d_sums + 2 * d, bt->stream));
     }

@@ -87,6 +87,11 @@ struct DevBufs {
     int *gr;
     double *dc;                      // decentered octahedron centres, x,y,z per cell (decentered_t)
     unsigned long long *mask;        // 1 bit per padded cell: gr > 0
+    // lean steps (View::lean): per buffer and mask word, the cells with gr > 0
+    // when the buffer was written (the others have fs = 0 there); and, per
+    // solute tile, the timestep it was last finished at
+    unsigned long long *act[2];
+    unsigned *stamp;
     unsigned char *xhalo;            // per padded row: gr > 0 of its x = 0 and x = nx+1 halo cells (2 bytes)
     // interface list and dc_tmp emulation
     int *diff_id;                    // slots 1..gindex
@@ -160,6 +165,12 @@ struct View {
     int ndom;
     int xcd_run;                 // solute tiles in a run on one XCD (xcd_tile)
     int zm_planes_max;           // largest zm_planes of the domains (LDS of the per-plane temperatures)
+    // Place of a step in its call: 0: ce, fs and the mask of every cell are
+    // written.  Lean steps leave out what stays as it is: fs and the mask of
+    // words without a solid cell now or when the buffer was last written, and
+    // (1: not the first step, 3, nor the last, 2) ce of words without a solid
+    // cell, which equals cl; a liquid cell's ce is read as its cl (1 and 2).
+    int lean;
     const long long *off_nuc;    // k_nuc_detect workgroups
     const long long *off_zm;     // z-marching solute tiles
     const long long *off_cell;   // cell-parallel solute workgroups

@@ -179,6 +179,14 @@ find_dom(const long long *off, int ndom, long long w)
 // ---------------------------------------------------------------------------
 constexpr int NUC_BS = 256;
 
+// A cell that becomes solid between lean steps: from the next step on its ce
+// is read, which for a liquid cell equals cl and need not have been written.
+__device__ __forceinline__ void
+put_ce_of_liquid(const DevBufs &b, int buf, long long idx)
+{
+    G(b.ce)[idx] = cl_buf(b, buf)[idx];
+}
+
 // Event ordering and activateNewGrains/createGrains on one rank
 // (grain.c:841-916, 348-425), one workgroup.
 // mode: 1 = order the detected events, 2 = activate, 4 = advance the timestep
@@ -186,7 +194,7 @@ constexpr int NUC_BS = 256;
 // nev1 >= 0: the number of events of a domain with one detecting workgroup,
 // already in order in `events`.
 __device__ __forceinline__ void
-nuc_activate(const DevBufs &b, const Consts &c, int mode, int nev1)
+nuc_activate(const DevBufs &b, const Consts &c, int mode, int nev1, int lean, int cur)
 {
     __shared__ int s_w[NUC_BS / 64];
     __shared__ int s_nev;
@@ -247,6 +255,8 @@ nuc_activate(const DevBufs &b, const Consts &c, int mode, int nev1)
                 if (id <= maxg)
                 {
                     int idx = G(b.site_idx)[s];
+                    if (lean == 1 || lean == 2)
+                        put_ce_of_liquid(b, cur, idx);
                     G(b.gr)[idx] = (int) id;
                     const double *rot;
                     int src;
@@ -305,7 +315,7 @@ k_nuc_activate(View V, int mode)
     const Consts c = V.dom[blockIdx.x].c;
     if (b.cnt->status != MMCA_OK)
         return;
-    nuc_activate(b, c, mode, -1);
+    nuc_activate(b, c, mode, -1, 0, 0);
 }
 
 // cell_nucleation (grain.c:1222-1318): one thread per site, sites sorted by
@@ -390,7 +400,7 @@ k_nuc_detect(View V, int mode, int cur)
         // nothing to wait for or to order
         if (flag)
             G(b.events)[r] = s;
-        nuc_activate(b, c, mode, tot);
+        nuc_activate(b, c, mode, tot, V.lean, cur);
         return;
     }
     if (flag)
@@ -398,7 +408,7 @@ k_nuc_detect(View V, int mode, int cur)
     if (threadIdx.x == 0)
         st_agent(&b.ev_cnt[blk], tot);
     if (last_workgroup(b.nuc_done, nwg))
-        nuc_activate(b, c, mode, -1);
+        nuc_activate(b, c, mode, -1, V.lean, cur);
 }
 
 
@@ -410,7 +420,7 @@ k_nuc_detect(View V, int mode, int cur)
 // share.  Every domain advances its timestep; running past MaxTotGrains
 // stops all of them, as createGrains' error() stops every rank.
 __global__ void __launch_bounds__(NUC_BS)
-k_nuc_activate_coupled(View V)
+k_nuc_activate_coupled(View V, int cur)
 {
     __shared__ int s_w[NUC_BS / 64];
     const int tid = threadIdx.x;
@@ -445,6 +455,8 @@ k_nuc_activate_coupled(View V)
             {
                 const long long id = (long long) next + e;
                 int idx = G(b.site_idx)[s];
+                if (V.lean == 1 || V.lean == 2)
+                    put_ce_of_liquid(b, cur, idx);
                 G(b.gr)[idx] = (int) id;
                 const double *rot;
                 int src;
@@ -941,7 +953,15 @@ struct RwPlane {
     double fs[RY + 2], efs[RY];
     float t[TF ? RY : 1];
     int g[RY];
+    unsigned long long w;            // act words of buffer nxt: lane r has row r
 };
+
+__device__ __forceinline__ unsigned long long
+lane_word(unsigned long long v, int lane)
+{
+    return (unsigned long long) (unsigned) __builtin_amdgcn_readlane((int) v, lane) |
+           (unsigned long long) (unsigned) __builtin_amdgcn_readlane((int) (v >> 32), lane) << 32;
+}
 
 // base + byte offset: a scalar base and a 32-bit lane offset, the addressing
 // form of a global load or store that needs no 64-bit lane arithmetic
@@ -970,16 +990,27 @@ at_byte(MMCA_GLOBAL T *base, unsigned off)
 // come last in the sum, so its x and y terms wait in a register until the
 // plane above has landed.
 //
+// Where the steps of a call are lean (V.lean), what stays as it is isn't
+// written: in a row of 64 liquid cells fs and the mask, zero in both buffers,
+// and ce, which is cl again after the partitioning (cl = ce, fs = 0).  Such a
+// row writes 8 bytes a cell instead of 24.  What decides it are gr, read
+// anyway, and one word a row, the cells that were solid when buffer nxt was
+// last written (act).  Leaving out the loads as well (of rows with no solid
+// cell in sight, from act words two planes ahead) made the kernel issue-bound
+// by the tests for it: 323 us for 256 x 256 x 512, and 55 instead of 36 for 150
+// x 140 x 165.
+//
 // Bound by memory: with the arithmetic taken out (a timing copy) the walk over
 // 256 x 256 x 512 takes the same time.  Two rows per wave and 16 planes read
 // the fewest halo rows that still leave two waves per SIMD in registers.
 // FP64, 256 x 256 x 512: 403 us (447 us with planes staged in LDS, 4.2 TB/s
-// of 56 B per cell); 128 x 128 x 256: 48 us (142); 40 x 36 x 44: 8.3 us (93).
-// FP32-deviation storage, 256 x 256 x 512: 293 us (337).
+// of 56 B per cell), 336 us lean with 2/3 of the rows liquid; 128 x 128 x 256:
+// 48 us (142), 45 lean; 40 x 36 x 44: 8.3 us (93).  FP32-deviation storage,
+// 256 x 256 x 512: 293 us (337).
 constexpr int RW_LATE = 2048;                    // waiting cells of a tile buffered in LDS
 
 template <int RY, bool F32, bool TF>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, RY == 1 ? 4 : 2)
 k_solute_rw(View V, int cur, int nxt)
 {
     using S = typename Store<F32>::T;
@@ -1018,6 +1049,9 @@ k_solute_rw(View V, int cur, int nxt)
     MMCA_GLOBAL int *grb = G(dd->b.gr);
     const MMCA_GLOBAL float *tb = G(dd->b.temp32);
     MMCA_GLOBAL unsigned long long *mask = G(dd->b.mask);
+    constexpr bool LEAN = !F32 && !TF;
+    const int lean = LEAN ? V.lean : 0;
+    MMCA_GLOBAL unsigned long long *actn = G(dd->b.act[nxt]);
     const int lane = threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int rows = blockDim.y * RY;
@@ -1061,8 +1095,13 @@ k_solute_rw(View V, int cur, int nxt)
         // rows relative to row j0 - 1: the padding row is the last one loaded
         const int rmax = c.ny + 2 - j0;
         const long long row0 = (long long) (j0 - 1) * c.sx;
+        const MMCA_GLOBAL unsigned long long *wsrc =
+            actn + (long long) (j0 - 1 + min(lane < RY ? lane + 1 : 1, rmax)) * c.w64 + bx;
+        const long long wplane = (long long) (c.ny + 2) * c.w64;
         auto load = [&](RwPlane<RY, F32, TF> &p, int k) {
             const long long at = k * c.sxy + row0;
+            if constexpr (LEAN)
+                p.w = wsrc[k * wplane];
 #pragma unroll
             for (int r = 0; r < RY + 2; ++r)
             {
@@ -1093,6 +1132,7 @@ k_solute_rw(View V, int cur, int nxt)
         double psum[RY], pcl[RY], pfs[RY], pce[RY], pfz[RY];
         float pt[TF ? RY : 1];
         int pg[RY];
+        unsigned long long pw = 0;
         RwPlane<RY, F32, TF> P0, P1;
         load(P0, k0);
         {
@@ -1130,6 +1170,8 @@ k_solute_rw(View V, int cur, int nxt)
                     const double ce_new = pce[r] + sum;
                     int g_new = 0;
                     bool wait = false;
+                    const unsigned long long solid = __ballot(pg[r] > 0 && x <= c.nx);
+                    const bool put_fs = !LEAN || !lean || (solid | lane_word(pw, r)) != 0, put_ce = lean != 1 || solid != 0;
                     if (j <= c.ny && x <= c.nx)
                     {
                         const long long at = (k - 1) * c.sxy + row0;
@@ -1140,9 +1182,10 @@ k_solute_rw(View V, int cur, int nxt)
                             const double dev = ce_new - c.cinit;
                             const float f = (float) dev;
                             lost += dev - (double) f;
-                            *at_byte(ceb + at, o * E) = f;
+                            if (put_ce)
+                                *at_byte(ceb + at, o * E) = f;
                         }
-                        else
+                        else if (put_ce)
                             *at_byte(ceb + at, o * E) = ce_new;
                         if constexpr (TF)
                             wait = pg[r] > 0 && !branch_decided(c, (double) pt[r], beam_margin(c, (double) pt[r]),
@@ -1171,7 +1214,8 @@ k_solute_rw(View V, int cur, int nxt)
                                 *at_byte(cln + at, o * E) = (float) (cl_out - c.cinit);
                             else
                                 *at_byte(cln + at, o * E) = cl_out;
-                            *at_byte(fsn + at, o * 8) = fs_out;
+                            if (put_fs)
+                                *at_byte(fsn + at, o * 8) = fs_out;
                             if (g_new != pg[r])
                             {
                                 *at_byte(grb + at, o * 4) = g_new;
@@ -1180,9 +1224,17 @@ k_solute_rw(View V, int cur, int nxt)
                             }
                         }
                     }
-                    const unsigned long long bits = __ballot(g_new > 0);
-                    if (lane == 0 && j <= c.ny)
-                        mask[((long long) (k - 1) * (c.ny + 2) + j) * c.w64 + bx] = bits;
+                    if (put_fs)
+                    {
+                        const unsigned long long bits = __ballot(g_new > 0);
+                        if (lane == 0 && j <= c.ny)
+                        {
+                            const long long w = ((long long) (k - 1) * (c.ny + 2) + j) * c.w64 + bx;
+                            mask[w] = bits;
+                            if (lean)
+                                actn[w] = solid;
+                        }
+                    }
                     if constexpr (TF)
                     {
                         const unsigned long long late = __ballot(wait);
@@ -1217,7 +1269,7 @@ k_solute_rw(View V, int cur, int nxt)
                 psum[r] = sum;
                 pcl[r] = cl;
                 pfs[r] = fs;
-                pce[r] = from_raw<F32>(c, A.ce[r]);
+                pce[r] = (lean == 0 || lean == 3 || A.g[r] > 0) ? from_raw<F32>(c, A.ce[r]) : cl;
                 pg[r] = A.g[r];
                 pfz[r] = fz;
                 if constexpr (TF)
@@ -1225,6 +1277,8 @@ k_solute_rw(View V, int cur, int nxt)
                 fy = fyu;
                 cl = clu;
             }
+            if constexpr (LEAN)
+                pw = A.w;
         };
         // the loop starts with nothing in flight, so that its waits are the
         // steady-state ones
@@ -1241,6 +1295,8 @@ k_solute_rw(View V, int cur, int nxt)
     }
     if (c.check_neg && neg)
         flag_negative_ce(V, c, dd->b.cnt);
+    if (lean && lane == 0 && threadIdx.y == 0)
+        G(dd->b.stamp)[tile] = (unsigned) G(dd->b.cnt)->timestep;
     if constexpr (TF)
     {
         __syncthreads();
@@ -1259,6 +1315,51 @@ k_solute_rw(View V, int cur, int nxt)
         const double tot = block_sum(lost, s_red, 64 * blockDim.y);
         if (lane == 0 && threadIdx.y == 0 && tot != 0.0)
             ledger_add(dd->b, tile, tot);
+    }
+}
+
+// upper bound of a block's solute tiles, of whatever shape
+__host__ __device__ __forceinline__ long long
+tile_slots_d(const Consts &c)
+{
+    return (long long) ((c.nx + 63) / 64) * ((c.ny + 3) / 4) * c.nz;
+}
+
+// Start of a call of lean steps: nothing is known of any cell.
+__global__ void __launch_bounds__(256)
+k_wake_all(View V)
+{
+    const DevBufs b = V.dom[blockIdx.y].b;    // private copy: stores cannot alias it
+    const Consts c = V.dom[blockIdx.y].c;
+    const long long n = (long long) (c.nz + 2) * (c.ny + 2) * c.w64;
+    const long long nt = tile_slots_d(c);
+    for (long long i = (long long) blockIdx.x * 256 + threadIdx.x; i < max(n, nt); i += 256ll * gridDim.x)
+    {
+        if (i < n)
+            G(b.act[0])[i] = G(b.act[1])[i] = ~0ull;
+        if (i < nt)
+            G(b.stamp)[i] = ~0u;
+    }
+}
+
+// After lean steps that stopped on an error at the timestep `failed` (not the
+// first of the call): ce of the liquid cells, which need not have been
+// written.  The tiles that finished that step left it as cl in the buffer
+// `cur`, the others in the one before.
+__global__ void __launch_bounds__(256)
+k_settle(DevBufs b, Consts c, int cur, unsigned failed)
+{
+    const unsigned ntx = (unsigned) (c.nx + 63) / 64, nty = (unsigned) (c.ny + c.zm_by - 1) / c.zm_by;
+    const long long N = (long long) c.nx * c.ny * c.nz;
+    for (long long i = (long long) blockIdx.x * 256 + threadIdx.x; i < N; i += 256ll * gridDim.x)
+    {
+        const int x = (int) (i % c.nx) + 1, j = (int) (i / c.nx % c.ny) + 1, k = (int) (i / c.nx / c.ny) + 1;
+        const unsigned tile = ((unsigned) (k - 1) / c.zm_planes * nty + (unsigned) (j - 1) / c.zm_by) * ntx +
+                              (unsigned) (x - 1) / 64;
+        const int buf = G(b.stamp)[tile] == failed ? cur : cur ^ 1;
+        const long long idx = k * c.sxy + (long long) j * c.sx + x;
+        if (G(b.gr)[idx] <= 0)
+            put_ce_of_liquid(b, buf, idx);
     }
 }
 
@@ -1705,7 +1806,9 @@ k_capture(View V, int cb, int rows)
             tz = ddz + nnz[found] + g20 * ncx + g21 * ncy + g22 * ncz;
             G(b.gr)[idx] = gfound;
             fsb[idx] = 0.;
-            if (c.f32)
+            if (V.lean)
+                put_ce_of_liquid(b, cb, idx);         // cl = ce already
+            else if (c.f32)
                 cl32_buf(b, cb)[idx] = G(b.ce32)[idx];
             else
                 clb[idx] = G(b.ce)[idx];
@@ -2328,7 +2431,7 @@ hipError_t launch_nucleate(const View &v, int mode, int cur, hipStream_t s)
 hipError_t launch_nucleate_coupled(const View &v, int cur, hipStream_t s)
 {
     hipLaunchKernelGGL(k_nuc_detect, dim3((unsigned) v.tot_nuc), dim3(NUC_BS), 0, s, v, 1 | 8, cur);
-    hipLaunchKernelGGL(k_nuc_activate_coupled, dim3(1), dim3(NUC_BS), 0, s, v);
+    hipLaunchKernelGGL(k_nuc_activate_coupled, dim3(1), dim3(NUC_BS), 0, s, v, cur);
     return hipGetLastError();
 }
 
@@ -2437,6 +2540,21 @@ long long zm_tiles(const Consts &c, int by)
 // 63.8 us with a launch of its own, 256 x 256 x 512 (8192) 603 against 571: the
 // counter that orders the workgroups is one address for all XCDs.
 constexpr long long LIST_FUSED = 192;
+
+long long tile_slots(const Consts &c) { return tile_slots_d(c); }
+
+
+hipError_t launch_wake_all(const View &v, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_wake_all, dim3(64, (unsigned) v.ndom), dim3(256), 0, s, v);
+    return hipGetLastError();
+}
+
+hipError_t launch_settle(const DevBufs &b, const Consts &c, int cur, unsigned failed, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_settle, dim3(1024), dim3(256), 0, s, b, c, cur, failed);
+    return hipGetLastError();
+}
 
 hipError_t launch_list(const View &v, int cb, int capture, int decide_realloc, hipStream_t s)
 {
