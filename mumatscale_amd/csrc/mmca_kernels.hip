@@ -1689,7 +1689,10 @@ k_list_write(View V)
 // its slot, so the slots may be dealt to the threads in any order.  `cb` is
 // the buffer holding fs/cl after fs_change; `rows` is 1 when the list writer
 // of the same list has filled row_first (the row bands need it).
-__global__ void __launch_bounds__(LIST_BS)
+// Bound by the latency of its loads (slot, then neighbours, then rotation
+// matrix; 2.3 TB/s), so by the waves in flight: 128 registers, for four waves
+// per SIMD instead of three.
+__global__ void __launch_bounds__(LIST_BS, 4)
 k_capture(View V, int cb, int rows)
 {
     const int dm = find_dom(V.off_cap, V.ndom, blockIdx.x);
@@ -1708,7 +1711,7 @@ k_capture(View V, int cb, int rows)
     MMCA_GLOBAL double *clb = cl_buf(b, cb);
     auto member = [&](long long t) {
         const int slot = (int) t + 1;
-        const unsigned idx = (unsigned) G(b.diff_id)[slot];
+        const int idx = G(b.diff_id)[slot];
         double tx, ty, tz;
         if (realloc)
             tx = ty = tz = 0.0;
@@ -1722,8 +1725,8 @@ k_capture(View V, int cb, int rows)
         const int nnx[6] = { 1, 0, -1, 0, 0, 0 };
         const int nny[6] = { 0, 1, 0, -1, 0, 0 };
         const int nnz[6] = { 0, 0, 0, 0, 1, -1 };
-        const long long ndxs[6] = { (long long) idx + 1, (long long) idx + c.sx, (long long) idx - 1,
-                                    (long long) idx - c.sx, (long long) idx + c.sxy, (long long) idx - c.sxy };
+        const int sxy = (int) c.sxy;                     // padded cells < 2^31
+        const int ndxs[6] = { idx + 1, idx + c.sx, idx - 1, idx - c.sx, idx + sxy, idx - sxy };
         // solid neighbours before capture (recorded by the list writer); their
         // grain ids, centres and fs are independent loads issued together
         const unsigned int sol = G(b.nbr)[slot];
@@ -1737,9 +1740,10 @@ k_capture(View V, int cb, int rows)
             if ((sol >> n) & 1u)
             {
                 gids[n] = G(b.gr)[ndxs[n]];
-                pdc[n][0] = G(b.dc)[3 * ndxs[n]];
-                pdc[n][1] = G(b.dc)[3 * ndxs[n] + 1];
-                pdc[n][2] = G(b.dc)[3 * ndxs[n] + 2];
+                const MMCA_GLOBAL double *p = G(b.dc) + 3 * (long long) ndxs[n];
+                pdc[n][0] = p[0];
+                pdc[n][1] = p[1];
+                pdc[n][2] = p[2];
                 pfs[n] = fsb[ndxs[n]];
             }
         }
