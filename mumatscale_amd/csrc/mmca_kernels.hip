@@ -1009,7 +1009,7 @@ at_byte(MMCA_GLOBAL T *base, unsigned off)
 // 256 x 256 x 512: 293 us (337).
 constexpr int RW_LATE = 2048;                    // waiting cells of a tile buffered in LDS
 
-template <int RY, bool F32, bool TF>
+template <int RY, bool F32, bool TF, bool LEAN>
 __global__ void __launch_bounds__(512, RY == 1 ? 4 : 2)
 k_solute_rw(View V, int cur, int nxt)
 {
@@ -1049,7 +1049,6 @@ k_solute_rw(View V, int cur, int nxt)
     MMCA_GLOBAL int *grb = G(dd->b.gr);
     const MMCA_GLOBAL float *tb = G(dd->b.temp32);
     MMCA_GLOBAL unsigned long long *mask = G(dd->b.mask);
-    constexpr bool LEAN = !F32 && !TF;
     const int lean = LEAN ? V.lean : 0;
     MMCA_GLOBAL unsigned long long *actn = G(dd->b.act[nxt]);
     const int lane = threadIdx.x;
@@ -1171,7 +1170,7 @@ k_solute_rw(View V, int cur, int nxt)
                     int g_new = 0;
                     bool wait = false;
                     const unsigned long long solid = __ballot(pg[r] > 0 && x <= c.nx);
-                    const bool put_fs = !LEAN || !lean || (solid | lane_word(pw, r)) != 0, put_ce = lean != 1 || solid != 0;
+                    const bool put_fs = !LEAN || (solid | lane_word(pw, r)) != 0, put_ce = !LEAN || lean != 1 || solid != 0;
                     if (j <= c.ny && x <= c.nx)
                     {
                         const long long at = (k - 1) * c.sxy + row0;
@@ -1231,7 +1230,7 @@ k_solute_rw(View V, int cur, int nxt)
                         {
                             const long long w = ((long long) (k - 1) * (c.ny + 2) + j) * c.w64 + bx;
                             mask[w] = bits;
-                            if (lean)
+                            if constexpr (LEAN)
                                 actn[w] = solid;
                         }
                     }
@@ -1269,7 +1268,7 @@ k_solute_rw(View V, int cur, int nxt)
                 psum[r] = sum;
                 pcl[r] = cl;
                 pfs[r] = fs;
-                pce[r] = (lean == 0 || lean == 3 || A.g[r] > 0) ? from_raw<F32>(c, A.ce[r]) : cl;
+                pce[r] = (!LEAN || lean == 3 || A.g[r] > 0) ? from_raw<F32>(c, A.ce[r]) : cl;
                 pg[r] = A.g[r];
                 pfz[r] = fz;
                 if constexpr (TF)
@@ -1295,7 +1294,7 @@ k_solute_rw(View V, int cur, int nxt)
     }
     if (c.check_neg && neg)
         flag_negative_ce(V, c, dd->b.cnt);
-    if (lean && lane == 0 && threadIdx.y == 0)
+    if (LEAN && lane == 0 && threadIdx.y == 0)
         G(dd->b.stamp)[tile] = (unsigned) G(dd->b.cnt)->timestep;
     if constexpr (TF)
     {
@@ -2467,10 +2466,19 @@ static void launch_solute_t(const View &v, int zm_by, int diff, int fsc, int rec
         const dim3 grid((unsigned) ((v.tot_zm + run - 1) / run * run));
         const size_t tlds = AM ? 0 : (size_t) std::max(v.zm_planes_max, 16) * sizeof(double);   // per plane or row
         const dim3 wg(64, zm_by == 16 ? 8 : 4);      // waves of 2 rows (of 1 row for 4-row tiles)
+        if constexpr (!F32 && !AM)
+            if (v.lean)
+            {
+                if (zm_by == 4)
+                    hipLaunchKernelGGL((k_solute_rw<1, F32, AM, true>), grid, wg, tlds, s, v, cur, nxt);
+                else
+                    hipLaunchKernelGGL((k_solute_rw<2, F32, AM, true>), grid, wg, tlds, s, v, cur, nxt);
+                return;
+            }
         if (zm_by == 4)
-            hipLaunchKernelGGL((k_solute_rw<1, F32, AM>), grid, wg, tlds, s, v, cur, nxt);
+            hipLaunchKernelGGL((k_solute_rw<1, F32, AM, false>), grid, wg, tlds, s, v, cur, nxt);
         else
-            hipLaunchKernelGGL((k_solute_rw<2, F32, AM>), grid, wg, tlds, s, v, cur, nxt);
+            hipLaunchKernelGGL((k_solute_rw<2, F32, AM, false>), grid, wg, tlds, s, v, cur, nxt);
     }
     else if (diff && fsc)
         hipLaunchKernelGGL((k_solute<true, true, AM, F32>), dim3((unsigned) v.tot_cell), blk, 0, s, v, cur, nxt);
