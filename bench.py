@@ -43,8 +43,8 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-TRAFFIC_PROFILES = {"fp64": os.path.join(ROOT, "profiles", "k_solute_zl_directional_256x256x512_fp64.md"),
-                    "fp32": os.path.join(ROOT, "profiles", "k_solute_zl_directional_256x256x512_fp32dev.md")}
+TRAFFIC_PROFILES = {"fp64": os.path.join(ROOT, "profiles", "k_solute_rw_directional_256x256x512_fp64.md"),
+                    "fp32": os.path.join(ROOT, "profiles", "k_solute_rw_directional_256x256x512_fp32dev.md")}
 
 
 def bandwidth_probe(cells, reps=20):
@@ -90,6 +90,14 @@ def measured_traffic(size, shape, prec="fp64"):
     if not rec or not m or rec.groups() != want:
         return None
     return float(m.group(1))
+
+
+def liquid_rows(sb):
+    """Share of the block's rows of 64 cells along x without a solid cell."""
+    import numpy as np
+    g = sb.download(abi.FIELD_GR)[1:-1, 1:-1, 1:-1] > 0
+    g = np.pad(g, ((0, 0), (0, 0), (0, -g.shape[2] % 64)))
+    return 1.0 - g.reshape(*g.shape[:2], -1, 64).any(-1).mean()
 
 
 def run_ensemble(steps, baseline_steps):
@@ -336,14 +344,14 @@ def run_am_track(steps=60):
     """The AM single track over a 2000-grain Voronoi substrate (1024 x 512 x
     256, dx = 0.5 um, Gaussian-beam temperature), its error against the FP64
     run of the same steps, in three forms:
-      fp32dev            FP32-deviation storage, the beam temperature from its
-                         separable factors (a 400-deep product over the block,
-                         computed once per step);
-      fp32dev_quadrature FP32-deviation storage, the 400-term quadrature per
-                         cell (temperature.c:88-118);
-      fp64               FP64 storage and the quadrature, bit for bit the
-                         reference's.
-    The quadrature forms are bound by FP64 VALU work, not HBM."""
+      fp32dev            FP32-deviation storage, temperature outputs from the
+                         beam's separable factors (a 400-deep product over the
+                         block);
+      fp32dev_quadrature FP32-deviation storage, temperature outputs from the
+                         400-term quadrature per cell (temperature.c:88-118);
+      fp64               FP64 storage, bit for bit the reference's.
+    The steps themselves take the quadrature's value in every form, at the
+    cells whose branch an approximate temperature leaves open."""
     import numpy as np
     from mumatscale_amd.lib import Subblock
     from mumatscale_amd.workloads import am_track_config, apply_substrate, voronoi_substrate
@@ -371,8 +379,6 @@ def run_am_track(steps=60):
             out[key] = {"value": round(n * steps / wall / 1e6, 1), "unit": "Mcell-updates/s",
                         "ms_per_step": round(wall / steps * 1e3, 3), "k_solute_ms": round(k_ms, 3),
                         "grains": rep.num_grains - 1, "solid_fraction": rep.solid_sum / n}
-            if key != "fp32dev":
-                out[key]["beam_terms_per_s"] = round(n * 400 / (k_ms * 1e-3), 1) if k_ms > 0 else None
             log("am track %s: %.3f ms/step" % (key, wall / steps * 1e3))
     c64, r64, t64 = fields["fp64"]
     for key in ("fp32dev", "fp32dev_quadrature"):
@@ -384,15 +390,7 @@ def run_am_track(steps=60):
         if t32 is not None:
             err["temperature_rel_max"] = float(np.max(np.abs(t32 - t64) / np.maximum(np.abs(t64), 1.0)))
         out[key]["error_vs_fp64"] = err
-    # The compiled quadrature loop issues 51 FP64 VALU instructions per term
-    # (two divisions and an exp each); MI355X issues 78.6e12 / 2 FP64 lane
-    # operations per second.
-    valu_per_term = 51
-    for key in ("fp32dev_quadrature", "fp64"):
-        t = out[key]["beam_terms_per_s"]
-        out[key]["valu_frac"] = round(t * valu_per_term / (78.6e12 / 2), 3) if t else None
-    out.update({"cells": n, "steps": steps, "dt": cfg.dt, "substrate_grains": len(recs) - 1,
-                "valu_ops_per_term": valu_per_term})
+    out.update({"cells": n, "steps": steps, "dt": cfg.dt, "substrate_grains": len(recs) - 1})
     return out
 
 
@@ -609,6 +607,7 @@ def main():
     n = nx * ny * nz
     if args.warmup:
         gpu.step(args.warmup)
+    rows = liquid_rows(gpu)
     gpu.set_kernel_timing(True)
     t0 = time.perf_counter()
     rep = gpu.step(args.steps)        # synchronises on return; raises on a negative ce
@@ -619,7 +618,10 @@ def main():
     value = n * args.steps / wall / 1e6
     log("gpu: %d steps in %.3f s, grains %d, gindex %d, k_solute avg %.4f ms over %d launches"
         % (args.steps, wall, rep.num_grains, rep.gindex, k_ms, k_n))
+    rows = (rows + liquid_rows(gpu)) / 2
     gpu.close()
+    if not fp32 and used["zm"] > 0:
+        b_alg -= 16.0 * rows          # lean steps don't write ce and fs of liquid rows
     probe = bandwidth_probe(n)
     log("bandwidth probe:", probe)
     achieved = n * b_alg / (k_ms * 1e-3) / 1e9 if k_ms > 0 else None
@@ -629,7 +631,7 @@ def main():
             "traffic": measured_traffic(args.size, used, "fp32" if fp32 else "fp64"),
             "kernel": ("k_solute_rw<%d>" % (1 if used["rows"] == 4 else 2)) if used["zm"] > 0
             else "k_solute<true,true>",
-            "bytes_per_cell": b_alg}
+            "bytes_per_cell": round(b_alg, 2), "liquid_rows": round(rows, 4)}
     if probe and achieved:
         mix = probe["solute_mix_fp32dev" if fp32 else "solute_mix_fp64"]["GB/s"]
         roof["probe_same_mix_gbs"] = mix

@@ -1939,8 +1939,9 @@ long long batch_chunk_steps(const mmca_batch *bt)
     return std::min<long long>(64, std::max<long long>(8, 32768 / std::max<long long>(1, ns)));
 }
 
-// one doiteration() of every domain: seven launches whatever the batch size
-// (ten for a coupled batch: two halo exchanges and the cross-rank activation)
+// one doiteration() of every domain: five or six launches whatever the batch
+// size (three more for a coupled batch: two halo exchanges and the cross-rank
+// activation)
 int batch_enqueue(mmca_batch *bt, int cur, int lean)
 {
     bt->view.lean = lean;
