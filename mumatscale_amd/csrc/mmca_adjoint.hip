@@ -92,11 +92,23 @@ struct Cell {
     bool active;
 };
 
+// Tile of this workgroup: the hardware places workgroup w on XCD w % 8, so each
+// XCD takes one contiguous eighth of the tiles, whose work is equal, and tiles
+// that share halo cells share an L2 (128 x 120 x 104: replay 23.7 us with tiles
+// dealt one by one, 22.1 with eighths, and no less with two to four planes per
+// thread on top of that; the adjoint step in place 66 and 52).
+__device__ __forceinline__ int
+xcd_eighth()
+{
+    const int per = gridDim.x / 8;
+    return (int) blockIdx.x < 8 * per ? (blockIdx.x % 8) * per + blockIdx.x / 8 : blockIdx.x;
+}
+
 __device__ __forceinline__ Cell
 cell_of(const Consts &c)
 {
     const int gbx = (c.nx + ADJ_BX - 1) / ADJ_BX, gby = (c.ny + ADJ_BY - 1) / ADJ_BY;
-    const long long blk = blockIdx.x;
+    const long long blk = xcd_eighth();
     Cell q;
     q.x = (int) (blk % gbx) * ADJ_BX + threadIdx.x + 1;
     q.j = (int) ((blk / gbx) % gby) * ADJ_BY + threadIdx.y + 1;
@@ -309,10 +321,11 @@ diff_adjoint(const Consts &c, double lc, const DiffSums &q)
 // the inputs again.
 // Partials of (d_liq, d_sol, part_coef) go to part[3 * blk]; the workgroup
 // that finishes last adds their sums, in fixed order, to g_param.
-// 128 x 120 x 104: 51 us against 31 + 33 + 10 of the two passes and their sum;
-// 48 x 41 x 56: 17 against 6 + 6 + 3 and two launches more.  A liquid block
-// stepped again and again, in one pass and in two: 24 x 20 x 22 11.9 and 12.0
-// us, 64^3 16.3 and 16.5, 256^3 283 and 735.  It is bound by
+// 128 x 120 x 104 along a trajectory: 51 us against 31 + 33 + 10 of the two
+// passes and their sum (before xcd_eighth).  A liquid block stepped again and
+// again, in one pass and in two: 24 x 20 x 22 12.0 and 12.4 us, 48 x 41 x 56
+// 14.4 and 13.7, 64^3 16.3 and 16.1, 128 x 120 x 104 30 and 52, 256^3 283 and
+// 692.  It is bound by
 // memory latency: the rings and the planes at the ends of the walks bring the
 // 121 MB to some 200, and LDS and registers hold one workgroup per CU (tiles
 // of 4, 5, 12 and 13 rows, two workgroups per CU: 49 to 53 us).
@@ -338,10 +351,7 @@ k_adj_fused(Consts c, Deriv dv, int kz, const unsigned char *code, double sim_ti
 
     const int tid = threadIdx.x;
     const int gbx = (c.nx + ADJ_TX - 1) / ADJ_TX, gby = (c.ny + TY - 1) / TY;
-    // workgroups go to the 8 XCDs in turn: neighbouring tiles, which share
-    // their rings, to the same one
-    const int per = gridDim.x / 8;
-    const int w = (int) blockIdx.x < 8 * per ? (blockIdx.x % 8) * per + blockIdx.x / 8 : blockIdx.x;
+    const int w = xcd_eighth();
     const int x0 = (w % gbx) * ADJ_TX + 1, j0 = ((w / gbx) % gby) * TY + 1, z0 = (w / (gbx * gby)) * kz + 1;
     const int z1 = min(z0 + kz - 1, c.nz);
 
