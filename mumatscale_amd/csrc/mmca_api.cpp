@@ -450,6 +450,16 @@ bool lean_call(mmca_ctx *const *ctxs, size_t n, int nsteps, bool tiles)
     return nsteps >= LEAN_STEPS && tiles && !c.f32 && !c.am && cells >= LEAN_CELLS;
 }
 
+// ce of the liquid cells after lean steps that end before the call's last one,
+// from cl in the buffer `cur` (no tile has the stamp 0: the first step's
+// timestep is 1)
+int settle_all(mmca_ctx *ctx, int cur, hipStream_t s)
+{
+    HIPCHK(launch_settle(ctx->b, ctx->c, cur ^ 1, 0u, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return MMCA_OK;
+}
+
 // View::lean of step n (from 0) of a call
 int lean_mode(bool lean, int n, int nsteps) { return !lean ? 0 : n == 0 ? 3 : n + 1 < nsteps ? 1 : 2; }
 
@@ -889,8 +899,11 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
                 if (ctx->rand_filled < ctx->rand_capacity)
                     k = std::min({ k, ch, cover });
             }
-            if (k < 1)
+            if (k < 1) {
+                if (lean && done > 0)
+                    TRY(settle_all(ctx, ctx->cur, ctx->stream));
                 return MMCA_ERR_STATE;
+            }
             for (long long n = 0; n < k; n++)
                 TRY(enqueue_iteration(ctx, true, lean_mode(lean, done + (int) n, nsteps)));
             done += (int) k;
@@ -2340,8 +2353,12 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
             if (c->rand_filled < c->rand_capacity)
                 k = std::min(k, spare / c->b.nsites);
         }
-        if (k < 1)
+        if (k < 1) {
+            for (mmca_ctx *c : bt->dom)
+                if (lean && done > 0 && c->hc.status == MMCA_OK)
+                    TRY(settle_all(c, bt->cur, bt->stream));
             return MMCA_ERR_STATE;
+        }
         long long n = 0;
         if (bt->use_graph && !bt->timing) {
             if (lean && done == 0) {                 // the first step is like no other
