@@ -2224,6 +2224,10 @@ k_beam_field(DevBufs b, Consts c, BeamSet p, int adv)
 // the grid's threads: one thread per cell, or two or four while the grid has
 // that many, so that the 400-term chains stay short.
 //
+// A step that the solute kernel stopped on a negative ce is finished too: its
+// waiting cells hold what defer_cell kept, and its buffers stay current.  The
+// steps issued after it leave the list empty (k_beam_ax).
+//
 // Bound by the FP64 VALU of the quadrature, about 40 instructions per term.
 // About 120 000 waiting cells of a 250 x 190 x 94 block: 85 us; a kernel that
 // evaluated every solid cell in place took 10 ms a step.
@@ -2234,7 +2238,8 @@ k_beam_finish(View V, int cur, int nxt)
     __shared__ BeamTab s_tab;
     const DevBufs b = V.dom[blockIdx.y].b;    // private copy: stores cannot alias it
     const Consts c = V.dom[blockIdx.y].c;
-    if (G(b.cnt)->status != MMCA_OK)
+    const MMCA_GLOBAL Counters *cnt = G(b.cnt);
+    if (cnt->status != MMCA_OK && !(cnt->status == MMCA_ERR_NEGATIVE_CE && cnt->failed_step == cnt->timestep))
         return;
     const int tid = threadIdx.x;
     const int n = *G(b.und_n);
