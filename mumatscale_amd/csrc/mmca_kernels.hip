@@ -2126,8 +2126,8 @@ __global__ void __launch_bounds__(256)
 k_beam_field(DevBufs b, Consts c, BeamSet p, int adv)
 {
     const MMCA_GLOBAL Counters *cnt = G(b.cnt);
-    if (cnt->status != MMCA_OK)
-        return;                                   // uniform over the workgroup
+    if (!OUT && cnt->status != MMCA_OK)
+        return;                                   // uniform over the workgroup; an output is one of a stopped block too
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int xp = beam_x_pitch(c), K = p.rank;
