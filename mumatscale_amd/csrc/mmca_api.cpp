@@ -11,6 +11,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "host_init.h"
@@ -73,6 +76,26 @@ using namespace mmca;
 #endif
 
 
+// Device memory through which FP32-deviation fields pass on their way to or from
+// the host, as doubles: one buffer of at most STAGE_CELLS (64 MB) for all
+// contexts on a device, so that many domains together don't hold a second copy
+// of their fields.  It comes with the first transfer, grows to the largest
+// block's need and goes with the last context.  A transfer holds the lock until
+// its stream has finished.
+constexpr size_t STAGE_CELLS = (size_t) 8 << 20;
+
+struct Staging {
+    std::mutex mu;
+    int device = 0;
+    double *buf = nullptr;
+    size_t cells = 0;
+    ~Staging()
+    {
+        if (buf && hipSetDevice(device) == hipSuccess)
+            (void) hipFree(buf);
+    }
+};
+
 struct mmca_ctx {
     mmca_params p;
     Consts c;
@@ -115,9 +138,9 @@ struct mmca_ctx {
     long long time_n = 0;
     // grain records set by mmca_set_grains (ids below ext_grains.size())
     std::vector<mmca_grain> ext_grains;
-    // staging buffer of mmca_io_fields and of FP32-deviation fields on their way
-    // to or from the host: 4 x P 32-bit values (allocated on first use)
+    // staging buffer of mmca_io_fields: 4 x P 32-bit values (allocated on first use)
     float *io_buf = nullptr;
+    std::shared_ptr<Staging> stage;   // FP32-deviation storage only
     // The random stream at the start of the orientation queue (before draw
     // q0).  mmca_rand draws from rng_now, the stream right after the
     // orientations consumed so far; the queue from there on is then redrawn
@@ -245,12 +268,70 @@ int ensure_d(mmca_ctx *ctx)
     return MMCA_OK;
 }
 
-// staging buffer of mmca_io_fields, as P doubles
-int staging(mmca_ctx *ctx, double **out)
+std::shared_ptr<Staging> staging_of(int device)
 {
-    if (!ctx->io_buf)
-        TRY(dev_alloc(&ctx->io_buf, 4 * (size_t) ctx->c.P));
-    *out = (double *) ctx->io_buf;
+    static std::mutex mu;
+    static std::map<int, std::weak_ptr<Staging>> all;
+    std::lock_guard<std::mutex> lock(mu);
+    std::shared_ptr<Staging> s = all[device].lock();
+    if (!s) {
+        s = std::make_shared<Staging>();
+        s->device = device;
+        all[device] = s;
+    }
+    return s;
+}
+
+// The buffer for a field of n cells, by a caller that holds its lock; a smaller
+// one where memory is short, for more and smaller pieces.
+int staging_buffer(Staging &s, size_t n)
+{
+    size_t want = std::min(n, STAGE_CELLS);
+    if (s.cells >= want)
+        return MMCA_OK;
+    if (s.buf)
+        HIPCHK(hipFree(s.buf));
+    s.buf = nullptr;
+    s.cells = 0;
+    while (hipMalloc((void **) &s.buf, want * sizeof(double)) != hipSuccess) {
+        (void) hipGetLastError();
+        s.buf = nullptr;
+        if (want <= (size_t) 1 << 16)
+            return MMCA_ERR_HIP;
+        want /= 2;
+    }
+    s.cells = want;
+    return MMCA_OK;
+}
+
+// values of an FP32-deviation field from the host (dev2: null or a second copy)
+int narrow_from_host(mmca_ctx *ctx, const double *host, float *dev, float *dev2)
+{
+    Staging &s = *ctx->stage;
+    const size_t P = (size_t) ctx->c.P;
+    std::lock_guard<std::mutex> lock(s.mu);
+    TRY(staging_buffer(s, P));
+    for (size_t at = 0; at < P; at += s.cells) {
+        const size_t n = std::min(s.cells, P - at);
+        HIPCHK(hipMemcpyAsync(s.buf, host + at, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(launch_narrow(s.buf, dev + at, dev2 ? dev2 + at : nullptr, ctx->c.cinit, (long long) n, ctx->stream));
+    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return MMCA_OK;
+}
+
+int widen_to_host(mmca_ctx *ctx, const float *dev, double *host)
+{
+    Staging &s = *ctx->stage;
+    const size_t P = (size_t) ctx->c.P;
+    std::lock_guard<std::mutex> lock(s.mu);
+    TRY(staging_buffer(s, P));
+    for (size_t at = 0; at < P; at += s.cells) {
+        const size_t n = std::min(s.cells, P - at);
+        HIPCHK(launch_widen(dev + at, s.buf, ctx->c.cinit, (long long) n, ctx->stream));
+        HIPCHK(hipMemcpyAsync(host + at, s.buf, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     return MMCA_OK;
 }
 
@@ -670,6 +751,7 @@ int mmca_create(const mmca_params *params, int device, mmca_ctx **out)
     const size_t P = (size_t) c.P;
     const size_t N = (size_t) c.nx * c.ny * c.nz;
     if (c.f32) {
+        ctx->stage = staging_of(device);
         TRY(dev_alloc(&b.ce32, P));
         TRY(dev_alloc(&b.cl32[0], P));
         TRY(dev_alloc(&b.cl32[1], P));
@@ -1137,14 +1219,8 @@ int mmca_upload_field(mmca_ctx *ctx, int field, const void *host)
     case MMCA_FIELD_CE:
     case MMCA_FIELD_CL:
         if (ctx->c.f32) {
-            double *wide;
-            TRY(staging(ctx, &wide));
-            HIPCHK(hipMemcpyAsync(wide, host, P * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-            if (field == MMCA_FIELD_CE)
-                HIPCHK(launch_narrow(wide, b.ce32, nullptr, ctx->c.cinit, ctx->c.P, ctx->stream));
-            else
-                HIPCHK(launch_narrow(wide, b.cl32[0], b.cl32[1], ctx->c.cinit, ctx->c.P, ctx->stream));
-            HIPCHK(hipStreamSynchronize(ctx->stream));
+            TRY(field == MMCA_FIELD_CE ? narrow_from_host(ctx, (const double *) host, b.ce32, nullptr)
+                                       : narrow_from_host(ctx, (const double *) host, b.cl32[0], b.cl32[1]));
         } else if (field == MMCA_FIELD_CE) {
             HIPCHK(hipMemcpy(b.ce, host, P * sizeof(double), hipMemcpyHostToDevice));
         } else {
@@ -1194,11 +1270,7 @@ int mmca_download_field(mmca_ctx *ctx, int field, void *host)
     case MMCA_FIELD_CE:
     case MMCA_FIELD_CL:
         if (c.f32) {
-            double *wide;
-            TRY(staging(ctx, &wide));
-            HIPCHK(launch_widen((field == MMCA_FIELD_CE) ? b.ce32 : b.cl32[ctx->cur], wide, c.cinit, c.P, ctx->stream));
-            HIPCHK(hipMemcpyAsync(host, wide, P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-            HIPCHK(hipStreamSynchronize(ctx->stream));
+            TRY(widen_to_host(ctx, (field == MMCA_FIELD_CE) ? b.ce32 : b.cl32[ctx->cur], (double *) host));
         } else {
             const double *src = (field == MMCA_FIELD_CE) ? b.ce : b.cl[ctx->cur];
             HIPCHK(hipMemcpy(host, src, P * sizeof(double), hipMemcpyDeviceToHost));
