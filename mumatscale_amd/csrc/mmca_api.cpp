@@ -30,7 +30,7 @@ hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStrea
 hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s);
 long long tile_slots(const Consts &c);
 hipError_t launch_wake_all(const View &v, hipStream_t s);
-hipError_t launch_settle(const DevBufs &b, const Consts &c, int cur, unsigned failed, hipStream_t s);
+hipError_t launch_settle(const DomainDesc *dom, int cur, unsigned failed, hipStream_t s);
 hipError_t launch_list(const View &v, int cb, int capture, int decide_realloc, hipStream_t s);
 hipError_t launch_nucleate_coupled(const View &v, int cur, hipStream_t s);
 hipError_t launch_halo_exchange(const View &v, int phase, int cb, long long max_face, hipStream_t s);
@@ -534,9 +534,9 @@ bool lean_call(mmca_ctx *const *ctxs, size_t n, int nsteps, bool tiles)
 // ce of the liquid cells after lean steps that end before the call's last one,
 // from cl in the buffer `cur` (no tile has the stamp 0: the first step's
 // timestep is 1)
-int settle_all(mmca_ctx *ctx, int cur, hipStream_t s)
+int settle_all(const DomainDesc *dom, int cur, hipStream_t s)
 {
-    HIPCHK(launch_settle(ctx->b, ctx->c, cur ^ 1, 0u, s));
+    HIPCHK(launch_settle(dom, cur ^ 1, 0u, s));
     HIPCHK(hipStreamSynchronize(s));
     return MMCA_OK;
 }
@@ -983,7 +983,7 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
             }
             if (k < 1) {
                 if (lean && done > 0)
-                    TRY(settle_all(ctx, ctx->cur, ctx->stream));
+                    TRY(settle_all(ctx->view.dom, ctx->cur, ctx->stream));
                 return MMCA_ERR_STATE;
             }
             for (long long n = 0; n < k; n++)
@@ -1006,7 +1006,7 @@ int mmca_step(mmca_ctx *ctx, int nsteps, int want_sums, mmca_report *report)
         if (ctx->hc.status != MMCA_OK) {
             ctx->cur = cur0 ^ (int) ((ctx->hc.timestep - t0) & 1);
             if (lean && ctx->hc.failed_step > t0 + 1) {
-                HIPCHK(launch_settle(ctx->b, ctx->c, ctx->cur, (unsigned) ctx->hc.failed_step, ctx->stream));
+                HIPCHK(launch_settle(ctx->view.dom, ctx->cur, (unsigned) ctx->hc.failed_step, ctx->stream));
                 HIPCHK(hipStreamSynchronize(ctx->stream));
             }
         }
@@ -2426,9 +2426,9 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
                 k = std::min(k, spare / c->b.nsites);
         }
         if (k < 1) {
-            for (mmca_ctx *c : bt->dom)
-                if (lean && done > 0 && c->hc.status == MMCA_OK)
-                    TRY(settle_all(c, bt->cur, bt->stream));
+            for (size_t d = 0; d < bt->dom.size(); d++)
+                if (lean && done > 0 && bt->dom[d]->hc.status == MMCA_OK)
+                    TRY(settle_all(bt->view.dom + d, bt->cur, bt->stream));
             return MMCA_ERR_STATE;
         }
         long long n = 0;
@@ -2455,7 +2455,7 @@ int mmca_batch_step(mmca_batch *bt, int nsteps, int want_sums, mmca_report *repo
         mmca_ctx *c = bt->dom[d];
         c->cur = c->hc.status == MMCA_OK ? bt->cur : start[d].first ^ (int) ((c->hc.timestep - start[d].second) & 1);
         if (lean && c->hc.status != MMCA_OK && c->hc.failed_step > start[d].second + 1)
-            HIPCHK(launch_settle(c->b, c->c, c->cur, (unsigned) c->hc.failed_step, bt->stream));
+            HIPCHK(launch_settle(bt->view.dom + d, c->cur, (unsigned) c->hc.failed_step, bt->stream));
         if (want_sums)
             HIPCHK(launch_reduce(c->b, c->c, c->cur, bt->d_sums + 2 * d, bt->stream));
     }

@@ -1361,8 +1361,10 @@ k_wake_all(View V)
 // written.  The tiles that finished that step left it as cl in the buffer
 // `cur`, the others in the one before.
 __global__ void __launch_bounds__(256)
-k_settle(DevBufs b, Consts c, int cur, unsigned failed)
+k_settle(const DomainDesc *dom, int cur, unsigned failed)
 {
+    const DevBufs b = dom->b;         // private copies: stores cannot alias them
+    const Consts c = dom->c;          // the tiles of the steps, whatever was set on the context since
     const unsigned ntx = (unsigned) (c.nx + 63) / 64, nty = (unsigned) (c.ny + c.zm_by - 1) / c.zm_by;
     const long long N = (long long) c.nx * c.ny * c.nz;
     for (long long i = (long long) blockIdx.x * 256 + threadIdx.x; i < N; i += 256ll * gridDim.x)
@@ -2582,9 +2584,9 @@ hipError_t launch_wake_all(const View &v, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_settle(const DevBufs &b, const Consts &c, int cur, unsigned failed, hipStream_t s)
+hipError_t launch_settle(const DomainDesc *dom, int cur, unsigned failed, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_settle, dim3(1024), dim3(256), 0, s, b, c, cur, failed);
+    hipLaunchKernelGGL(k_settle, dim3(1024), dim3(256), 0, s, dom, cur, failed);
     return hipGetLastError();
 }
 
