@@ -24,8 +24,11 @@ hipError_t launch_nucleate(const View &v, int mode, int cur, hipStream_t s);
 hipError_t launch_solute(const View &v, int am, int f32, int zm_by, int diff, int fsc, int rec, int cur, int nxt,
                          hipStream_t s);
 hipError_t launch_beam_nodes(const DevBufs &b, const Consts &c, hipStream_t s);
-hipError_t launch_beam_field(const DevBufs &b, const Consts &c, const BeamSet &p, int out, int adv, int rows,
-                             hipStream_t s);
+hipError_t launch_beam_field(const BeamView &v, int adv, int rows, hipStream_t s);
+hipError_t launch_beam_output(const BeamView &v, const Consts &c, const BeamSet &p, hipStream_t s);
+long long beam_x_blocks(const Consts &c, int rank);
+long long beam_row_blocks(const Consts &c);
+long long beam_field_blocks(const Consts &c);
 hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStream_t s);
 hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s);
 long long tile_slots(const Consts &c);
@@ -129,6 +132,7 @@ struct mmca_ctx {
     DomainDesc *d_desc = nullptr;
     long long *d_off = nullptr;
     View view;
+    BeamView beam_view;
     bool view_dirty = true;
     // kernel timing
     bool timing = false;
@@ -391,28 +395,19 @@ int ensure_beam(mmca_ctx *ctx)
     return make_beam_set(ctx, c.beam_rank, &ctx->beam_step);
 }
 
-// the approximate beam temperature of timestep + adv, before the kernels that read it
-int refresh_beam(mmca_ctx *ctx, int adv, hipStream_t s)
+// the approximate beam temperature of timestep + adv in the n domains of a view,
+// before the kernels that read it
+int refresh_beam(mmca_ctx *const *ctxs, size_t n, const BeamView &view, int adv, hipStream_t s)
 {
-    if (!ctx->c.am)
+    if (!ctxs[0]->c.am)
         return MMCA_OK;
     // the row factors change with the track only
-    HIPCHK(launch_beam_field(ctx->b, ctx->c, ctx->beam_step, 0, adv, ctx->c.am_tracks > 1 || !ctx->beam_rows, s));
-    ctx->beam_rows = true;
-    return MMCA_OK;
-}
-
-// the temperature of a beam block at the current timestep into b.temp, halo included
-int beam_output(mmca_ctx *ctx)
-{
-    if (!ctx->b.temp)
-        TRY(dev_alloc(&ctx->b.temp, (size_t) ctx->c.P));
-    if (ctx->c.beam_sep) {
-        if (!ctx->beam_out.key)
-            TRY(make_beam_set(ctx, BEAM_NT, &ctx->beam_out));
-        HIPCHK(launch_beam_field(ctx->b, ctx->c, ctx->beam_out, 1, 0, 1, ctx->stream));
-    }
-    HIPCHK(launch_fill_temp(ctx->b, ctx->c, ctx->b.temp, ctx->stream));
+    int rows = 0;
+    for (size_t d = 0; d < n; d++)
+        rows |= ctxs[d]->c.am_tracks > 1 || !ctxs[d]->beam_rows;
+    HIPCHK(launch_beam_field(view, adv, rows, s));
+    for (size_t d = 0; d < n; d++)
+        ctxs[d]->beam_rows = true;
     return MMCA_OK;
 }
 
@@ -430,7 +425,7 @@ int zm_rows(const Consts &c)
 // Upload the descriptors of n domains and the per-kernel workgroup prefix
 // tables; fills `v`.  `desc`/`off` are (re)allocated to hold n domains.
 int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDesc **desc, long long **off,
-               int *cap, View *v, hipStream_t s)
+               int *cap, View *v, BeamView *bv, hipStream_t s)
 {
     if (*cap < n) {
         if (*desc)
@@ -440,22 +435,28 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
         *desc = nullptr;
         *off = nullptr;
         TRY(dev_alloc(desc, (size_t) n));
-        TRY(dev_alloc(off, (size_t) 6 * (n + 1)));
+        TRY(dev_alloc(off, (size_t) 9 * (n + 1)));
         *cap = n;
     }
     std::vector<DomainDesc> h(n);
-    std::vector<long long> t((size_t) 6 * (n + 1), 0);
+    std::vector<long long> t((size_t) 9 * (n + 1), 0);
     long long *on = &t[0], *oz = &t[n + 1], *oc = &t[2 * (n + 1)], *ol = &t[3 * (n + 1)], *ok = &t[4 * (n + 1)],
-              *op = &t[5 * (n + 1)];
+              *op = &t[5 * (n + 1)], *ox = &t[6 * (n + 1)], *ow = &t[7 * (n + 1)], *of = &t[8 * (n + 1)];
     for (int d = 0; d < n; d++) {
         h[d].b = ctxs[d]->b;
         h[d].c = ctxs[d]->c;
+        h[d].beam = ctxs[d]->beam_step;
         on[d + 1] = on[d] + nuc_blocks(ctxs[d]->b.nsites);
         oz[d + 1] = oz[d] + (zm_by > 0 ? zm_tiles(ctxs[d]->c, zm_by) : 0);
         oc[d + 1] = oc[d] + cell_blocks(ctxs[d]->c);
         ol[d + 1] = ol[d] + list_blocks(ctxs[d]->c);
         ok[d + 1] = ok[d] + count_blocks(ctxs[d]->c);
         op[d + 1] = op[d] + capture_blocks(ctxs[d]->c);
+        if (ctxs[d]->c.am) {
+            ox[d + 1] = ox[d] + beam_x_blocks(ctxs[d]->c, ctxs[d]->beam_step.rank);
+            ow[d + 1] = ow[d] + beam_row_blocks(ctxs[d]->c);
+            of[d + 1] = of[d] + beam_field_blocks(ctxs[d]->c);
+        }
     }
     HIPCHK(hipMemcpyAsync(*desc, h.data(), sizeof(DomainDesc) * (size_t) n, hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(*off, t.data(), sizeof(long long) * t.size(), hipMemcpyHostToDevice, s));
@@ -478,6 +479,7 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
     v->tot_list = ol[n];
     v->tot_count = ok[n];
     v->tot_cap = op[n];
+    *bv = { *desc, n, *off + 6 * (n + 1), *off + 7 * (n + 1), *off + 8 * (n + 1), ox[n], ow[n], of[n] };
     return MMCA_OK;
 }
 
@@ -487,9 +489,26 @@ int ensure_view(mmca_ctx *ctx)
         return MMCA_OK;
     int cap = ctx->d_desc ? 1 : 0;
     mmca_ctx *one[1] = { ctx };
-    TRY(build_view(one, 1, ctx->c.xcd_remap, zm_rows(ctx->c), &ctx->d_desc, &ctx->d_off, &cap, &ctx->view,
+    TRY(build_view(one, 1, ctx->c.xcd_remap, zm_rows(ctx->c), &ctx->d_desc, &ctx->d_off, &cap, &ctx->view, &ctx->beam_view,
                    ctx->stream));
     ctx->view_dirty = false;
+    return MMCA_OK;
+}
+
+// the temperature of a beam block at the current timestep into b.temp, halo included
+int beam_output(mmca_ctx *ctx)
+{
+    if (!ctx->b.temp) {
+        TRY(dev_alloc(&ctx->b.temp, (size_t) ctx->c.P));
+        ctx->view_dirty = true;
+    }
+    if (ctx->c.beam_sep) {
+        if (!ctx->beam_out.key)
+            TRY(make_beam_set(ctx, BEAM_NT, &ctx->beam_out));
+        TRY(ensure_view(ctx));
+        HIPCHK(launch_beam_output(ctx->beam_view, ctx->c, ctx->beam_out, ctx->stream));
+    }
+    HIPCHK(launch_fill_temp(ctx->b, ctx->c, ctx->b.temp, ctx->stream));
     return MMCA_OK;
 }
 
@@ -550,7 +569,7 @@ int enqueue_iteration(mmca_ctx *ctx, bool advance, int lean)
     const int nxt = ctx->cur ^ 1;
     TRY(ensure_view(ctx));
     ctx->view.lean = lean;
-    TRY(refresh_beam(ctx, advance ? 1 : 0, ctx->stream));
+    TRY(refresh_beam(&ctx, 1, ctx->beam_view, advance ? 1 : 0, ctx->stream));
     HIPCHK(launch_nucleate(ctx->view, advance ? 7 : 3, ctx->cur, ctx->stream));
     const size_t ev0 = ctx->ev_used;
     if (ctx->timing) {
@@ -1084,7 +1103,7 @@ int mmca_cell_nucleation(mmca_ctx *ctx, int32_t *n_new)
         return MMCA_ERR_ARG;
     HIPCHK(hipSetDevice(ctx->device));
     TRY(ensure_view(ctx));
-    TRY(refresh_beam(ctx, 0, ctx->stream));
+    TRY(refresh_beam(&ctx, 1, ctx->beam_view, 0, ctx->stream));
     HIPCHK(launch_nucleate(ctx->view, 1, ctx->cur, ctx->stream));
     TRY(sync_counters(ctx));
     if (n_new)
@@ -1954,6 +1973,7 @@ struct mmca_batch {
     long long *d_off = nullptr;
     int cap = 0;
     View view;
+    BeamView beam_view;
     bool view_dirty = true;
     // counters of all domains: gathered on the device, and their pinned copy
     Counters *d_cnt = nullptr, *h_cnt = nullptr;
@@ -1990,7 +2010,7 @@ int batch_view(mmca_batch *bt)
         c->view_dirty = true;
     }
     TRY(build_view(bt->dom.data(), (int) bt->dom.size(), bt->xcd_remap, bt->zm_planes > 0 ? bt->zm_by : 0,
-                   &bt->d_desc, &bt->d_off, &bt->cap, &bt->view, bt->stream));
+                   &bt->d_desc, &bt->d_off, &bt->cap, &bt->view, &bt->beam_view, bt->stream));
     for (int p = 0; p < 6; p++)
         if (bt->graph[p]) {
             (void) hipGraphExecDestroy(bt->graph[p]);
@@ -2032,8 +2052,7 @@ int batch_enqueue(mmca_batch *bt, int cur, int lean)
     bt->view.lean = lean;
     const Consts &c0 = bt->dom[0]->c;
     const int nxt = cur ^ 1;
-    for (mmca_ctx *c : bt->dom)
-        TRY(refresh_beam(c, 1, bt->stream));
+    TRY(refresh_beam(bt->dom.data(), bt->dom.size(), bt->beam_view, 1, bt->stream));
     if (bt->coupled) {
         HIPCHK(launch_halo_exchange(bt->view, 0, cur, bt->max_face, bt->stream));
         HIPCHK(launch_nucleate_coupled(bt->view, cur, bt->stream));

@@ -155,6 +155,7 @@ struct BeamSet {
 struct DomainDesc {
     DevBufs b;
     Consts c;
+    BeamSet beam;                // of the approximate temperature (beam blocks)
 };
 
 // The domains advanced by one launch.  Workgroup w of a kernel belongs to
@@ -178,6 +179,15 @@ struct View {
     const long long *off_count;  // list count workgroups
     const long long *off_cap;    // capture workgroups
     long long tot_nuc, tot_zm, tot_cell, tot_list, tot_count, tot_cap;
+};
+
+// The domains of a launch as the kernels of the approximate beam temperature
+// see them (apart from View, whose size every launch of a step pays for).
+struct BeamView {
+    const DomainDesc *dom;
+    int ndom;
+    const long long *off_ax, *off_aw, *off_field;    // workgroups of k_beam_ax, _aw and _field
+    long long tot_ax, tot_aw, tot_field;
 };
 
 }  // namespace mmca

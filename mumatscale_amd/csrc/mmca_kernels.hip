@@ -2040,15 +2040,26 @@ k_beam_nodes(DevBufs b, Consts c)
     }
 }
 
-// x factors at the interpolation nodes for timestep cnt->timestep + adv; says
-// in beam_key[1] whether the row factors have to be built for a new track, and
-// empties the list of waiting cells
+// The next three kernels take all domains of a view in one launch: a step of 64
+// blocks of 20 x 18 x 16 cells takes 62 us, and took 920 with launches for each
+// domain (256 blocks of 12^3: 98 and 3020).  A step uses the points of each
+// domain's description; an output (OUT) of one block the points `out`.
+//
+// x factors at the interpolation points for timestep cnt->timestep + adv; says
+// in BeamSet::key[1] whether the row factors have to be built for a new track,
+// and empties the list of waiting cells
+template <bool OUT>
 __global__ void __launch_bounds__(256)
-k_beam_ax(DevBufs b, Consts c, BeamSet p, int adv)
+k_beam_ax(BeamView V, BeamSet out, int adv)
 {
+    const int dm = OUT ? 0 : find_dom(V.off_ax, V.ndom, blockIdx.x);
+    const int blk = (int) blockIdx.x - (OUT ? 0 : (int) V.off_ax[dm]);
+    const DevBufs b = V.dom[dm].b;    // private copies: stores cannot alias them
+    const Consts c = V.dom[dm].c;
+    const BeamSet p = OUT ? out : V.dom[dm].beam;
     const double sim_time = (G(b.cnt)->timestep + (unsigned long long) adv) * c.dt;
     const BeamNow bn = beam_now(c, sim_time);
-    if (blockIdx.x == 0 && threadIdx.x == 0)
+    if (blk == 0 && threadIdx.x == 0)
     {
         const double held = G(p.key)[0];
         G(p.key)[1] = __double_as_longlong(held) == __double_as_longlong(bn.ynow) ? 0.0 : 1.0;
@@ -2057,7 +2068,7 @@ k_beam_ax(DevBufs b, Consts c, BeamSet p, int adv)
     }
     const double ls = c.lsd / (2. * 1.414);
     const double lalpha = beam_lalpha(c);
-    const int e = blockIdx.x * 256 + threadIdx.x, xp = beam_x_pitch(c);
+    const int e = blk * 256 + threadIdx.x, xp = beam_x_pitch(c);
     const int j = e / xp, q = e - j * xp;
     if (j >= p.rank)
         return;
@@ -2069,14 +2080,20 @@ k_beam_ax(DevBufs b, Consts c, BeamSet p, int adv)
 
 // row factors: one workgroup per (z, y) row; 16 groups of 16 threads share the
 // nodes, each thread sums for one interpolation point at a time
+template <bool OUT>
 __global__ void __launch_bounds__(256)
-k_beam_aw(DevBufs b, Consts c, BeamSet p)
+k_beam_aw(BeamView V, BeamSet out)
 {
     __shared__ double s_w[BEAM_NT];
     __shared__ double s_p[16][17];
+    const int dm = OUT ? 0 : find_dom(V.off_aw, V.ndom, blockIdx.x);
+    const unsigned row = blockIdx.x - (OUT ? 0u : (unsigned) V.off_aw[dm]);
+    const DevBufs b = V.dom[dm].b;
+    const Consts c = V.dom[dm].c;
+    const BeamSet p = OUT ? out : V.dom[dm].beam;
     if (G(p.key)[1] == 0.0)
         return;
-    const int z = (int) (blockIdx.x / (unsigned) c.ny), y = (int) (blockIdx.x - (unsigned) z * (unsigned) c.ny);
+    const int z = (int) (row / (unsigned) c.ny), y = (int) (row - (unsigned) z * (unsigned) c.ny);
     const double ldt = beam_ldt(c);
     const double ry = c.origin[1] + ((c.off[1] + y + 1) + 0.5) * c.cell_size;
     const double ly = ry - G(p.key)[0];
@@ -2087,7 +2104,7 @@ k_beam_aw(DevBufs b, Consts c, BeamSet p)
     if (!p.weights)
     {
         for (int i = threadIdx.x; i < BEAM_NT; i += 256)
-            G(p.aw)[(long long) blockIdx.x * BEAM_NT + i] = s_w[i];
+            G(p.aw)[(long long) row * BEAM_NT + i] = s_w[i];
         return;
     }
     const int jj = threadIdx.x & 15, g = threadIdx.x >> 4;
@@ -2103,7 +2120,7 @@ k_beam_aw(DevBufs b, Consts c, BeamSet p)
             double t = 0.0;
             for (int q = 0; q < 16; ++q)
                 t += s_p[q][jj];
-            G(p.aw)[(long long) blockIdx.x * p.rank + j0 + jj] = t;
+            G(p.aw)[(long long) row * p.rank + j0 + jj] = t;
         }
         __syncthreads();
     }
@@ -2125,17 +2142,22 @@ typedef double dvec4 __attribute__((ext_vector_type(4)));
 
 template <bool OUT>
 __global__ void __launch_bounds__(256)
-k_beam_field(DevBufs b, Consts c, BeamSet p, int adv)
+k_beam_field(BeamView V, BeamSet out, int adv)
 {
+    const int dm = OUT ? 0 : find_dom(V.off_field, V.ndom, blockIdx.x);
+    const unsigned blk = blockIdx.x - (OUT ? 0u : (unsigned) V.off_field[dm]);
+    const DevBufs b = V.dom[dm].b;
+    const Consts c = V.dom[dm].c;
+    const BeamSet p = OUT ? out : V.dom[dm].beam;
     const MMCA_GLOBAL Counters *cnt = G(b.cnt);
     if (!OUT && cnt->status != MMCA_OK)
         return;                                   // uniform over the workgroup; an output is one of a stopped block too
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int xp = beam_x_pitch(c), K = p.rank;
-    const unsigned ntx = (unsigned) (xp / BF_COLS), slab = blockIdx.x / ntx;
+    const unsigned ntx = (unsigned) (xp / BF_COLS), slab = blk / ntx;
     const long long q0 = (long long) slab * BF_ROWS;
-    const int x0 = (int) (blockIdx.x - slab * ntx) * BF_COLS + wave * 32;      // 0-based interior column
+    const int x0 = (int) (blk - slab * ntx) * BF_COLS + wave * 32;      // 0-based interior column
     const int kk = lane >> 4, lr = lane & 15;
     const double sim_time = (cnt->timestep + (unsigned long long) adv) * c.dt;
     const BeamNow bn = beam_now(c, sim_time);
@@ -2331,21 +2353,29 @@ hipError_t launch_beam_nodes(const DevBufs &b, const Consts &c, hipStream_t s)
     return hipGetLastError();
 }
 
-// The beam temperature of timestep cnt->timestep + adv from the point set p,
-// in double into b.temp (out) or rounded into b.temp32; the row factors too
-// when `rows` (they may be stale)
-hipError_t launch_beam_field(const DevBufs &b, const Consts &c, const BeamSet &p, int out, int adv, int rows,
-                             hipStream_t s)
+long long beam_x_blocks(const Consts &c, int rank) { return ((long long) rank * beam_x_pitch(c) + 255) / 256; }
+long long beam_row_blocks(const Consts &c) { return (long long) c.ny * c.nz; }
+long long beam_field_blocks(const Consts &c) { return beam_x_pitch(c) / BF_COLS * (beam_w_rows(c) / BF_ROWS); }
+
+// The approximate beam temperature of timestep cnt->timestep + adv into b.temp32
+// of every domain; the row factors too when `rows` (they may be stale)
+hipError_t launch_beam_field(const BeamView &v, int adv, int rows, hipStream_t s)
 {
-    const long long n = (long long) p.rank * beam_x_pitch(c);
-    hipLaunchKernelGGL(k_beam_ax, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, b, c, p, adv);
+    const BeamSet none = {};
+    hipLaunchKernelGGL(k_beam_ax<false>, dim3((unsigned) v.tot_ax), dim3(256), 0, s, v, none, adv);
     if (rows)
-        hipLaunchKernelGGL(k_beam_aw, dim3((unsigned) ((long long) c.ny * c.nz)), dim3(256), 0, s, b, c, p);
-    const dim3 grid((unsigned) (beam_x_pitch(c) / BF_COLS * (beam_w_rows(c) / BF_ROWS)));
-    if (out)
-        hipLaunchKernelGGL(k_beam_field<true>, grid, dim3(256), 0, s, b, c, p, adv);
-    else
-        hipLaunchKernelGGL(k_beam_field<false>, grid, dim3(256), 0, s, b, c, p, adv);
+        hipLaunchKernelGGL(k_beam_aw<false>, dim3((unsigned) v.tot_aw), dim3(256), 0, s, v, none);
+    hipLaunchKernelGGL(k_beam_field<false>, dim3((unsigned) v.tot_field), dim3(256), 0, s, v, none, adv);
+    return hipGetLastError();
+}
+
+// The temperature of timestep cnt->timestep into b.temp of a view's only domain,
+// from the point set p
+hipError_t launch_beam_output(const BeamView &v, const Consts &c, const BeamSet &p, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_beam_ax<true>, dim3((unsigned) beam_x_blocks(c, p.rank)), dim3(256), 0, s, v, p, 0);
+    hipLaunchKernelGGL(k_beam_aw<true>, dim3((unsigned) beam_row_blocks(c)), dim3(256), 0, s, v, p);
+    hipLaunchKernelGGL(k_beam_field<true>, dim3((unsigned) beam_field_blocks(c)), dim3(256), 0, s, v, p, 0);
     return hipGetLastError();
 }
 

@@ -1,0 +1,107 @@
+"""Batches of Gaussian-beam blocks of uneven sizes, with and without graphs,
+against the same blocks stepped alone, bit for bit; FP32 storage over the
+cell-parallel kernel and tiles that hold more waiting cells than their buffer;
+and that the launches of a step do not grow with the domains."""
+import time
+
+import numpy as np
+import pytest
+
+from mumatscale_amd import abi
+from mumatscale_amd.lib import Batch, Subblock
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = (abi.FIELD_CE, abi.FIELD_CL, abi.FIELD_FS, abi.FIELD_GR, abi.FIELD_DC)
+#        dims, tracks, speed, spot: 32, 32, 400 and 48 or more interpolation points
+BLOCKS = [((70, 37, 21), 1, 0.8, 130e-6), ((13, 9, 33), 2, 0.8, 130e-6), ((129, 5, 8), 1, 0.05, 20e-6),
+          ((64, 64, 16), 2, 0.5, 30e-6)]
+
+
+def _cfg(dims, tracks, speed, spot):
+    from mumatscale_amd.workloads import am_track_config
+    cfg = am_track_config(*dims)
+    cfg.cell_size, cfg.dt = 1.0e-6, 2.0e-6
+    cfg.am_tracks = tracks
+    cfg.laser.update(power=60.0 if spot > 1e-4 else 8.0, speed=speed, spot=spot, hatch=9e-6, sub_init_temp=600.0,
+                     start=[0.0, dims[1] * 0.5e-6, dims[2] * 1.0e-6])
+    return cfg
+
+
+def _fill(sb, cfg, fs0):
+    from mumatscale_amd.workloads import voronoi_substrate
+    gr, recs = voronoi_substrate(cfg, 20, 5)
+    fs = np.zeros(gr.shape)
+    fs[1:-1, 1:-1, 1:-1] = fs0
+    sb.set_grains(recs)
+    sb.upload(abi.FIELD_GR, gr)
+    sb.upload(abi.FIELD_FS, fs)
+
+
+def _same(a, b, where):
+    for f in FIELDS:
+        x, y = a.download(f), b.download(f)
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (where, f)
+
+
+@pytest.mark.parametrize("graph", [0, 1], ids=["launches", "graph"])
+@pytest.mark.parametrize("prec", [abi.PREC_FP64, abi.PREC_FP32DEV], ids=["fp64", "fp32"])
+def test_batch_matches_blocks_alone(prec, graph):
+    cfgs = [_cfg(*b) for b in BLOCKS]
+    params = [c.params(check_negative_ce=False, precision=prec) for c in cfgs]
+    nucs = [c.nucleation() for c in cfgs]
+    with Batch(params, nucs) as bt:
+        bt.set_tuning(abi.TUNE_GRAPH, graph)
+        for sb, c in zip(bt.domains, cfgs):
+            _fill(sb, c, 1.0)
+        alone = [Subblock(p, n) for p, n in zip(params, nucs)]
+        for sb, c in zip(alone, cfgs):
+            _fill(sb, c, 1.0)
+        for n in (1, 50, 60, 23):                    # the beam turns on at step 50
+            bt.step(n)
+            for d, sb in enumerate(alone):
+                sb.step(n)
+                _same(bt.domains[d], sb, (n, d))
+                assert np.array_equal(bt.domains[d].download(abi.FIELD_TEMP), sb.download(abi.FIELD_TEMP)), (n, d)
+        for sb, c in zip(alone, cfgs):
+            sb.close()
+
+
+@pytest.mark.parametrize("block", BLOCKS, ids=["x".join(map(str, b[0])) for b in BLOCKS])
+@pytest.mark.parametrize("fs0", [1.0, 0.5], ids=["solid", "mushy"])
+def test_fp32_tiles_match_the_cell_parallel_kernel(block, fs0):
+    """Mushy: every cell waits, 8192 of a 16 x 8 tile, of which the buffer holds 2048."""
+    cfg = _cfg(*block)
+    want = None
+    for planes, rows in ((0, 4), (16, 8), (16, 16), (1, 4), (8, 4)):
+        with Subblock(cfg.params(check_negative_ce=False, precision=abi.PREC_FP32DEV), cfg.nucleation()) as sb:
+            sb.set_tuning(abi.TUNE_ZM_PLANES, planes)
+            sb.set_tuning(abi.TUNE_ZM_ROWS, rows)
+            _fill(sb, cfg, fs0)
+            sb.step(110)
+            got = [sb.download(f) for f in FIELDS]
+        if want is None:
+            want = got
+            assert not np.all(got[2][1:-1, 1:-1, 1:-1] == fs0)
+        for f, a, b in zip(FIELDS, got, want):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), (planes, rows, f)
+
+
+@pytest.mark.parametrize("prec", [abi.PREC_FP64, abi.PREC_FP32DEV], ids=["fp64", "fp32"])
+def test_step_of_many_small_blocks(prec):
+    """A step of 64 small blocks in a batch against a step of one of them: a
+    set of launches for each block took 20 times as long."""
+    cfg = _cfg((20, 18, 16), 1, 0.8, 130e-6)
+    t = {}
+    for n in (1, 64):
+        with Batch([cfg.params(check_negative_ce=False, precision=prec)] * n, [cfg.nucleation()] * n) as bt:
+            for sb in bt.domains:
+                _fill(sb, cfg, 1.0)
+            bt.step(70)
+            best = 1e9
+            for _ in range(5):
+                a = time.perf_counter()
+                bt.step(50)
+                best = min(best, time.perf_counter() - a)
+            t[n] = best
+    assert t[64] < 8 * t[1], t
