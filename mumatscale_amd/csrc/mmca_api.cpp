@@ -27,7 +27,7 @@ hipError_t launch_beam_nodes(const DevBufs &b, const Consts &c, hipStream_t s);
 hipError_t launch_beam_field(const BeamView &v, int adv, int rows, hipStream_t s);
 hipError_t launch_beam_output(const BeamView &v, const Consts &c, const BeamSet &p, hipStream_t s);
 long long beam_x_blocks(const Consts &c, int rank);
-long long beam_row_blocks(const Consts &c);
+long long beam_rows(const Consts &c);
 long long beam_field_blocks(const Consts &c);
 hipError_t launch_beam_finish(const View &v, int f32, int cur, int nxt, hipStream_t s);
 hipError_t launch_mask_from_gr(const DevBufs &b, const Consts &c, hipStream_t s);
@@ -454,7 +454,7 @@ int build_view(mmca_ctx *const *ctxs, int n, int xcd_remap, int zm_by, DomainDes
         op[d + 1] = op[d] + capture_blocks(ctxs[d]->c);
         if (ctxs[d]->c.am) {
             ox[d + 1] = ox[d] + beam_x_blocks(ctxs[d]->c, ctxs[d]->beam_step.rank);
-            ow[d + 1] = ow[d] + beam_row_blocks(ctxs[d]->c);
+            ow[d + 1] = ow[d] + beam_rows(ctxs[d]->c);
             of[d + 1] = of[d] + beam_field_blocks(ctxs[d]->c);
         }
     }

@@ -186,7 +186,7 @@ struct View {
 struct BeamView {
     const DomainDesc *dom;
     int ndom;
-    const long long *off_ax, *off_aw, *off_field;    // workgroups of k_beam_ax, _aw and _field
+    const long long *off_ax, *off_aw, *off_field;    // workgroups of k_beam_ax and _field, rows of k_beam_aw
     long long tot_ax, tot_aw, tot_field;
 };
 

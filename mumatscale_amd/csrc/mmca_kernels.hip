@@ -2078,51 +2078,55 @@ k_beam_ax(BeamView V, BeamSet out, int adv)
     G(p.ax)[e] = q < c.nx ? exp(-(u * u) / (ls * ls + 4. * lalpha * t)) : 0.0;   // columns past nx pad the row
 }
 
-// row factors: one workgroup per (z, y) row; 16 groups of 16 threads share the
-// nodes, each thread sums for one interpolation point at a time
+// row factors: one workgroup per (z, y) row at a time; 16 groups of 16 threads
+// share the nodes, each thread sums for one interpolation point at a time
 template <bool OUT>
 __global__ void __launch_bounds__(256)
 k_beam_aw(BeamView V, BeamSet out)
 {
     __shared__ double s_w[BEAM_NT];
     __shared__ double s_p[16][17];
-    const int dm = OUT ? 0 : find_dom(V.off_aw, V.ndom, blockIdx.x);
-    const unsigned row = blockIdx.x - (OUT ? 0u : (unsigned) V.off_aw[dm]);
-    const DevBufs b = V.dom[dm].b;
-    const Consts c = V.dom[dm].c;
-    const BeamSet p = OUT ? out : V.dom[dm].beam;
-    if (G(p.key)[1] == 0.0)
-        return;
-    const int z = (int) (row / (unsigned) c.ny), y = (int) (row - (unsigned) z * (unsigned) c.ny);
-    const double ldt = beam_ldt(c);
-    const double ry = c.origin[1] + ((c.off[1] + y + 1) + 0.5) * c.cell_size;
-    const double ly = ry - G(p.key)[0];
-    for (int i = threadIdx.x; i < BEAM_NT; i += 256)
-        s_w[i] = ldt / G(b.beam_nodes)[BN_TL * BEAM_NT + i] *
-                 exp(-(ly * ly) / G(b.beam_nodes)[BN_A * BEAM_NT + i] - G(b.beam_zq)[(long long) (z + 1) * BEAM_NT + i]);
-    __syncthreads();
-    if (!p.weights)
-    {
-        for (int i = threadIdx.x; i < BEAM_NT; i += 256)
-            G(p.aw)[(long long) row * BEAM_NT + i] = s_w[i];
-        return;
-    }
     const int jj = threadIdx.x & 15, g = threadIdx.x >> 4;
-    for (int j0 = 0; j0 < p.rank; j0 += 16)
+    for (long long w = blockIdx.x; w < V.tot_aw; w += gridDim.x)
     {
-        double v = 0.0;
-        for (int i = g; i < BEAM_NT; i += 16)
-            v += s_w[i] * G(p.weights)[(long long) i * p.rank + j0 + jj];
-        s_p[g][jj] = v;
+        const int dm = OUT ? 0 : find_dom(V.off_aw, V.ndom, w);
+        const long long row = w - (OUT ? 0 : V.off_aw[dm]);
+        const DevBufs b = V.dom[dm].b;
+        const Consts c = V.dom[dm].c;
+        const BeamSet p = OUT ? out : V.dom[dm].beam;
+        if (G(p.key)[1] == 0.0)
+            continue;                             // uniform over the workgroup
+        const int z = (int) (row / c.ny), y = (int) (row - (long long) z * c.ny);
+        const double ldt = beam_ldt(c);
+        const double ry = c.origin[1] + ((c.off[1] + y + 1) + 0.5) * c.cell_size;
+        const double ly = ry - G(p.key)[0];
+        const MMCA_GLOBAL double *node = G(b.beam_nodes), *zq = G(b.beam_zq) + (long long) (z + 1) * BEAM_NT;
+        __syncthreads();                          // the row before has been read
+        for (int i = threadIdx.x; i < BEAM_NT; i += 256)
+            s_w[i] = ldt / node[BN_TL * BEAM_NT + i] * exp(-(ly * ly) / node[BN_A * BEAM_NT + i] - zq[i]);
         __syncthreads();
-        if (g == 0)
+        if (!p.weights)
         {
-            double t = 0.0;
-            for (int q = 0; q < 16; ++q)
-                t += s_p[q][jj];
-            G(p.aw)[(long long) row * p.rank + j0 + jj] = t;
+            for (int i = threadIdx.x; i < BEAM_NT; i += 256)
+                G(p.aw)[row * BEAM_NT + i] = s_w[i];
+            continue;
         }
-        __syncthreads();
+        for (int j0 = 0; j0 < p.rank; j0 += 16)
+        {
+            double v = 0.0;
+            for (int i = g; i < BEAM_NT; i += 16)
+                v += s_w[i] * G(p.weights)[(long long) i * p.rank + j0 + jj];
+            s_p[g][jj] = v;
+            __syncthreads();
+            if (g == 0)
+            {
+                double t = 0.0;
+                for (int q = 0; q < 16; ++q)
+                    t += s_p[q][jj];
+                G(p.aw)[row * p.rank + j0 + jj] = t;
+            }
+            __syncthreads();
+        }
     }
 }
 
@@ -2354,8 +2358,11 @@ hipError_t launch_beam_nodes(const DevBufs &b, const Consts &c, hipStream_t s)
 }
 
 long long beam_x_blocks(const Consts &c, int rank) { return ((long long) rank * beam_x_pitch(c) + 255) / 256; }
-long long beam_row_blocks(const Consts &c) { return (long long) c.ny * c.nz; }
+long long beam_rows(const Consts &c) { return (long long) c.ny * c.nz; }
 long long beam_field_blocks(const Consts &c) { return beam_x_pitch(c) / BF_COLS * (beam_w_rows(c) / BF_ROWS); }
+
+// a launch takes less than 2^32 threads; a block of 2^24 rows would need more
+static dim3 aw_grid(const BeamView &v) { return dim3((unsigned) std::min<long long>(v.tot_aw, 65536)); }
 
 // The approximate beam temperature of timestep cnt->timestep + adv into b.temp32
 // of every domain; the row factors too when `rows` (they may be stale)
@@ -2364,7 +2371,7 @@ hipError_t launch_beam_field(const BeamView &v, int adv, int rows, hipStream_t s
     const BeamSet none = {};
     hipLaunchKernelGGL(k_beam_ax<false>, dim3((unsigned) v.tot_ax), dim3(256), 0, s, v, none, adv);
     if (rows)
-        hipLaunchKernelGGL(k_beam_aw<false>, dim3((unsigned) v.tot_aw), dim3(256), 0, s, v, none);
+        hipLaunchKernelGGL(k_beam_aw<false>, aw_grid(v), dim3(256), 0, s, v, none);
     hipLaunchKernelGGL(k_beam_field<false>, dim3((unsigned) v.tot_field), dim3(256), 0, s, v, none, adv);
     return hipGetLastError();
 }
@@ -2374,7 +2381,7 @@ hipError_t launch_beam_field(const BeamView &v, int adv, int rows, hipStream_t s
 hipError_t launch_beam_output(const BeamView &v, const Consts &c, const BeamSet &p, hipStream_t s)
 {
     hipLaunchKernelGGL(k_beam_ax<true>, dim3((unsigned) beam_x_blocks(c, p.rank)), dim3(256), 0, s, v, p, 0);
-    hipLaunchKernelGGL(k_beam_aw<true>, dim3((unsigned) beam_row_blocks(c)), dim3(256), 0, s, v, p);
+    hipLaunchKernelGGL(k_beam_aw<true>, aw_grid(v), dim3(256), 0, s, v, p);
     hipLaunchKernelGGL(k_beam_field<true>, dim3((unsigned) beam_field_blocks(c)), dim3(256), 0, s, v, p, 0);
     return hipGetLastError();
 }

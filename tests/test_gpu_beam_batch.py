@@ -105,3 +105,36 @@ def test_step_of_many_small_blocks(prec):
                 best = min(best, time.perf_counter() - a)
             t[n] = best
     assert t[64] < 8 * t[1], t
+
+
+def test_more_rows_than_a_launch_has_workgroups():
+    """16.8 M rows along x, in workgroups of 256 threads: more threads than one
+    launch takes.  Against the recorded step (the quadrature in place), where
+    the beam melts cells in rows past the first 33 000."""
+    import torch
+    from mumatscale_amd.adjoint import record_bytes
+    n = 4100
+    cfg = _cfg((1, n, n), 1, 0.8, 130e-6)
+    recs = [abi.Grain(), abi.Grain()]
+    for q in range(3):
+        recs[1].rotmat[q][q] = 1.0
+    gr = np.zeros((n + 2, n + 2, 3), np.int32)
+    gr[1:-1, 1:-1, 1] = 1
+    want = None
+    for recorded in (True, False):
+        with Subblock(cfg.params(check_negative_ce=False), cfg.nucleation()) as sb:
+            sb.set_grains(recs)
+            sb.upload(abi.FIELD_GR, gr)
+            sb.upload(abi.FIELD_FS, gr.astype(np.float64))
+            sb.timestep = 60                         # the beam is on
+            if recorded:
+                codes = torch.zeros((2, record_bytes(sb.params)), dtype=torch.uint8, device="cuda")
+                torch.cuda.synchronize()
+                sb.set_record(codes.data_ptr(), 2)
+            sb.step(2)
+            got = [sb.download(f)[1:-1, 1:-1, 1] for f in (abi.FIELD_GR, abi.FIELD_FS)]
+        if want is None:
+            want = got
+            assert (want[0] <= 0).sum() > 1000
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
