@@ -2530,16 +2530,16 @@ int mmca_batch_autotune(const mmca_params *params, const mmca_nucleation_cfg *nu
     if (!params || ndomains < 1 || trial_steps < 1 || warmup < 0)
         return MMCA_ERR_ARG;
     // solute-kernel shapes tried: (planes per workgroup, rows); planes 0 is
-    // the cell-parallel kernel
-    static const int cand[][2] = { { 0, 4 }, { 8, 4 }, { 16, 4 }, { 8, 8 }, { 16, 8 }, { 32, 8 },
-                                   { 64, 8 }, { 16, 16 }, { 32, 16 }, { 64, 16 } };
+    // the cell-parallel kernel.  All shapes of default_tile are among them.
+    static const int cand[][2] = { { 0, 4 }, { 1, 4 }, { 2, 4 }, { 4, 4 }, { 8, 4 }, { 16, 4 }, { 8, 8 }, { 16, 8 },
+                                   { 32, 8 }, { 64, 8 }, { 16, 16 }, { 32, 16 }, { 64, 16 } };
     mmca_batch *bt = nullptr;
     int st = mmca_batch_create(params, nucleation, ndomains, device, &bt);
     if (st != MMCA_OK) {
         mmca_batch_destroy(bt);
         return st;
     }
-    int bp = 16, br = 8;
+    int bp = bt->zm_planes, br = bt->zm_by;
     double bms = 1e300;
     if (warmup > 0)
         st = mmca_batch_step(bt, warmup, 0, nullptr);
