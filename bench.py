@@ -69,7 +69,7 @@ def apply_shape(sb, shape):
     """Tile shape of a subblock or batch: the settings given (None: the
     library's default for its size)."""
     for key, name in ((abi.TUNE_ZM_PLANES, "zm"), (abi.TUNE_ZM_ROWS, "rows"), (abi.TUNE_XCD_REMAP, "xcd"),
-                      (abi.TUNE_CAPTURE_CHUNK, "chunk"), (abi.TUNE_CAPTURE_BAND, "band")):
+                      (abi.TUNE_ZM_LDS, "lds"), (abi.TUNE_CAPTURE_CHUNK, "chunk"), (abi.TUNE_CAPTURE_BAND, "band")):
         if shape.get(name) is not None:
             sb.set_tuning(key, shape[name])
 
@@ -552,6 +552,8 @@ def main():
                     help="rows per z-marching workgroup (4, 8, 16; default: the library's)")
     ap.add_argument("--xcd", type=int, default=None,
                     help="1: one contiguous run of tiles per XCD, 0: short runs (default: the library's)")
+    ap.add_argument("--lds", type=int, default=1,
+                    help="0 or 1: MMCA_TUNE_ZM_LDS, which selects nothing any more")
     ap.add_argument("--capture-chunk", type=int, default=0,
                     help=">0: capture deals its list slots in chunks of this many, pinned to XCDs")
     ap.add_argument("--capture-band", type=int, default=0,
@@ -576,7 +578,7 @@ def main():
               % args.gpus, file=sys.stderr)
         sys.exit(2)
     dims = tuple(int(v) for v in args.size.split("x"))
-    shape = {"zm": args.zm, "rows": args.zm_rows, "xcd": args.xcd, "chunk": args.capture_chunk,
+    shape = {"zm": args.zm, "rows": args.zm_rows, "xcd": args.xcd, "lds": args.lds, "chunk": args.capture_chunk,
              "band": args.capture_band}
     if args.capture_footprint:
         capture_footprint(shape)
@@ -680,7 +682,7 @@ def main():
                                                                                   "FP32-deviation" if fp32
                                                                                   else "plain FP64"),
                    "cells": n, "dt": cfg.dt, "zm_planes": used["zm"], "zm_rows": used["rows"],
-                   "xcd_remap": used["xcd"], "capture_chunk": args.capture_chunk,
+                   "xcd_remap": used["xcd"], "zm_lds": args.lds, "capture_chunk": args.capture_chunk,
                    "capture_band": args.capture_band,
                    "parallelism": "single GPU"},
         "roofline": roof,
