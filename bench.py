@@ -100,6 +100,21 @@ def liquid_rows(sb):
     return 1.0 - g.reshape(*g.shape[:2], -1, 64).any(-1).mean()
 
 
+def mean_liquid_rows(cfg, prec, shape, warmup, steps, samples=8):
+    """liquid_rows over the steps of a run, by the trapezoid rule over
+    `samples` intervals, from a second run of the same steps."""
+    from mumatscale_amd.lib import Subblock
+    with Subblock(cfg.params(check_negative_ce=True, precision=prec), cfg.nucleation(), device=0) as sb:
+        apply_shape(sb, shape)
+        sb.step(warmup)
+        at, vals, done = [round(steps * q / samples) for q in range(samples + 1)], [], 0
+        for t in at:
+            sb.step(t - done)
+            done = t
+            vals.append(liquid_rows(sb))
+    return sum((at[q + 1] - at[q]) * (vals[q] + vals[q + 1]) / 2 for q in range(samples)) / steps
+
+
 def run_ensemble(steps, baseline_steps):
     """Batched FP32-deviation step of the 96-domain ensemble (graph replay,
     autotuned tile) against the same domains stepped one at a time in plain
@@ -609,7 +624,8 @@ def main():
     n = nx * ny * nz
     if args.warmup:
         gpu.step(args.warmup)
-    rows = liquid_rows(gpu)
+    lean_steps = gpu.get_tuning(abi.TUNE_LEAN_STEPS)
+    lean = 0 < lean_steps <= args.steps
     gpu.set_kernel_timing(True)
     t0 = time.perf_counter()
     rep = gpu.step(args.steps)        # synchronises on return; raises on a negative ce
@@ -620,10 +636,11 @@ def main():
     value = n * args.steps / wall / 1e6
     log("gpu: %d steps in %.3f s, grains %d, gindex %d, k_solute avg %.4f ms over %d launches"
         % (args.steps, wall, rep.num_grains, rep.gindex, k_ms, k_n))
-    rows = (rows + liquid_rows(gpu)) / 2
     gpu.close()
-    if not fp32 and used["zm"] > 0:
-        b_alg -= 16.0 * rows          # lean steps don't write ce and fs of liquid rows
+    rows = None
+    if lean:                          # lean steps don't write ce and fs of liquid rows
+        rows = mean_liquid_rows(cfg, prec, shape, args.warmup, args.steps)
+        b_alg -= 16.0 * rows
     probe = bandwidth_probe(n)
     log("bandwidth probe:", probe)
     achieved = n * b_alg / (k_ms * 1e-3) / 1e9 if k_ms > 0 else None
@@ -633,7 +650,7 @@ def main():
             "traffic": measured_traffic(args.size, used, "fp32" if fp32 else "fp64"),
             "kernel": ("k_solute_rw<%d>" % (1 if used["rows"] == 4 else 2)) if used["zm"] > 0
             else "k_solute<true,true>",
-            "bytes_per_cell": round(b_alg, 2), "liquid_rows": round(rows, 4)}
+            "bytes_per_cell": round(b_alg, 2), "liquid_rows": None if rows is None else round(rows, 4)}
     if probe and achieved:
         mix = probe["solute_mix_fp32dev" if fp32 else "solute_mix_fp64"]["GB/s"]
         roof["probe_same_mix_gbs"] = mix

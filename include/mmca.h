@@ -342,6 +342,9 @@ int  mmca_orientation_draws(const mmca_params *params, const mmca_nucleation_cfg
                                      of every plane on XCD q % 8, units taken plane by plane; used
                                      when the block has at least 8 bands and the step builds the
                                      list itself (mmca_step, batches), before CAPTURE_CHUNK */
+#define MMCA_TUNE_LEAN_STEPS 9   /* read only: the least number of steps in one mmca_step that leaves unwritten
+                                    what stays as it is in rows of liquid cells; 0: the block's calls write
+                                    everything */
 int  mmca_set_tuning(mmca_ctx *ctx, int key, int value);
 int  mmca_get_tuning(mmca_ctx *ctx, int key, int *value);
 

@@ -1936,6 +1936,9 @@ int mmca_get_tuning(mmca_ctx *ctx, int key, int *value)
     case MMCA_TUNE_BEAM_SEP:
         *value = ctx->c.beam_sep;
         return MMCA_OK;
+    case MMCA_TUNE_LEAN_STEPS:
+        *value = lean_call(&ctx, 1, LEAN_STEPS, !ctx->b.rec && zm_rows(ctx->c) > 0) ? LEAN_STEPS : 0;
+        return MMCA_OK;
     default:
         return MMCA_ERR_ARG;
     }
