@@ -74,10 +74,11 @@ def apply_shape(sb, shape):
             sb.set_tuning(key, shape[name])
 
 
-def measured_traffic(size, shape, prec="fp64"):
+def measured_traffic(size, shape, steps, warmup, prec="fp64"):
     """HBM bytes per launch of the solute kernel from the committed
     FETCH_SIZE/WRITE_SIZE summary, when this run has the shape it was
-    measured on (None otherwise)."""
+    measured on and, where the summary names them (lean steps write the more
+    the more is solid), its steps (None otherwise)."""
     import re
     path = TRAFFIC_PROFILES[prec]
     if not os.path.exists(path):
@@ -88,6 +89,9 @@ def measured_traffic(size, shape, prec="fp64"):
     m = re.search(r"traffic_bytes_per_launch = ([0-9.eE+]+)", text)
     want = (size, str(shape["zm"]), str(shape["rows"]), str(shape["xcd"]))
     if not rec or not m or rec.groups() != want:
+        return None
+    run = re.search(r"^steps = (\d+) warmup (\d+)", text, re.M)
+    if run and run.groups() != (str(steps), str(warmup)):
         return None
     return float(m.group(1))
 
@@ -647,7 +651,7 @@ def main():
     roof = {"bound": "hbm", "achieved": round(achieved, 1) if achieved else None,
             "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
-            "traffic": measured_traffic(args.size, used, "fp32" if fp32 else "fp64"),
+            "traffic": measured_traffic(args.size, used, args.steps, args.warmup, "fp32" if fp32 else "fp64"),
             "kernel": ("k_solute_rw<%d>" % (1 if used["rows"] == 4 else 2)) if used["zm"] > 0
             else "k_solute<true,true>",
             "bytes_per_cell": round(b_alg, 2), "liquid_rows": None if rows is None else round(rows, 4)}
