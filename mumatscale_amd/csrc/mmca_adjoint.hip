@@ -335,7 +335,7 @@ using u32x2 = unsigned __attribute__((ext_vector_type(2)));
 // threads of a workgroup: the tile's, and whole waves for the ring and its corners
 constexpr int adj_threads(int ty) { return ADJ_TX * ty + (2 * ADJ_TX + 2 * ty + 4 + 63) / 64 * 64; }
 
-template <bool AM, int TY>
+template <int TY>
 __global__ void __launch_bounds__(adj_threads(TY))
 k_adj_fused(Consts c, Deriv dv, int kz, const unsigned char *code, double sim_time, const double *ce,
             const double *cl, const double *fs, const double *g_ce, const double *g_cl, const double *g_fs,
@@ -486,7 +486,7 @@ k_adj_fused(Consts c, Deriv dv, int kz, const unsigned char *code, double sim_ti
             };
             const int bit = (x - 1) & 31;
             const int br = (int) ((w0 >> bit) & 1u) | (int) (((w1 >> bit) & 1u) << 1) | (int) (((w2 >> bit) & 1u) << 2);
-            const BranchAdj d = branch_adjoint<AM>(c, dv, br, sim_time, x, j, kk, ce_n, C[0], F[0], diffused,
+            const BranchAdj d = branch_adjoint<false>(c, dv, br, sim_time, x, j, kk, ce_n, C[0], F[0], diffused,
                                                    here && tile, gce_n, gcl_n, gfs_n);
             lam0 = d.lam;
             ece = d.ce;
@@ -752,21 +752,19 @@ adjoint_launch(const Consts &c, const Deriv &dv, uint64_t timestep, const uint8_
 {
     const long long nblk = adj_blocks(c);
     const double sim_time = timestep * c.dt;
-    // one pass where no output is an input, and a plane's byte offsets fit 31 bits
-    if (c.sxy <= (1ll << 28) - 1 && adj_separate(c, { g_ce_in, g_cl_in, g_fs_in }, { ce, cl, fs, g_ce, g_cl, g_fs }))
+    // One pass where no output is an input, and a plane's byte offsets fit 31
+    // bits; not for beam blocks: in the one pass the quadratures of growing cells
+    // in successive planes of a walk follow one another (128 x 120 x 104 melt
+    // pool: 9350 us in one pass, 720 in two).
+    if (!c.am && c.sxy <= (1ll << 28) - 1 &&
+        adj_separate(c, { g_ce_in, g_cl_in, g_fs_in }, { ce, cl, fs, g_ce, g_cl, g_fs }))
     {
         const int kz = adj_planes(c);
         const dim3 fgrid((unsigned) (adj_tiles(c) * ((c.nz + kz - 1) / kz)));
         // the first cell of lam is a halo cell, 0 between the calls
         int *done = (int *) lam;
-        if (c.am)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_fused<true, ADJ_TY>), fgrid, dim3(adj_threads(ADJ_TY)), 0, s, c, dv, kz,
-                               codes, sim_time, ce, cl, fs, g_ce, g_cl, g_fs, g_ce_in, g_cl_in, g_fs_in, pa, done,
-                               g_param);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_fused<false, ADJ_TY>), fgrid, dim3(adj_threads(ADJ_TY)), 0, s, c, dv, kz,
-                               codes, sim_time, ce, cl, fs, g_ce, g_cl, g_fs, g_ce_in, g_cl_in, g_fs_in, pa, done,
-                               g_param);
+        hipLaunchKernelGGL(k_adj_fused<ADJ_TY>, fgrid, dim3(adj_threads(ADJ_TY)), 0, s, c, dv, kz, codes, sim_time, ce,
+                           cl, fs, g_ce, g_cl, g_fs, g_ce_in, g_cl_in, g_fs_in, pa, done, g_param);
         return hipGetLastError();
     }
     const dim3 grid((unsigned) nblk), blk(ADJ_BX, ADJ_BY);
