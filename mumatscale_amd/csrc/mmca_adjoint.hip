@@ -96,7 +96,10 @@ struct Cell {
 // XCD takes one contiguous eighth of the tiles, whose work is equal, and tiles
 // that share halo cells share an L2 (128 x 120 x 104: replay 23.7 us with tiles
 // dealt one by one, 22.1 with eighths, and no less with two to four planes per
-// thread on top of that; the adjoint step in place 66 and 52).
+// thread on top of that; the adjoint step in place 66 and 52).  Of a beam block
+// the tiles where cells grow evaluate the quadrature, 400 terms a cell, and lie
+// side by side: its tiles are dealt one by one (replay of a 128 x 120 x 104 melt
+// pool 730 us, 1270 with eighths).
 __device__ __forceinline__ int
 xcd_eighth()
 {
@@ -104,11 +107,12 @@ xcd_eighth()
     return (int) blockIdx.x < 8 * per ? (blockIdx.x % 8) * per + blockIdx.x / 8 : blockIdx.x;
 }
 
+template <bool AM = false>
 __device__ __forceinline__ Cell
 cell_of(const Consts &c)
 {
     const int gbx = (c.nx + ADJ_BX - 1) / ADJ_BX, gby = (c.ny + ADJ_BY - 1) / ADJ_BY;
-    const long long blk = xcd_eighth();
+    const long long blk = AM ? (int) blockIdx.x : xcd_eighth();
     Cell q;
     q.x = (int) (blk % gbx) * ADJ_BX + threadIdx.x + 1;
     q.j = (int) ((blk / gbx) % gby) * ADJ_BY + threadIdx.y + 1;
@@ -142,7 +146,7 @@ __global__ void __launch_bounds__(ADJ_BS)
 k_replay(Consts c, const unsigned char *code, double sim_time, const double *ce, const double *cl,
          const double *fs, double *ce_o, double *cl_o, double *fs_o)
 {
-    const Cell q = cell_of(c);
+    const Cell q = cell_of<AM>(c);
     if (!q.active)
         return;
     long long nb[6];
@@ -566,7 +570,7 @@ k_adj_part(Consts c, Deriv dv, const unsigned char *code, double sim_time, const
            double *lam, double *gce_in, double *gcl_in, double *gfs_in, double *part)
 {
     __shared__ double s_red[ADJ_BS / 64];
-    const Cell q = cell_of(c);
+    const Cell q = cell_of<AM>(c);
     double p_dl = 0.0, p_k = 0.0;
     if (q.active)
     {

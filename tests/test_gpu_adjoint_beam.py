@@ -84,3 +84,36 @@ def test_step_apart_against_in_place():
     codes = _codes(slice(None, None, 4))
     apart, inplace = _ms(lambda: b.adjoint(codes, b.out)), _ms(lambda: b.adjoint(codes, b.grads))
     assert apart < 2 * inplace, (apart, inplace)
+
+
+@pytest.mark.parametrize("what", ["replay", "adjoint"])
+def test_growing_cells_side_by_side_against_spread(what):
+    b = _Block()
+    t = {}
+    for name, planes in (("spread", slice(None, None, 4)), ("side", slice(48, 64))):
+        codes = _codes(planes)
+        t[name] = _ms(lambda: b.replay(codes) if what == "replay" else b.adjoint(codes, b.grads))
+    assert t["side"] < 2 * t["spread"], t
+
+
+def test_replay_of_a_recorded_beam_run():
+    """Bit for bit the state that the recorded run ended in."""
+    from mumatscale_amd import adjoint as ADJ
+    from mumatscale_amd.lib import Subblock
+    from mumatscale_amd.workloads import am_track_config, voronoi_substrate
+    cfg = am_track_config(70, 37, 21)
+    cfg.cell_size, cfg.dt = 1.0e-6, 2.0e-6
+    cfg.laser.update(power=60.0, spot=130e-6, sub_init_temp=600.0, start=[0.0, 18.5e-6, 21e-6])
+    gr, recs = voronoi_substrate(cfg, 40, 5)
+    fs = np.zeros(gr.shape)
+    fs[1:-1, 1:-1, 1:-1] = 1.0
+    with Subblock(cfg.params(check_negative_ce=False), cfg.nucleation()) as sb:
+        sb.set_grains(recs)
+        sb.upload(abi.FIELD_GR, gr)
+        sb.upload(abi.FIELD_FS, fs)
+        traj = ADJ.record(sb, 120)
+        want = [sb.download(f).reshape(-1) for f in (abi.FIELD_CE, abi.FIELD_CL, abi.FIELD_FS)]
+    assert (want[2].reshape(gr.shape)[1:-1, 1:-1, 1:-1] < 1.0).any()
+    got, _ = ADJ.replay(traj, cfg.d_liq, cfg.d_sol, cfg.part_coef)
+    for w, t in zip(want, got):
+        assert np.array_equal(t.cpu().numpy().view(np.uint64), w.view(np.uint64))
