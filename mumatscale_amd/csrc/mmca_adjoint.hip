@@ -710,21 +710,38 @@ long long adj_tiles(const Consts &c)
 // a walk takes two planes more than it finishes: the fewest rounds of the
 // chip's 256 CUs times the planes of a walk.  128 x 120 x 104 (30 tiles): 13
 // planes (240 workgroups) 50 us, 7 (450) 59, 15 (210) 55, 4 (780) 68.
-int adj_planes(const Consts &c)
+// *cost: that product.
+int adj_planes(const Consts &c, long long *cost)
 {
     const long long t = adj_tiles(c);
     int best = 1;
-    long long cost = -1;
+    *cost = -1;
     for (int kz = 1; kz <= std::min(64, c.nz); ++kz)
     {
         const long long rounds = (t * ((c.nz + kz - 1) / kz) + 255) / 256;
-        if (cost < 0 || rounds * (kz + 2) < cost)
+        if (*cost < 0 || rounds * (kz + 2) < *cost)
         {
             best = kz;
-            cost = rounds * (kz + 2);
+            *cost = rounds * (kz + 2);
         }
     }
     return best;
+}
+
+// True where one pass is the faster way.  Not in boxes of one or two rows or
+// planes, where the walks' rows are idle or two of three planes walked are not
+// finished, unless the walks are so short that one launch less decides: one pass
+// and two take 74 and 40 us for 1000 x 1000 x 1 (cost 24), 85 and 69 for 1000 x
+// 1000 x 2 (32), 18.5 and 16.6 for 300 x 1 x 300 (8), 16.3 and 14.8 for 64 x 1 x
+// 1000 (6), 19.6 and 18.7 for 1000 x 2 x 100 (9); but 13.4 and 15.2 for 300 x 300 x
+// 1 (3), 14.9 and 17.1 for 300 x 300 x 2 (4), 12.0 and 14.4 for 128 x 1 x 64 (3);
+// and 97 and 100 for 1000 x 1000 x 3, 19.1 and 19.9 for 300 x 3 x 300.
+// Not for beam blocks either: the quadratures of growing cells in successive
+// planes of a walk follow one another (128 x 120 x 104 melt pool: 9350 us in one
+// pass, 700 in two).
+bool adj_one_pass(const Consts &c, long long cost)
+{
+    return !c.am && ((c.ny >= 3 && c.nz >= 3) || cost <= 4);
 }
 
 // True when none of the outputs overlaps an input or another output.
@@ -756,14 +773,12 @@ adjoint_launch(const Consts &c, const Deriv &dv, uint64_t timestep, const uint8_
 {
     const long long nblk = adj_blocks(c);
     const double sim_time = timestep * c.dt;
-    // One pass where no output is an input, and a plane's byte offsets fit 31
-    // bits; not for beam blocks: in the one pass the quadratures of growing cells
-    // in successive planes of a walk follow one another (128 x 120 x 104 melt
-    // pool: 9350 us in one pass, 720 in two).
-    if (!c.am && c.sxy <= (1ll << 28) - 1 &&
+    // one pass needs outputs apart from the inputs, and a plane's byte offsets in 31 bits
+    long long cost = 0;
+    const int kz = adj_planes(c, &cost);
+    if (adj_one_pass(c, cost) && c.sxy <= (1ll << 28) - 1 &&
         adj_separate(c, { g_ce_in, g_cl_in, g_fs_in }, { ce, cl, fs, g_ce, g_cl, g_fs }))
     {
-        const int kz = adj_planes(c);
         const dim3 fgrid((unsigned) (adj_tiles(c) * ((c.nz + kz - 1) / kz)));
         // the first cell of lam is a halo cell, 0 between the calls
         int *done = (int *) lam;
