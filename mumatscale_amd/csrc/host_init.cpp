@@ -128,7 +128,12 @@ long long padded_cells(const mmca_params &p)
 // workgroups), 445 with 4 x 8; 205x251x303 (2432 workgroups) 222 against 230;
 // 150x140x165 (594) 52 against 45 with 4 x 8; 128x128x256 (512) 52 against 48;
 // 72^3 14.5 with 4 x 4, 15.9 with 4 x 8 (324 workgroups); 40x36x44 8.3 with
-// 4 x 2, 9.5 with 4 x 4.
+// 4 x 2, 9.5 with 4 x 4.  The lines lie the same for the other forms of the
+// kernel.  FP32 storage: 256x256x512 305 with 8 x 16, 312 with 4 x 8;
+// 205x251x303 172 and 175; 150x140x165 49 and 37; 99x130x121 29 and 23; 72^3 16.2
+// with 4 x 8, 14.5 with 4 x 4; 40x36x44 9.1 with 4 x 1, 10.3 with 4 x 4.  Beams,
+// with the quadrature of the waiting cells: 500x256x128 FP32 269 with 8 x 16, 303
+// with 4 x 8, FP64 322 and 372; 250x190x94 FP32 154 and 136, FP64 163 and 155.
 void default_tile(const Consts *const *doms, int n, int *planes, int *rows)
 {
     static const struct { int rows, planes; long long least; } rule[] = {

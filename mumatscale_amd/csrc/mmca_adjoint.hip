@@ -19,7 +19,7 @@
 // the diffusion stencil, and sums the parameter partials in fixed order, so
 // that the gradients are reproducible run to run:
 //   k_adj_fused            all of it in one pass, outputs apart from inputs
-//   k_adj_part, _diff, _sum  the same in place
+//   k_adj_part, _diff, _sum  the same in place, and for beams and thin boxes
 
 #include <hip/hip_runtime.h>
 
@@ -559,8 +559,9 @@ k_adj_fused(Consts c, Deriv dv, int kz, const unsigned char *code, double sim_ti
             g_param[n] += t[n];
 }
 
-// The same step in place, in two passes: the outputs may be the incoming
-// derivatives, which only the cell itself reads in each pass.
+// The same step in two passes: the outputs may be the incoming derivatives,
+// which only the cell itself reads in each pass.  Also the way of beam blocks
+// and thin boxes (adj_one_pass).
 // First the branch: lam, and the direct derivatives; partials of (d_liq,
 // part_coef) per workgroup into part[2 * blk].
 template <bool AM>

@@ -535,9 +535,11 @@ int read_ledger(mmca_ctx *ctx, double *out)
 // the solute kernel is not bound by what it writes there, and testing for it
 // takes longer than it saves (FP32 205 x 251 x 303, 45 % of the words liquid:
 // 177 us a step against 173; FP32 beam 500 x 256 x 128: 187 against 170).
-// Nor do blocks whose fields (56 bytes a cell) the 256 MB of last-level cache
-// hold: 40 x 36 x 44 8.49 ms a pass against 8.27, 8 x 64 x 60 x 96 35.0 against
-// 34.6; above, 150 x 140 x 165 22.7 against 24.2, 256 x 256 x 512 147 against 160.
+// Nor do small blocks, whose writes stay in the 256 MB of last-level cache: 40 x
+// 36 x 44 8.49 ms a pass against 8.27, 8 x 64 x 60 x 96 (2.9 M cells) 35.0 against
+// 34.6; 150 x 140 x 165 (3.5 M) 22.7 against 24.2, 256 x 256 x 512 147 against 160.
+// The line lies between the two sizes measured on its sides.  How much is liquid
+// is not asked: a half solid 256 x 256 x 96 block takes 209 us a step lean, 207 not.
 constexpr int LEAN_STEPS = 8;
 constexpr long long LEAN_CELLS = 3ll << 20;
 
@@ -1861,7 +1863,7 @@ int mmca_set_tuning(mmca_ctx *ctx, int key, int value)
     switch (key) {
     case MMCA_TUNE_ZM_PLANES:
         if (value < 0 || value > 1024)
-            return MMCA_ERR_ARG;   // the LDS-staged kernel keeps one temperature per plane of a tile
+            return MMCA_ERR_ARG;   // the kernel keeps one temperature per plane of a tile in LDS
         ctx->c.zm_planes = value;
         ctx->view_dirty = true;
         return MMCA_OK;

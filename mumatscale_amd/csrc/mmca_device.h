@@ -70,10 +70,11 @@ ld_agent(const T *p)
 
 // True in the workgroup, of n, that gets here last; all of its threads call it.
 // Every thread first waits until its st_agent stores have arrived, so that the
-// last workgroup's ld_agent loads see all of them; a __threadfence() instead
-// would write back and invalidate the whole L2 in every workgroup (it took
-// k_list_count of a 256 x 256 x 512 block from 7 to 150 us).  *done is 0
-// before and after.
+// last workgroup's ld_agent loads see all of them.  Only such values may be
+// handed on: a plain store may still be in the L2 of its XCD, and a plain load
+// may find an old line there.  (A __threadfence() instead would write back and
+// invalidate the whole L2 in every workgroup: it took k_list_count of a 256 x
+// 256 x 512 block from 7 to 150 us.)  *done is 0 before and after.
 __device__ __forceinline__ bool
 last_workgroup(int *done, int n)
 {
